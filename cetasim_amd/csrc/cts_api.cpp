@@ -111,9 +111,6 @@ struct cts_handle {
     int32_t *d_seg_bunch = nullptr, *d_wg_seg = nullptr, *d_bunch_seg = nullptr, *d_seg_rank = nullptr;
     int32_t *d_seg_order = nullptr;  // inverse of d_seg_rank: the segment at each place in particle order
     double *d_seg_part = nullptr;
-    double *d_chunk_part = nullptr;
-    uint32_t *d_chunk_cnt = nullptr;
-    int max_chunks = 1;
 
     // moments
     double *d_shift = nullptr;
@@ -299,7 +296,7 @@ void free_bunch_state(cts_handle *h)
                     h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part, h->d_shift,
                     h->d_cur, h->d_hist, h->d_sigz, h->d_zrange, h->d_noise, h->d_ion_e, h->d_ion_bview,
                     h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev,
-                    h->d_edges_now, h->d_table, h->d_scale, h->d_chunk_part, h->d_chunk_cnt,
+                    h->d_edges_now, h->d_table, h->d_scale,
                     h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -315,8 +312,6 @@ void free_bunch_state(cts_handle *h)
     h->d_bhist = nullptr;
     h->d_counts = nullptr;
     h->d_kick = h->d_poten = h->d_edges_prev = h->d_edges_now = h->d_table = h->d_scale = nullptr;
-    h->d_chunk_part = nullptr;
-    h->d_chunk_cnt = nullptr;
     h->d_fb_count = nullptr;
     h->d_fb_list = nullptr;
 }
@@ -544,9 +539,6 @@ FinParams base_fin(cts_handle *h, uint32_t ops, int slot, int prev_slot)
     f.edges_now = h->d_edges_now;
     f.status = h->d_status;
     f.nseg = h->nseg;
-    f.chunk_part = h->d_chunk_part;
-    f.chunk_cnt = h->d_chunk_cnt;
-    f.max_chunks = h->max_chunks;
     f.lr_cen = h->d_lrw_cen;
     if (h->capturing) {
         f.turn_dev = h->d_turn;
@@ -783,20 +775,17 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
     wgseg[nwg] = (int32_t)sb.size();
     bool identity = true;
     for (int s = 0; s < nseg && identity; s++) identity = rank[s] == s;
-    int max_chunks = 1;
-    for (int bb = 0; bb < nb; bb++) max_chunks = std::max(max_chunks, (bseg[bb + 1] - bseg[bb] + 63) / 64);
     void *old[] = {h->d_seg_begin, h->d_seg_end, h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part,
-                   h->d_chunk_part, h->d_seg_rank, h->d_seg_order};
+                   h->d_seg_rank, h->d_seg_order};
     for (void *p : old)
         if (p) (void)hipFree(p);
     h->d_seg_begin = h->d_seg_end = nullptr;
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = h->d_seg_rank = h->d_seg_order = nullptr;
-    h->d_seg_part = h->d_chunk_part = nullptr;
+    h->d_seg_part = nullptr;
     int rc;
     if ((rc = dalloc(&h->d_seg_begin, nseg)) || (rc = dalloc(&h->d_seg_end, nseg)) ||
         (rc = dalloc(&h->d_seg_bunch, nseg)) || (rc = dalloc(&h->d_wg_seg, nwg + 1)) ||
         (rc = dalloc(&h->d_bunch_seg, nb + 1)) || (rc = dalloc(&h->d_seg_part, (size_t)nseg * kNPart)) ||
-        (rc = dalloc(&h->d_chunk_part, (size_t)nb * max_chunks * kNPart)) ||
         (!identity && ((rc = dalloc(&h->d_seg_rank, nseg)) || (rc = dalloc(&h->d_seg_order, nseg)))))
         return rc;
     if (!identity) {
@@ -812,7 +801,6 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
     HIPCHK(hipMemcpy(h->d_bunch_seg, bseg.data(), bseg.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     h->nwg = nwg;
     h->nseg = nseg;
-    h->max_chunks = max_chunks;
     h->tile = tile;
     return CTS_OK;
 }
@@ -1140,8 +1128,7 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
         (rc = dalloc(&h->d_flag, n)) || (rc = dalloc(&h->d_bunch_off, nb + 1)) ||
         (rc = dalloc(&h->d_bunch_count, nb)) || (rc = dalloc(&h->d_shift, (size_t)nb * 6)) ||
         (rc = dalloc(&h->d_cur, nb)) || (rc = dalloc(&h->d_sigz, nb)) || (rc = dalloc(&h->d_zrange, (size_t)nb * 2)) ||
-        (rc = dalloc(&h->d_ion_e, (size_t)nb * CTS_MAX_SPECIES * 5)) || (rc = dalloc(&h->d_ion_bview, (size_t)nb * 4)) ||
-        (rc = dalloc(&h->d_chunk_cnt, nb)))
+        (rc = dalloc(&h->d_ion_e, (size_t)nb * CTS_MAX_SPECIES * 5)) || (rc = dalloc(&h->d_ion_bview, (size_t)nb * 4)))
         return rc;
     if ((rc = layout_segments(h, h->wg_target, h->tile))) return rc;
     HIPCHK(hipMemcpy(h->d_bunch_off, h->offsets.data(), (nb + 1) * sizeof(int64_t), hipMemcpyHostToDevice));

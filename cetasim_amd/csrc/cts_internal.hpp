@@ -15,6 +15,8 @@
 namespace cts {
 
 constexpr int kBlock = 256;
+constexpr int kPostWaves = 8;  // waves of a block that closes a turn (moments of a bunch, or 64 wake bins)
+constexpr int kPostBlock = 64 * kPostWaves;
 constexpr uint32_t kNewLost = 0x80u;
 
 enum : uint32_t {
@@ -217,9 +219,6 @@ struct FinParams {
     double *zrange;     // survivors' z range (GetZMinMax, without the pad)
     double *edges_now;
     uint32_t *status;
-    double *chunk_part;   // [nb][max_chunks][kNPart]
-    uint32_t *chunk_cnt;  // [nb], left at zero after each launch
-    int32_t max_chunks;
     // history slots from the device turn counter (graph replays):
     // slot = t % hist_cap, prev_slot = (t - 1) % hist_cap, t = *turn_dev + turn_off
     const uint32_t *turn_dev;

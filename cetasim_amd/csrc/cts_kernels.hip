@@ -564,137 +564,136 @@ k_bin(BinParams P)
 }
 
 // ----------------------------------------------------------- finalize
-// Per bunch: reduce the segment partials and write the moment record.
-// grid = (chunks, nb), one wave per chunk of 64 segments: every lane folds
-// one segment, the wave reduces, and the last chunk of a bunch to finish
-// (device-scope counter) folds the chunk results in chunk order, so the
-// result does not depend on scheduling.
-__device__ __forceinline__ double part_identity(int j)
+// Per bunch: fold the segment partials and write the moment record.  One
+// block of kPostWaves waves per bunch: a wave folds four of the values at
+// once (lane = every 64th segment) and reduces them over its lanes; the record's 20 numbers are then
+// formed one per lane.  Everything is added in a fixed order, so the result
+// does not depend on scheduling.  The kernel is bound by latency: with one
+// wave per bunch, its 30 values reduced through LDS shuffles and the record
+// formed by a single thread, it took 17 to 19 us whatever the bunch (20 000
+// or 1e7 macroparticles).
+__device__ __forceinline__ bool part_needed(uint32_t ops, int j)
 {
-    return (j == A_ZMIN || j == C_ZMIN) ? INFINITY : (j == A_ZMAX || j == C_ZMAX) ? -INFINITY : 0.0;
-}
-__device__ __forceinline__ double part_fold(int j, double a, double v)
-{
-    return (j == A_ZMIN || j == C_ZMIN) ? fmin(a, v) : (j == A_ZMAX || j == C_ZMAX) ? fmax(a, v) : a + v;
-}
-__device__ __forceinline__ double part_wave(int j, double a)
-{
-    return (j == A_ZMIN || j == C_ZMIN) ? wave_min(a) : (j == A_ZMAX || j == C_ZMAX) ? wave_max(a) : wave_sum(a);
+    return (j <= A_ZMAX && j != A_LOSS) ? (ops & OP_MOMA) != 0
+         : j == A_LOSS                  ? (ops & OP_LOSS) != 0
+         : j <= B_QZD                   ? (ops & (OP_MOMB | OP_MOMD)) != 0
+         : j <= C_ZMAX                  ? (ops & OP_ZSTAT) != 0
+                                        : (ops & OP_LRC) != 0;
 }
 
-__device__ __forceinline__ void finalize_body(const FinParams &P, int c, int b)
+__device__ __forceinline__ void finalize_body(const FinParams &P, int b)
 {
-    __shared__ double tot[kNPart];
-    __shared__ uint32_t last;
-    const int lane = threadIdx.x;
+    __shared__ double tot[kNPart + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int s0 = P.bunch_seg[b], s1 = P.bunch_seg[b + 1];
-    const int nchunk = (s1 - s0 + 63) / 64;
-    if (c >= nchunk && !(c == 0 && nchunk == 0)) return;
-    {
-        const int s = s0 + c * 64 + lane;
-        double v[kNPart];
+    // the record and the shift as they are, needed after the fold
+    double *curd = reinterpret_cast<double *>(P.cur + b);
+    double *sh = P.shift + 6 * b;
+    double old = 0, sh_l = 0, sh_r = 0;
+    if (tid < 20) old = curd[tid];
+    if (tid < 7) sh_l = tid == 0 ? 0.0 : sh[tid - 1];
+    if (tid >= 32 && tid < 35) sh_r = sh[2 * (tid - 32)];
+    for (int j0 = 4 * wave; j0 < kNPart; j0 += 4 * kPostWaves) {
+        double v[4], v0[4];
+        bool need[4];
 #pragma unroll
-        for (int j = 0; j < kNPart; j++) v[j] = (s < s1) ? P.seg_part[(int64_t)j * P.nseg + s] : part_identity(j);
-        double *dst = P.chunk_part + ((int64_t)b * P.max_chunks + c) * kNPart;
-#pragma unroll
-        for (int j = 0; j < kNPart; j++) {
-            const double r = part_wave(j, v[j]);
-            if (lane == 0) dst[j] = r;
+        for (int u = 0; u < 4; u++) {
+            const int j = j0 + u;
+            need[u] = j < kNPart && part_needed(P.ops, j);
+            v0[u] = (j == A_ZMIN || j == C_ZMIN) ? INFINITY : (j == A_ZMAX || j == C_ZMAX) ? -INFINITY : 0.0;
+            v[u] = v0[u];
         }
-    }
-    if (nchunk > 1) {
-        __threadfence();
-        if (lane == 0) last = atomicAdd(&P.chunk_cnt[b], 1u) == (uint32_t)(nchunk - 1);
-        __syncthreads();
-        if (!last) return;
-        __threadfence();
-        if (lane == 0) P.chunk_cnt[b] = 0u;
-    }
-    {
-        // lane q folds chunks q, q + 64, ...; then the fixed wave tree
-        const double *src = P.chunk_part + (int64_t)b * P.max_chunks * kNPart;
-        const int nc = nchunk > 0 ? nchunk : 1;
-        double v[kNPart];
+        // sixteen loads in flight: four segments of four values
+        for (int s = s0 + lane; s < s1; s += 4 * 64) {
+            double x[4][4];
 #pragma unroll
-        for (int j = 0; j < kNPart; j++) v[j] = part_identity(j);
-        for (int q0 = 0; q0 < nc; q0 += 64) {
-            const int q = q0 + lane;
+            for (int u = 0; u < 4; u++)
 #pragma unroll
-            for (int j = 0; j < kNPart; j++)
-                v[j] = part_fold(j, v[j], q < nc ? src[(int64_t)q * kNPart + j] : part_identity(j));
+                for (int q = 0; q < 4; q++) {
+                    x[u][q] = v0[u];
+                    if (need[u] && s + 64 * q < s1) x[u][q] = P.seg_part[(int64_t)(j0 + u) * P.nseg + s + 64 * q];
+                }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int j = j0 + u;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (j == A_ZMIN || j == C_ZMIN) v[u] = fmin(v[u], x[u][q]);
+                    else if (j == A_ZMAX || j == C_ZMAX) v[u] = fmax(v[u], x[u][q]);
+                    else v[u] += x[u][q];
+                }
+            }
         }
 #pragma unroll
-        for (int j = 0; j < kNPart; j++) {
-            const double r = part_wave(j, v[j]);
+        for (int u = 0; u < 4; u++) {
+            const int j = j0 + u;
+            if (!need[u]) continue;
+            double r;
+            if (j == A_ZMIN || j == C_ZMIN) r = wave_min(v[u]);
+            else if (j == A_ZMAX || j == C_ZMAX) r = wave_max(v[u]);
+            else r = wave_sum_dpp(v[u]);
             if (lane == 0) tot[j] = r;
         }
     }
     __syncthreads();
-    if (lane != 0) return;
+    if (wave != 0) return;
 
-    double *sh = P.shift + 6 * b;
     const double ncount = (double)P.bunch_count[b];
-    cts_moments *cur = P.cur + b;
     int32_t slot = P.slot, prev_slot = P.prev_slot;
     if (P.turn_dev && P.hist_cap > 0) {
         const uint32_t t = *P.turn_dev + (uint32_t)P.turn_off;
         slot = (int32_t)(t % (uint32_t)P.hist_cap);
         prev_slot = t >= 1u ? (int32_t)((t - 1u) % (uint32_t)P.hist_cap) : -1;
     }
-    if ((P.ops & OP_LRC) && P.lr_cen) {
+    if ((P.ops & OP_LRC) && P.lr_cen && lane >= 32 && lane < 35) {
         // post-map centroids (with the shift of the pass, before MOMA moves it)
-        const double n = tot[L_N];
-        P.lr_cen[3 * b] = sh[0] + tot[L_SX] / n;
-        P.lr_cen[3 * b + 1] = sh[2] + tot[L_SY] / n;
-        P.lr_cen[3 * b + 2] = sh[4] + tot[L_SZ] / n;
+        P.lr_cen[3 * b + lane - 32] = sh_r + tot[L_SX + lane - 32] / tot[L_N];
     }
-    double dmean = 0, dzd = 0, ddd = 0;
-    if (P.ops & (OP_MOMB | OP_MOMD)) {
+    // the record, one number per lane: n_alive, mean[6], c2[9], zmin, zmax,
+    // loss_count, transmission.  Means are shift + S / n, second moments
+    // Q / n - (S_i / n) (S_k / n).
+    const bool momb = (P.ops & OP_MOMB) != 0, momd = (P.ops & OP_MOMD) != 0;
+    const bool is_b = lane == 6 || lane == 14 || lane == 15;
+    double vb = 0, va = 0;
+    if ((momb || momd) && is_b) {
         const double n = tot[B_N];
         const double mz = tot[B_SZ] / n, md = tot[B_SD] / n;
-        dmean = sh[5] + md;
-        dzd = tot[B_QZD] / n - mz * md;
-        ddd = tot[B_QDD] / n - md * md;
+        vb = lane == 6 ? sh_l + md : lane == 14 ? tot[B_QZD] / n - mz * md : tot[B_QDD] / n - md * md;
     }
-    if (P.ops & OP_MOMB) {
-        // completes the dp part of the record that was current
-        cur->mean[5] = dmean;
-        cur->c2[7] = dzd;
-        cur->c2[8] = ddd;
-        if (P.hist && prev_slot >= 0) P.hist[(int64_t)prev_slot * P.nb + b] = *cur;
-        sh[5] = dmean;
-    }
-    if (P.ops & OP_MOMA) {
+    const bool is_a = (lane <= 13 && lane != 6) || lane == 16 || lane == 17;
+    if ((P.ops & OP_MOMA) && is_a) {
         const double n = tot[A_N];
-        double m[5];
-        for (int j = 0; j < 5; j++) m[j] = tot[A_S + j] / n;
-        cur->n_alive = n;
-        for (int j = 0; j < 5; j++) cur->mean[j] = sh[j] + m[j];
-        cur->c2[0] = tot[A_Q + 0] / n - m[0] * m[0];
-        cur->c2[1] = tot[A_Q + 1] / n - m[0] * m[1];
-        cur->c2[2] = tot[A_Q + 2] / n - m[1] * m[1];
-        cur->c2[3] = tot[A_Q + 3] / n - m[2] * m[2];
-        cur->c2[4] = tot[A_Q + 4] / n - m[2] * m[3];
-        cur->c2[5] = tot[A_Q + 5] / n - m[3] * m[3];
-        cur->c2[6] = tot[A_Q + 6] / n - m[4] * m[4];
-        cur->zmin = tot[A_ZMIN];
-        cur->zmax = tot[A_ZMAX];
-        for (int j = 0; j < 5; j++) sh[j] = cur->mean[j];
+        if (lane == 0) va = n;
+        else if (lane <= 5) va = sh_l + tot[A_S + lane - 1] / n;
+        else if (lane <= 13) {
+            const int q = lane - 7;  // xx xpx pxpx yy ypy pypy zz
+            const int i = q < 2 ? 0 : q == 2 ? 1 : q < 5 ? 2 : q == 5 ? 3 : 4;
+            const int k = (q == 1 || q == 2) ? 1 : (q == 4 || q == 5) ? 3 : i;
+            va = tot[A_Q + q] / n - (tot[A_S + i] / n) * (tot[A_S + k] / n);
+        } else va = tot[lane == 16 ? A_ZMIN : A_ZMAX];
     }
-    if (P.ops & OP_MOMD) {
-        cur->mean[5] = dmean;
-        cur->c2[7] = dzd;
-        cur->c2[8] = ddd;
-        sh[5] = dmean;
-    }
+    double rec = old;
+    if (momb && is_b) rec = vb;
+    // MOMB completes the dp part of the record that was current
+    if (momb && lane < 20 && P.hist && prev_slot >= 0)
+        reinterpret_cast<double *>(P.hist + (int64_t)prev_slot * P.nb + b)[lane] = rec;
+    if ((P.ops & OP_MOMA) && is_a) rec = va;
+    if (momd && is_b) rec = vb;
     if (P.ops & OP_LOSS) {
-        cur->loss_count = tot[A_LOSS];
-        cur->transmission = (ncount - tot[A_LOSS]) / ncount;
-        if (cur->transmission < 0.5) atomicOr(P.status, 1u);
+        if (lane == 18) rec = tot[A_LOSS];
+        if (lane == 19) {
+            rec = (ncount - tot[A_LOSS]) / ncount;
+            if (rec < 0.5) atomicOr(P.status, 1u);
+        }
     }
-    if ((P.ops & (OP_MOMA | OP_MOMD | OP_LOSS)) && P.hist && slot >= 0)
-        P.hist[(int64_t)slot * P.nb + b] = *cur;
-    if (P.ops & OP_ZSTAT) {
+    if ((P.ops & (OP_MOMA | OP_MOMB | OP_MOMD | OP_LOSS)) && lane < 20) {
+        curd[lane] = rec;
+        if ((P.ops & (OP_MOMA | OP_MOMD | OP_LOSS)) && P.hist && slot >= 0)
+            reinterpret_cast<double *>(P.hist + (int64_t)slot * P.nb + b)[lane] = rec;
+        // the shift follows the means
+        if (((P.ops & OP_MOMA) && lane >= 1 && lane <= 5) || ((momb || momd) && lane == 6)) sh[lane - 1] = rec;
+    }
+    if ((P.ops & OP_ZSTAT) && lane == 63) {
         const double n = tot[C_N];
         const double mz = tot[C_SZ] / n;
         const double sig = sqrt(tot[C_QZZ] / n - mz * mz);
@@ -751,53 +750,64 @@ k_wake_table(WakeTableParams P)
 
 // --------------------------------------------------------------- wake
 // Per bunch: kick_i = (poten_i + sum_j W[i-j] * n_j) * (-e*q/E)
-// (src/MPBunch.cpp:1983-1998), summed over j in order.  grid = (bin groups
-// of 64, nb): each wave stages the table and the counts in LDS and owns 64
-// bins.  The histogram is double-buffered: this turn's buffer is read, the
-// other one (next turn's) is cleared.
+// (src/MPBunch.cpp:1983-1998).  A block owns 64 bins (lane = bin) and stages
+// the table and the counts in LDS; wave w sums the w-th part of the j range
+// in order, and the parts are added in wave order (one wave over the whole
+// range waits 400 dependent additions at 400 bins).  The histogram is
+// double-buffered: this turn's buffer is read, the other one (next turn's)
+// is cleared.
 __device__ __forceinline__ void wake_body(const WakeParams &P, int group, int b)
 {
     extern __shared__ double smem_d[];
     const int nb = P.nbins, nlag = 2 * nb - 1;
     double *n_lds = smem_d;
     double *w_lds = smem_d + nb;
-    const int lane = threadIdx.x;
+    double *part = w_lds + nlag;  // [kPostWaves][64]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = group * 64 + lane;
     const uint32_t *hist = P.bunch_hist + (int64_t)b * nb;
-    for (int j = lane; j < nb; j += 64) n_lds[j] = (double)hist[j];
+    const bool owner = wave == 0 && i < nb;
+    const double poten = owner ? P.poten[(int64_t)b * nb + i] : 0.0;
+    for (int j = tid; j < nb; j += kPostBlock) n_lds[j] = (double)hist[j];
     const double *W = P.table + (P.per_bunch_table ? (int64_t)b * nlag : 0);
-    for (int j = lane; j < nlag; j += 64) w_lds[j] = W[j];
-    if (i < nb) {
+    for (int j = tid; j < nlag; j += kPostBlock) w_lds[j] = W[j];
+    if (owner) {
         P.counts_out[(int64_t)b * nb + i] = (int32_t)hist[i];
         P.hist_clear[(int64_t)b * nb + i] = 0u;
     }
     __syncthreads();
+    const int per = (nb + kPostWaves - 1) / kPostWaves;
+    const int j0 = wave * per, j1 = min(nb, j0 + per);
+    double a = 0.0;
     if (i < nb) {
-        double a = P.poten[(int64_t)b * nb + i];
         const double *Wi = w_lds + i + (nb - 1);
-#pragma unroll 16
-        for (int j = 0; j < nb; j++) a += Wi[-j] * n_lds[j];
+#pragma unroll 8
+        for (int j = j0; j < j1; j++) a += Wi[-j] * n_lds[j];
+    }
+    part[wave * 64 + lane] = a;
+    __syncthreads();
+    if (owner) {
+        a = poten;
+        for (int w = 0; w < kPostWaves; w++) a += part[w * 64 + lane];
         a *= P.scale[b];
         P.poten[(int64_t)b * nb + i] = a;
         P.kick[(int64_t)b * nb + i] = a;
     }
-    if (group == 0 && lane == 0) {
+    if (group == 0 && tid == 0) {
         P.edges_prev[2 * b] = P.edges_now[2 * b];
         P.edges_prev[2 * b + 1] = P.edges_now[2 * b + 1];
     }
 }
+size_t wake_lds(int nbins) { return (size_t)(3 * nbins - 1 + kPostBlock) * sizeof(double); }
 
-__global__ void __launch_bounds__(64) k_finalize(FinParams P) { finalize_body(P, blockIdx.x, blockIdx.y); }
-__global__ void __launch_bounds__(64) k_wake(WakeParams P)
+__global__ void __launch_bounds__(kPostBlock) k_finalize(FinParams P) { finalize_body(P, blockIdx.x); }
+__global__ void __launch_bounds__(kPostBlock) k_wake(WakeParams P) { wake_body(P, blockIdx.x, blockIdx.y); }
+// finalize (x = 0) and wake (x > 0: 64 bins each) of one turn in a single
+// launch: the fixed-grid wake needs only the histogram, not the moments
+__global__ void __launch_bounds__(kPostBlock) k_post(FinParams F, WakeParams W)
 {
-    if ((int)blockIdx.x * 64 < P.nbins) wake_body(P, blockIdx.x, blockIdx.y);
-}
-// finalize (z = 0) and wake (z = 1) of one turn in a single launch: the
-// fixed-grid wake needs only the histogram, not the moments
-__global__ void __launch_bounds__(64) k_post(FinParams F, WakeParams W)
-{
-    if (blockIdx.z == 0) finalize_body(F, blockIdx.x, blockIdx.y);
-    else if ((int)blockIdx.x * 64 < W.nbins) wake_body(W, blockIdx.x, blockIdx.y);
+    if (blockIdx.x == 0) finalize_body(F, blockIdx.y);
+    else wake_body(W, blockIdx.x - 1, blockIdx.y);
 }
 
 // ------------------------------------------------------- ion kick
@@ -1368,14 +1378,13 @@ hipError_t launch_bin(const BinParams &p, int nwg, hipStream_t st)
 }
 hipError_t launch_finalize(const FinParams &p, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_finalize, dim3(p.max_chunks, p.nb), dim3(64), 0, st, p);
+    hipLaunchKernelGGL(k_finalize, dim3(p.nb), dim3(kPostBlock), 0, st, p);
     return hipGetLastError();
 }
 hipError_t launch_post(const FinParams &f, const WakeParams &w, hipStream_t st)
 {
-    const int gx = std::max(f.max_chunks, (w.nbins + 63) / 64);
-    const size_t shm = (size_t)(3 * w.nbins - 1) * sizeof(double);
-    hipLaunchKernelGGL(k_post, dim3(gx, f.nb, 2), dim3(64), shm, st, f, w);
+    const dim3 g(1 + (w.nbins + 63) / 64, f.nb);
+    hipLaunchKernelGGL(k_post, g, dim3(kPostBlock), wake_lds(w.nbins), st, f, w);
     return hipGetLastError();
 }
 hipError_t launch_wake_table(const WakeTableParams &p, int ntables, hipStream_t st)
@@ -1387,8 +1396,7 @@ hipError_t launch_wake_table(const WakeTableParams &p, int ntables, hipStream_t 
 }
 hipError_t launch_wake(const WakeParams &p, int nb, hipStream_t st)
 {
-    const size_t shm = (size_t)(3 * p.nbins - 1) * sizeof(double);
-    hipLaunchKernelGGL(k_wake, dim3((p.nbins + 63) / 64, nb), dim3(64), shm, st, p);
+    hipLaunchKernelGGL(k_wake, dim3((p.nbins + 63) / 64, nb), dim3(kPostBlock), wake_lds(p.nbins), st, p);
     return hipGetLastError();
 }
 hipError_t launch_qe_debug(const float2 *tab, uint64_t seed, uint32_t turn, uint64_t base, int64_t n, double *out,
