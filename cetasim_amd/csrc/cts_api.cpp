@@ -105,10 +105,12 @@ struct cts_handle {
     uint8_t *d_flag = nullptr;
 
     // segments
-    int nwg = 0, nseg = 0, wg_target = 1024;
-    int tile = 0;  // 0: contiguous chunk per workgroup; > 0: tiles dealt round-robin
+    int nwg = 0, nseg = 0;
+    int wg_target = 0;  // workgroups asked for (0: the default layout)
+    int tile = 0;       // 0: contiguous chunk per workgroup; > 0: tiles dealt round-robin
     int64_t *d_seg_begin = nullptr, *d_seg_end = nullptr, *d_bunch_off = nullptr, *d_bunch_count = nullptr;
     int32_t *d_seg_bunch = nullptr, *d_wg_seg = nullptr, *d_bunch_seg = nullptr, *d_seg_rank = nullptr;
+    int32_t *d_seg_step = nullptr;
     int32_t *d_seg_order = nullptr;  // inverse of d_seg_rank: the segment at each place in particle order
     double *d_seg_part = nullptr;
 
@@ -152,6 +154,10 @@ struct cts_handle {
     // the interaction points (their phases run one after the other on the
     // stream); one IonIp per section, nspec 0 where there are no ions
     double *d_ion_e = nullptr;
+    double *d_ion_f = nullptr;  // the clouds' field constants ([nb][species][kBePlan])
+    // items of the electron-side kick (kBlock particles of one bunch each)
+    int32_t *d_item_bunch = nullptr, *d_item_first = nullptr;
+    int nitem = 0;
     double *d_ion_bview = nullptr;
     std::vector<IonIp> ips;
     // d_cur holds the moments of the present coordinates
@@ -277,7 +283,7 @@ BbiParams bbi_params(cts_handle *h)
     for (int q = 0; q < 5; q++) p.planes[q] = h->bbi.planes[q];
     p.energy = h->ring.energy; p.beta2 = std::pow(h->ring.rbeta, 2);
     p.seg_begin = h->d_seg_begin; p.seg_end = h->d_seg_end;
-    p.seg_bunch = h->d_seg_bunch; p.wg_seg = h->d_wg_seg;
+    p.seg_bunch = h->d_seg_bunch; p.wg_seg = h->d_wg_seg; p.seg_step = h->d_seg_step;
     p.x = h->d_x; p.y = h->d_y; p.z = h->d_z;
     p.px = h->d_px; p.py = h->d_py; p.dp = h->d_dp; p.flag = h->d_flag;
     p.hist = h->d_bbi_hist; p.dsum = h->d_bbi_dsum; p.prof = h->d_bbi_prof; p.wake = h->d_bbi_wake;
@@ -295,19 +301,22 @@ void free_bunch_state(cts_handle *h)
                     h->d_seg_begin, h->d_seg_end, h->d_bunch_off, h->d_bunch_count,
                     h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part, h->d_shift,
                     h->d_cur, h->d_hist, h->d_sigz, h->d_zrange, h->d_noise, h->d_ion_e, h->d_ion_bview,
+                    h->d_ion_f, h->d_item_bunch, h->d_item_first,
                     h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev,
                     h->d_edges_now, h->d_table, h->d_scale,
-                    h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order};
+                    h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order, h->d_seg_step};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     h->d_eig = nullptr;
-    h->d_seg_rank = h->d_seg_order = nullptr;
+    h->d_seg_rank = h->d_seg_order = h->d_seg_step = nullptr;
     h->eig_cap = 0;
     h->d_x = h->d_px = h->d_y = h->d_py = h->d_z = h->d_dp = nullptr;
     h->d_flag = nullptr;
     h->d_seg_begin = h->d_seg_end = h->d_bunch_off = h->d_bunch_count = nullptr;
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = nullptr;
     h->d_seg_part = h->d_shift = h->d_sigz = h->d_zrange = h->d_noise = h->d_ion_e = h->d_ion_bview = nullptr;
+    h->d_ion_f = nullptr;
+    h->d_item_bunch = h->d_item_first = nullptr;
     h->d_cur = h->d_hist = nullptr;
     h->d_bhist = nullptr;
     h->d_counts = nullptr;
@@ -476,7 +485,7 @@ PassParams base_pass(cts_handle *h, uint32_t ops, int k)
     p.x = h->d_x; p.px = h->d_px; p.y = h->d_y; p.py = h->d_py; p.z = h->d_z; p.dp = h->d_dp;
     p.flag = h->d_flag;
     p.seg_begin = h->d_seg_begin; p.seg_end = h->d_seg_end;
-    p.seg_bunch = h->d_seg_bunch; p.wg_seg = h->d_wg_seg;
+    p.seg_bunch = h->d_seg_bunch; p.wg_seg = h->d_wg_seg; p.seg_step = h->d_seg_step;
     p.bunch_off = h->d_bunch_off;
     p.seg_part = h->d_seg_part;
     p.seg_rank = h->d_seg_rank;
@@ -613,7 +622,7 @@ int run_bin(cts_handle *h)
     BinParams b;
     b.z = h->d_z;
     b.seg_begin = h->d_seg_begin; b.seg_end = h->d_seg_end;
-    b.seg_bunch = h->d_seg_bunch; b.wg_seg = h->d_wg_seg;
+    b.seg_bunch = h->d_seg_bunch; b.wg_seg = h->d_wg_seg; b.seg_step = h->d_seg_step;
     b.edges = h->d_edges_now;
     b.bunch_hist = h->d_bhist + (size_t)h->hist_parity * h->nb * h->nbins;
     b.nbins = h->nbins;
@@ -695,96 +704,152 @@ int reset_status(cts_handle *h)
     return CTS_OK;
 }
 
-// Segment table.  tile == 0: the particle range cut into wg_target
-// contiguous chunks (multiples of 64); tile > 0: cut into tiles of `tile`
-// particles dealt round-robin to min(wg_target, tiles) workgroups, so the
-// workgroups running at any moment stream one compact window of the arrays
-// (as a grid-stride loop does).  Every piece is cut again at bunch
-// boundaries.  Workgroup w owns the segments wg_seg[w] .. wg_seg[w+1]; the
-// segments are numbered in workgroup order, and seg_rank[s] is segment s's
-// place in particle order, where each bunch's segments are consecutive
+// Workgroups of the streaming pass that the device holds at one time: three
+// of 256 threads per compute unit (the turn's variants use 130 to 152
+// registers).  The default layouts cut the particles for exactly that many,
+// so that no workgroup waits for a second round: with 1024 on 256 compute
+// units the 480-bunch train's pass took 1.50 ms, with 768 1.33 ms.
+constexpr int kPassPerCu = 3;
+
+struct Seg {
+    int64_t begin, end;
+    int32_t bunch, wg, step;
+};
+
+// The segment table of a layout, in particle order within every bunch.
+//  tile == 0, wg > 0: contiguous chunks (multiples of 64, 2048 particles at
+//    least), one per workgroup, cut at bunch boundaries.
+//  tile == 256: a bunch's blocks of 256 particles dealt round-robin to the
+//    workgroups; a workgroup's blocks of one bunch are one strided segment
+//    (one prologue and one reduction for all of them).
+//  other tiles: pieces of `tile` particles of the whole range dealt
+//    round-robin, cut at bunch boundaries.
+//  wg == 0 (the default), by what the 256-CU device measured (us per pass):
+//    one bunch: blocks of 256 round-robin over the resident workgroups, which
+//    streams in grid-stride order (1e7 macroparticles: 246 as 1024 chunks,
+//    235); few particles: equal pieces of whole blocks that never cross a
+//    bunch (a workgroup with two segments takes twice the latency where a
+//    segment is one block); up to 6144 per resident workgroup, one chunk each
+//    (3.5e6 in 60 bunches: 112 over 1024 workgroups, 97); above, a workgroup
+//    per tile, large enough to pay for its prologue and reduction and many
+//    enough for a short last round (8.4e6 in 80 bunches: 206 as 1024 chunks,
+//    178 as 768, 170 in tiles of 4096; 5.9e7 in 480: 1520, 1540, 1278 and
+//    1205 in tiles of 8192).  Chunks of whole blocks, or of a power of two,
+//    put the workgroups on the same memory channels (8.4e6: 229).
+//    `tile` returns the layout that this chose.
+void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
+{
+    const int nb = (int)off.size() - 1;
+    const int64_t n = off[nb];
+    int64_t least = 2048;  // particles of a chunk at least
+    out.clear();
+    if (wg == 0) {
+        wg = resident;
+        tile = 0;
+        least = kBlock;
+        if (nb == 1) tile = kBlock;
+        else if (nb <= resident / 8 && n <= (int64_t)resident * 1024) {
+            int64_t piece = std::max<int64_t>(1, (n + wg - 1) / wg);
+            int64_t total;
+            do {
+                piece = (piece + kBlock - 1) / kBlock * kBlock;
+                total = 0;
+                for (int b = 0; b < nb; b++) total += (off[b + 1] - off[b] + piece - 1) / piece;
+                if (total > wg) piece++;
+            } while (total > wg);
+            nwg = 0;
+            for (int b = 0; b < nb; b++)
+                for (int64_t p = off[b]; p < off[b + 1]; p += piece)
+                    out.push_back({p, std::min(off[b + 1], p + piece), b, nwg++, kBlock});
+            nwg = std::max(nwg, 1);
+            return;
+        } else if (n > (int64_t)resident * 6144) {
+            tile = n > (int64_t)resident * 4 * 8192 ? 8192 : 4096;
+            wg = INT32_MAX / kBlock;
+        }
+    }
+    // a strided segment is walked with 32-bit offsets
+    bool strided = tile == kBlock;
+    for (int b = 0; b < nb; b++) strided = strided && off[b + 1] - off[b] < (int64_t)1 << 31;
+    if (strided) {
+        int64_t blocks = 0;
+        for (int b = 0; b < nb; b++) blocks += (off[b + 1] - off[b] + kBlock - 1) / kBlock;
+        nwg = (int)std::max<int64_t>(1, std::min<int64_t>(wg, blocks));
+        int64_t first = 0;  // the next bunch starts at the workgroup the last one stopped at
+        for (int b = 0; b < nb; b++) {
+            const int64_t nblk = (off[b + 1] - off[b] + kBlock - 1) / kBlock;
+            for (int64_t j = 0; j < std::min<int64_t>(nblk, nwg); j++)
+                out.push_back({off[b] + j * kBlock, off[b + 1], b, (int32_t)((first + j) % nwg), nwg * kBlock});
+            first += nblk;
+        }
+        return;
+    }
+    int64_t piece;
+    if (tile > 0) {
+        piece = ((int64_t)tile + kBlock - 1) / kBlock * kBlock;
+        const int64_t ntile = std::max<int64_t>(1, (n + piece - 1) / piece);
+        nwg = (int)std::min<int64_t>(std::max(wg, 1), ntile);
+    } else {
+        int64_t want = std::max<int64_t>(1, std::min<int64_t>((n + least - 1) / least, wg));
+        piece = std::max<int64_t>(64, ((n + want - 1) / want + 63) / 64 * 64);
+        nwg = (int)std::max<int64_t>(1, (n + piece - 1) / piece);
+    }
+    int b = 0;
+    for (int64_t t = 0; t * piece < n; t++) {
+        const int64_t hi = std::min<int64_t>(n, (t + 1) * piece);
+        for (int64_t p = t * piece; p < hi;) {
+            while (b < nb && off[b + 1] <= p) b++;
+            const int64_t e = std::min<int64_t>(hi, off[b + 1]);
+            out.push_back({p, e, b, (int32_t)(t % nwg), kBlock});
+            p = e;
+        }
+    }
+}
+
+// Segment table on the device (cut_segments): the segments in workgroup
+// order, workgroup w owns wg_seg[w] .. wg_seg[w+1]; seg_rank[s] is segment
+// s's place in particle order, where each bunch's segments are consecutive
 // (bunch_seg) and its partial sums are folded (seg_part is indexed by rank).
 // (Re)allocates everything sized by the number of segments.
 int layout_segments(cts_handle *h, int wg_target, int tile)
 {
     const int nb = h->nb;
-    const int64_t n = h->ntot;
-    int64_t piece;
-    int nwg;
-    if (tile > 0) {
-        piece = ((int64_t)tile + kBlock - 1) / kBlock * kBlock;
-        const int64_t ntile = std::max<int64_t>(1, (n + piece - 1) / piece);
-        nwg = (int)std::min<int64_t>(std::max(wg_target, 1), ntile);
-    } else {
-        int64_t want = (n + 2047) / 2048;
-        if (want < 1) want = 1;
-        if (want > wg_target) want = wg_target;
-        piece = (n + want - 1) / want;
-        piece = (piece + 63) / 64 * 64;
-        if (piece < 64) piece = 64;
-        nwg = (int)((n + piece - 1) / piece) > 0 ? (int)((n + piece - 1) / piece) : 1;
-    }
-    const int64_t npiece = std::max<int64_t>(1, (n + piece - 1) / piece);
-    // segments in particle order, with the piece each belongs to
-    std::vector<int64_t> pb, pe;
-    std::vector<int32_t> pbunch, ppiece;
+    std::vector<Seg> segs;
+    int nwg = 1;
+    cut_segments(h->offsets, wg_target, tile, kPassPerCu * h->ncu, segs, nwg);
+    const int nseg = (int)segs.size();
+    std::vector<int32_t> bseg(nb + 1, nseg);
+    for (int s = nseg - 1; s >= 0; s--) bseg[segs[s].bunch] = s;
+    for (int b = nb - 1; b >= 0; b--)
+        if (h->offsets[b + 1] == h->offsets[b]) bseg[b] = bseg[b + 1];
+    std::vector<int32_t> rank(nseg), wgseg(nwg + 1, 0);
+    for (const Seg &s : segs) wgseg[s.wg + 1]++;
+    for (int w = 0; w < nwg; w++) wgseg[w + 1] += wgseg[w];
     {
-        int b = 0;
-        for (int64_t t = 0; t < npiece; t++) {
-            const int64_t lo = t * piece, hi = std::min<int64_t>(n, lo + piece);
-            int64_t p = lo;
-            while (p < hi) {
-                while (b < nb && h->offsets[b + 1] <= p) b++;
-                const int64_t e2 = std::min<int64_t>(hi, h->offsets[b + 1]);
-                pb.push_back(p);
-                pe.push_back(e2);
-                pbunch.push_back(b);
-                ppiece.push_back((int32_t)t);
-                p = e2;
-            }
-        }
+        std::vector<int32_t> next(wgseg.begin(), wgseg.end() - 1);
+        for (int s = 0; s < nseg; s++) rank[next[segs[s].wg]++] = s;
     }
-    const int nseg = (int)pb.size();
-    std::vector<int32_t> bseg(nb + 1, 0);
-    {
-        int s = 0;
-        for (int bb = 0; bb < nb; bb++) {
-            while (s < nseg && pbunch[s] < bb) s++;
-            bseg[bb] = s;
-        }
-        bseg[nb] = nseg;
+    std::vector<int64_t> sb(nseg), se(nseg);
+    std::vector<int32_t> sbunch(nseg), sstep(nseg);
+    for (int s = 0; s < nseg; s++) {
+        const Seg &g = segs[rank[s]];
+        sb[s] = g.begin;
+        se[s] = g.end;
+        sbunch[s] = g.bunch;
+        sstep[s] = g.step;
     }
-    // workgroup order: piece t goes to workgroup t % nwg (chunked: t == w)
-    std::vector<int32_t> first_seg(npiece + 1, nseg);
-    for (int s = nseg - 1; s >= 0; s--) first_seg[ppiece[s]] = s;
-    for (int64_t t = npiece - 1; t >= 0; t--)
-        if (first_seg[t] == nseg) first_seg[t] = first_seg[t + 1];
-    std::vector<int64_t> sb, se;
-    std::vector<int32_t> sbunch, rank, wgseg(nwg + 1, 0);
-    sb.reserve(nseg); se.reserve(nseg); sbunch.reserve(nseg); rank.reserve(nseg);
-    for (int w = 0; w < nwg; w++) {
-        wgseg[w] = (int32_t)sb.size();
-        for (int64_t t = w; t < npiece; t += nwg)
-            for (int s = first_seg[t]; s < first_seg[t + 1]; s++) {
-                sb.push_back(pb[s]);
-                se.push_back(pe[s]);
-                sbunch.push_back(pbunch[s]);
-                rank.push_back(s);
-            }
-    }
-    wgseg[nwg] = (int32_t)sb.size();
     bool identity = true;
     for (int s = 0; s < nseg && identity; s++) identity = rank[s] == s;
     void *old[] = {h->d_seg_begin, h->d_seg_end, h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part,
-                   h->d_seg_rank, h->d_seg_order};
+                   h->d_seg_rank, h->d_seg_order, h->d_seg_step};
     for (void *p : old)
         if (p) (void)hipFree(p);
     h->d_seg_begin = h->d_seg_end = nullptr;
-    h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = h->d_seg_rank = h->d_seg_order = nullptr;
+    h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = h->d_seg_rank = h->d_seg_order = h->d_seg_step = nullptr;
     h->d_seg_part = nullptr;
     int rc;
     if ((rc = dalloc(&h->d_seg_begin, nseg)) || (rc = dalloc(&h->d_seg_end, nseg)) ||
-        (rc = dalloc(&h->d_seg_bunch, nseg)) || (rc = dalloc(&h->d_wg_seg, nwg + 1)) ||
+        (rc = dalloc(&h->d_seg_bunch, nseg)) || (rc = dalloc(&h->d_seg_step, nseg)) || (rc = dalloc(&h->d_wg_seg, nwg + 1)) ||
         (rc = dalloc(&h->d_bunch_seg, nb + 1)) || (rc = dalloc(&h->d_seg_part, (size_t)nseg * kNPart)) ||
         (!identity && ((rc = dalloc(&h->d_seg_rank, nseg)) || (rc = dalloc(&h->d_seg_order, nseg)))))
         return rc;
@@ -796,6 +861,7 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
     }
     HIPCHK(hipMemcpy(h->d_seg_begin, sb.data(), sb.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_seg_end, se.data(), se.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(h->d_seg_step, sstep.data(), sstep.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_seg_bunch, sbunch.data(), sbunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_wg_seg, wgseg.data(), wgseg.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_seg, bseg.data(), bseg.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -971,6 +1037,7 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
     F.n_alive = Ip.d_nalive;
     F.mean_state = Ip.d_mean;
     F.ion_e = h->d_ion_e;
+    F.ion_f = h->d_ion_f;
     F.cloud = Ip.d_cloud;
     F.status = h->d_status;
     F.gamma = h->ring.rgamma;
@@ -986,8 +1053,10 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
     IonKickParams ik;
     ik.x = h->d_x; ik.y = h->d_y; ik.px = h->d_px; ik.py = h->d_py; ik.flag = h->d_flag;
     ik.seg_begin = h->d_seg_begin; ik.seg_end = h->d_seg_end;
-    ik.seg_bunch = h->d_seg_bunch; ik.wg_seg = h->d_wg_seg;
+    ik.seg_bunch = h->d_seg_bunch; ik.wg_seg = h->d_wg_seg; ik.seg_step = h->d_seg_step;
     ik.ion_e = h->d_ion_e;
+    ik.ion_f = h->d_ion_f;
+    ik.item_bunch = h->d_item_bunch; ik.item_first = h->d_item_first; ik.nitem = h->nitem;
     ik.nspec = Ip.nspec;
     ik.sur_params = nullptr;
     if (h->sur && (h->sur_mode & 2)) sur_export(h->sur, &ik.sur_params, &ik.sur_norm);
@@ -1131,6 +1200,21 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
         (rc = dalloc(&h->d_ion_e, (size_t)nb * CTS_MAX_SPECIES * 5)) || (rc = dalloc(&h->d_ion_bview, (size_t)nb * 4)))
         return rc;
     if ((rc = layout_segments(h, h->wg_target, h->tile))) return rc;
+    {
+        std::vector<int32_t> first(nb + 1, 0), bunch;
+        for (int b = 0; b < nb; b++) {
+            const int64_t items = (counts[b] + kBlock - 1) / kBlock;
+            if (first[b] + items > INT32_MAX / 2) return fail(CTS_ERR_ARG, "cts_set_bunches: too many particles");
+            first[b + 1] = first[b] + (int32_t)items;
+            bunch.insert(bunch.end(), (size_t)items, b);
+        }
+        h->nitem = first[nb];
+        if ((rc = dalloc(&h->d_item_bunch, bunch.size())) || (rc = dalloc(&h->d_item_first, first.size())) ||
+            (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)))
+            return rc;
+        HIPCHK(hipMemcpy(h->d_item_bunch, bunch.data(), bunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(h->d_item_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    }
     HIPCHK(hipMemcpy(h->d_bunch_off, h->offsets.data(), (nb + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_count, h->counts.data(), nb * sizeof(int64_t), hipMemcpyHostToDevice));
     h->kick_pending = false;
@@ -1693,11 +1777,13 @@ int cts_autotune(cts_handle *h, int32_t *nwg_out)
         return rc;
     }
     // (workgroups, tile): contiguous chunks for 1..8 workgroups per CU, then
-    // round-robin tiles of 2048..16384 particles over 2..4 per CU
+    // round-robin tiles of 2048..16384 particles over 2..4 per CU and with a
+    // workgroup each
     std::vector<std::pair<int, int>> cand;
     for (int m = 1; m <= 8; m++) cand.push_back({cus * m, 0});
     for (int m = 2; m <= 4; m++)
         for (int t = 2048; t <= 16384; t *= 2) cand.push_back({cus * m, t});
+    for (int t = 2048; t <= 16384; t *= 2) cand.push_back({INT32_MAX / kBlock, t});
     cand.push_back({h->wg_target, h->tile});
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));

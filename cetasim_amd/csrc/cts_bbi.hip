@@ -204,19 +204,19 @@ __global__ void __launch_bounds__(kBlock) k_bbi_bin(BbiParams P)
     for (int s = P.wg_seg[blockIdx.x]; s < P.wg_seg[blockIdx.x + 1]; s++) {
         const int b = P.seg_bunch[s];
         if (P.scale[b] == 0.0) continue;  // uniform: the whole block skips
-        const int64_t e = P.seg_end[s];
+        const int64_t e = P.seg_end[s], step = P.seg_step[s];
         // the range of bins the segment's counted particles reach; a grid
         // that fits one window is taken whole (no sweep for the range)
         const bool whole = P.n <= (dip ? kBbiDipWin : kBbiWinCopies);
         if (tid == 0) { krange[0] = whole ? 0 : INT_MAX; krange[1] = whole ? P.n - 1 : -1; }
         __syncthreads();
         int rlo = INT_MAX, rhi = -1;
-        for (int64_t i0 = P.seg_begin[s] + tid; !whole && i0 < e; i0 += kUnroll * kBlock) {
+        for (int64_t i0 = P.seg_begin[s] + tid; !whole && i0 < e; i0 += kUnroll * step) {
             double zz[kUnroll];
             uint8_t ff[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + (int64_t)u * kBlock;
+                const int64_t i = i0 + u * step;
                 ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
                 zz[u] = i < e ? P.z[i] : 0.0;
             }
@@ -243,12 +243,12 @@ __global__ void __launch_bounds__(kBlock) k_bbi_bin(BbiParams P)
                 for (int j = tid; j < 4 * wn; j += kBlock) ds[j] = 0ull;
             __syncthreads();
             // four particles per thread in flight: all loads before any use
-            for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * kBlock) {
+            for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * step) {
                 double zz[kUnroll], xx[kUnroll], yy[kUnroll];
                 uint8_t ff[kUnroll];
 #pragma unroll
                 for (int u = 0; u < kUnroll; u++) {
-                    const int64_t i = i0 + (int64_t)u * kBlock;
+                    const int64_t i = i0 + u * step;
                     ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
                     zz[u] = i < e ? P.z[i] : 0.0;
                     xx[u] = (i < e && dipx) ? P.x[i] : 0.0;
@@ -441,20 +441,20 @@ __global__ void __launch_bounds__(kBlock) k_bbi_kick(BbiParams P)
         const double *wz = P.wake + (int64_t)b * P.n;
         const double *wdx = P.wake + nbn + (int64_t)b * P.n, *wdy = P.wake + 2 * nbn + (int64_t)b * P.n;
         const double *wqx = P.wake + 3 * nbn + (int64_t)b * P.n, *wqy = P.wake + 4 * nbn + (int64_t)b * P.n;
-        const int64_t e = P.seg_end[s];
-        for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * kBlock) {
+        const int64_t e = P.seg_end[s], step = P.seg_step[s];
+        for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * step) {
             double zz[kUnroll], d[kUnroll];
             uint8_t ff[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + (int64_t)u * kBlock;
+                const int64_t i = i0 + u * step;
                 ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
                 zz[u] = i < e ? P.z[i] : 0.0;
                 d[u] = (i < e && P.planes[0]) ? P.dp[i] : 0.0;
             }
 #pragma unroll
             for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + (int64_t)u * kBlock;
+                const int64_t i = i0 + u * step;
                 if (!bbi_alive(ff[u])) continue;
                 const int k = bbi_bin(zz[u], P);
                 if (k < 0) continue;

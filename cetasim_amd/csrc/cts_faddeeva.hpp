@@ -385,6 +385,21 @@ __device__ __host__ inline BeField be_plan(double sx, double sy)
     return F;
 }
 
+// The constants as doubles in memory, for kernels that read them as scalars.
+constexpr int kBePlan = 10;
+__device__ __forceinline__ void be_plan_store(const BeField &F, double *g)
+{
+    g[0] = (double)F.mode; g[1] = F.isx; g[2] = F.isy; g[3] = F.isig; g[4] = F.r;
+    g[5] = F.ir; g[6] = F.coeff; g[7] = F.hx; g[8] = F.hy; g[9] = F.sx;
+}
+__device__ __forceinline__ BeField be_plan_load(cdptr g)
+{
+    BeField F;
+    F.mode = (int32_t)g[0]; F.isx = g[1]; F.isy = g[2]; F.isig = g[3]; F.r = g[4];
+    F.ir = g[5]; F.coeff = g[6]; F.hx = g[7]; F.hy = g[8]; F.sx = g[9];
+    return F;
+}
+
 __device__ __forceinline__ bool w_kick_region(double x, double y)
 {
     return x < 100.0 && y < 1000.0;

@@ -76,7 +76,7 @@ struct PassParams {
     double *x, *px, *y, *py, *z, *dp;
     uint8_t *flag;
     const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg;
+    const int32_t *seg_bunch, *wg_seg, *seg_step;
     const int64_t *bunch_off;
     double *seg_part;
     const int32_t *seg_rank;  // segment's place in particle order (null: identity)
@@ -116,8 +116,13 @@ struct IonKickParams {
     double *px, *py;
     const uint8_t *flag;
     const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg;
+    const int32_t *seg_bunch, *wg_seg, *seg_step;
     const double *ion_e;  // per bunch CTS_MAX_SPECIES x {coeffE, xbar, ybar, sx, sy}
+    const double *ion_f;  // per bunch CTS_MAX_SPECIES x the cloud's field constants (kBePlan)
+    // the exact kick's items, up to kBlock particles of one bunch each: the
+    // bunch of every item, and every bunch's first item
+    const int32_t *item_bunch, *item_first;
+    int32_t nitem;
     const float *sur_params;  // field surrogate (null: exact field)
     SurNorm sur_norm;
     // exact-field fallback list of the surrogate variant: entries
@@ -174,6 +179,7 @@ struct IonFinishParams {
     int64_t *n_alive;        // [nspec] out: after the last passage
     double *mean_state;      // [2 * nspec]
     double *ion_e;           // [nb][CTS_MAX_SPECIES][5]
+    double *ion_f;           // [nb][CTS_MAX_SPECIES][kBePlan]
     double *cloud;           // [nb][CTS_MAX_SPECIES][6]
     uint32_t *status;
     double gamma;
@@ -200,7 +206,7 @@ struct IonCompactParams {
 struct BinParams {
     const double *z;
     const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg;
+    const int32_t *seg_bunch, *wg_seg, *seg_step;
     const double *edges;
     uint32_t *bunch_hist;
     int32_t nbins;
@@ -276,7 +282,7 @@ struct BbiParams {
     int planes[5];
     double zmin, dz, half, energy, beta2, bx, by;
     const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg;
+    const int32_t *seg_bunch, *wg_seg, *seg_step;
     const double *x, *y, *z;
     double *px, *py, *dp;
     const uint8_t *flag;

@@ -327,6 +327,7 @@ k_ion_finish(IonFinishParams P)
         e[2] = my;
         e[3] = rx;
         e[4] = ry;
+        be_plan_store(be_plan(rx, ry), P.ion_f + ((int64_t)j * CTS_MAX_SPECIES + p) * kBePlan);
         double *c = P.cloud + ((int64_t)j * CTS_MAX_SPECIES + p) * 6;
         c[0] = n; c[1] = mx; c[2] = my; c[3] = rx; c[4] = ry; c[5] = nI0;
         const double before = j == 0 ? (double)P.len0[p] : ion_sum(acc, j - 1, 5);

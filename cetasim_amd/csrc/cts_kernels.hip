@@ -3,9 +3,9 @@
 // Data layout in HBM: FP64 structure of arrays x, px, y, py, z, dp for all
 // bunches concatenated, one uint8 flag per macroparticle (bits 0-1: the
 // reference's loss code eSurive, bit 7: "lost during the last marking"),
-// and a segment table that cuts the particle range into contiguous
-// per-workgroup chunks intersected with bunch boundaries.  Every workgroup
-// owns one chunk; per-segment partial moments are written without atomics
+// and a segment table that assigns each workgroup its particles: per segment
+// one bunch's particles begin, begin + step, ... in blocks of 256 (step 256:
+// a contiguous piece); per-segment partial moments are written without atomics
 // and reduced per bunch in a fixed order, so moments are reproducible run to
 // run.  Longitudinal histograms are LDS-private per workgroup and merged
 // into the per-bunch histogram with integer atomics (exact, order-free).
@@ -194,6 +194,36 @@ __host__ __device__ constexpr bool acc_used(uint32_t M, int j)
                                         : (M & OP_LRC) != 0;
 }
 
+// the values of the stage set M that are sums (bit j: value j); the extremes
+// follow them in the block's scratch
+__host__ __device__ constexpr uint32_t acc_sums(uint32_t M)
+{
+    uint32_t m = 0;
+    for (int j = 0; j < kNPart; j++)
+        if (acc_used(M, j) && j != A_ZMIN && j != A_ZMAX && j != C_ZMIN && j != C_ZMAX) m |= 1u << j;
+    return m;
+}
+constexpr int kRedExt = (kNPart + 3) / 4 * 4;
+
+// the coordinates a stage set reads and writes (bit j: coordinate j); a pass
+// moves only those
+__host__ __device__ constexpr uint32_t pass_reads(uint32_t M)
+{
+    const bool xy = (M & (OP_MAP | OP_SKEW | OP_SYNRAD | OP_LOSS | OP_MOMA | OP_LRC)) != 0;
+    const bool p = (M & (OP_MAP | OP_SKEW | OP_SYNRAD | OP_MOMA | OP_LRK)) != 0;
+    const bool d = (M & (OP_KICK | OP_LRK | OP_MOMB | OP_MOMD | OP_MAP | OP_RF | OP_BL | OP_DRIFT | OP_U0 |
+                         OP_SYNRAD)) != 0;
+    return (xy ? 5u : 0u) | (p ? 10u : 0u) | 16u | (d ? 32u : 0u);
+}
+__host__ __device__ constexpr uint32_t pass_writes(uint32_t M)
+{
+    if (!(M & OP_WRITE)) return 0u;
+    const bool xy = (M & (OP_MAP | OP_SYNRAD)) != 0, p = (M & (OP_MAP | OP_SKEW | OP_SYNRAD | OP_LRK)) != 0;
+    const bool z = (M & (OP_MAP | OP_DRIFT | OP_SYNRAD)) != 0;
+    const bool d = (M & (OP_KICK | OP_LRK | OP_MAP | OP_RF | OP_BL | OP_U0 | OP_SYNRAD)) != 0;
+    return (xy ? 5u : 0u) | (p ? 10u : 0u) | (z ? 16u : 0u) | (d ? 32u : 0u);
+}
+
 // particles each thread has in flight ahead of the one it computes (two or
 // three steps ahead measured 2 % and 4 % slower on the 480-bunch train: the
 // pass is not short of loads in flight)
@@ -207,7 +237,7 @@ k_pass(PassParams P)
     double *kick_lds = smem_d;                                            // nbins
     uint32_t *hist_lds = reinterpret_cast<uint32_t *>(smem_d + P.nbins);  // nbins
     double *bl_lds = smem_d + P.nbins + (P.nbins + 1) / 2;                // bl_nbl * (bl_nbins + 1)
-    __shared__ double red[kBlock / 64][kNPart];
+    __shared__ double red[kBlock / 64][kRedExt + 4];
 
     // EXACT variants run exactly the stages in M (no runtime stage tests);
     // NOISE >= 0 fixes the noise source at compile time
@@ -226,6 +256,37 @@ k_pass(PassParams P)
     for (int s = s_first; s < s_last; s++) {
         const int b = P.seg_bunch[s];
         const int64_t i0 = P.seg_begin[s], i1 = P.seg_end[s];
+        // per-segment base pointers (uniform) and a 32-bit lane offset, so the
+        // loads and stores use scalar-base + vector-offset addressing
+        double *__restrict__ sx_ = P.x + i0, *__restrict__ spx_ = P.px + i0, *__restrict__ sy_ = P.y + i0;
+        double *__restrict__ spy_ = P.py + i0, *__restrict__ sz_ = P.z + i0, *__restrict__ sdp_ = P.dp + i0;
+        uint8_t *__restrict__ sfl_ = P.flag + i0;
+        constexpr uint32_t rd = pass_reads(M), wr = pass_writes(M);
+        const uint32_t nseg_i = (uint32_t)(i1 - i0), step = (uint32_t)P.seg_step[s];
+        // software pipeline, its first loads issued before the tables are
+        // staged: the coordinates of the particles kPassDepth
+        // steps ahead are loaded while the current one is computed, so HBM
+        // latency (longer than one step's VALU work) overlaps the compute
+        double Xq[kPassDepth][6];
+        uint32_t fq[kPassDepth];
+        // the coordinates are streamed once per pass: nontemporal loads and
+        // stores keep them from displacing the tables in the caches
+#pragma unroll
+        for (int d = 0; d < kPassDepth; d++) {
+            const uint32_t kd = (uint32_t)tid + (uint32_t)d * step;
+#pragma unroll
+            for (int j = 0; j < 6; j++) Xq[d][j] = 0.0;
+            fq[d] = 0u;
+            if (kd < nseg_i) {
+                if (rd & 1u) Xq[d][0] = ntload(sx_ + kd);
+                if (rd & 2u) Xq[d][1] = ntload(spx_ + kd);
+                if (rd & 4u) Xq[d][2] = ntload(sy_ + kd);
+                if (rd & 8u) Xq[d][3] = ntload(spy_ + kd);
+                if (rd & 16u) Xq[d][4] = ntload(sz_ + kd);
+                if (rd & 32u) Xq[d][5] = ntload(sdp_ + kd);
+                fq[d] = ntload(sfl_ + kd);
+            }
+        }
         const int64_t bunch_first = P.bunch_off[b];
         // the bunch's moment shift, re-read as scalars where it is used
         const uint64_t sh_addr = (uint64_t)(uintptr_t)(P.shift + 6 * b);
@@ -294,32 +355,7 @@ k_pass(PassParams P)
         acc[A_ZMIN] = INFINITY; acc[A_ZMAX] = -INFINITY;
         acc[C_ZMIN] = INFINITY; acc[C_ZMAX] = -INFINITY;
 
-        // per-segment base pointers (uniform) and a 32-bit lane offset, so the
-        // loads and stores use scalar-base + vector-offset addressing
-        double *__restrict__ sx_ = P.x + i0, *__restrict__ spx_ = P.px + i0, *__restrict__ sy_ = P.y + i0;
-        double *__restrict__ spy_ = P.py + i0, *__restrict__ sz_ = P.z + i0, *__restrict__ sdp_ = P.dp + i0;
-        uint8_t *__restrict__ sfl_ = P.flag + i0;
-        const uint32_t nseg_i = (uint32_t)(i1 - i0);
-        // software pipeline: the coordinates of the particles kPassDepth
-        // steps ahead are loaded while the current one is computed, so HBM
-        // latency (longer than one step's VALU work) overlaps the compute
-        double Xq[kPassDepth][6];
-        uint32_t fq[kPassDepth];
-        // the coordinates are streamed once per pass: nontemporal loads and
-        // stores keep them from displacing the tables in the caches
-#pragma unroll
-        for (int d = 0; d < kPassDepth; d++) {
-            const uint32_t kd = (uint32_t)tid + (uint32_t)d * kBlock;
-#pragma unroll
-            for (int j = 0; j < 6; j++) Xq[d][j] = 0.0;
-            fq[d] = 0u;
-            if (kd < nseg_i) {
-                Xq[d][0] = ntload(sx_ + kd); Xq[d][1] = ntload(spx_ + kd); Xq[d][2] = ntload(sy_ + kd);
-                Xq[d][3] = ntload(spy_ + kd); Xq[d][4] = ntload(sz_ + kd); Xq[d][5] = ntload(sdp_ + kd);
-                fq[d] = ntload(sfl_ + kd);
-            }
-        }
-        for (uint32_t k = tid; k < nseg_i; k += kBlock) {
+        for (uint32_t k = tid; k < nseg_i; k += step) {
             const int64_t i = i0 + k;
             double X[6];
 #pragma unroll
@@ -331,11 +367,15 @@ k_pass(PassParams P)
                 for (int j = 0; j < 6; j++) Xq[d][j] = Xq[d + 1][j];
                 fq[d] = fq[d + 1];
             }
-            const uint32_t kn = k + (uint32_t)kPassDepth * kBlock;
+            const uint32_t kn = k + (uint32_t)kPassDepth * step;
             if (kn < nseg_i) {
                 double *Xl = Xq[kPassDepth - 1];
-                Xl[0] = ntload(sx_ + kn); Xl[1] = ntload(spx_ + kn); Xl[2] = ntload(sy_ + kn);
-                Xl[3] = ntload(spy_ + kn); Xl[4] = ntload(sz_ + kn); Xl[5] = ntload(sdp_ + kn);
+                if (rd & 1u) Xl[0] = ntload(sx_ + kn);
+                if (rd & 2u) Xl[1] = ntload(spx_ + kn);
+                if (rd & 4u) Xl[2] = ntload(sy_ + kn);
+                if (rd & 8u) Xl[3] = ntload(spy_ + kn);
+                if (rd & 16u) Xl[4] = ntload(sz_ + kn);
+                if (rd & 32u) Xl[5] = ntload(sdp_ + kn);
                 fq[kPassDepth - 1] = ntload(sfl_ + kn);
             }
 
@@ -486,34 +526,57 @@ k_pass(PassParams P)
                 acc[B_QZD] += dz * dd;
             }
             if (ops & OP_WRITE) {
-                ntstore(sx_ + k, X[0]); ntstore(spx_ + k, X[1]); ntstore(sy_ + k, X[2]);
-                ntstore(spy_ + k, X[3]); ntstore(sz_ + k, X[4]); ntstore(sdp_ + k, X[5]);
+                if (wr & 1u) ntstore(sx_ + k, X[0]);
+                if (wr & 2u) ntstore(spx_ + k, X[1]);
+                if (wr & 4u) ntstore(sy_ + k, X[2]);
+                if (wr & 8u) ntstore(spy_ + k, X[3]);
+                if (wr & 16u) ntstore(sz_ + k, X[4]);
+                if (wr & 32u) ntstore(sdp_ + k, X[5]);
                 ntstore(sfl_ + k, (uint8_t)fnew);
             }
         }
 
-        // block reduction of the accumulators -> segment partials
+        // block reduction of the accumulators -> segment partials: the sums
+        // of the stage set four at a time, then the z extremes (maxima as
+        // minima of the negated values)
         const int lane = tid & 63, wave = tid >> 6;
+        constexpr uint32_t sums = acc_sums(M);
+        double sv[kNPart + 3];
+        {
+            int c = 0;
 #pragma unroll
-        for (int j = 0; j < kNPart; j++) {
-            if (!acc_used(M, j)) continue;
-            double v;
-            if (j == A_ZMIN || j == C_ZMIN) v = wave_min(acc[j]);
-            else if (j == A_ZMAX || j == C_ZMAX) v = wave_max(acc[j]);
-            else v = wave_sum(acc[j]);
-            if (lane == 0) red[wave][j] = v;
+            for (int j = 0; j < kNPart; j++)
+                if ((sums >> j) & 1u) sv[c++] = acc[j];
+#pragma unroll
+            for (int u = 0; u < 3; u++) sv[c + u] = 0.0;
+        }
+        const bool store = (lane & 15) == 0;
+        const int sub = pack4_value(lane >> 4);
+#pragma unroll
+        for (int g = 0; g < (kNPart + 3) / 4; g++) {
+            if (4 * g >= __builtin_popcount(sums)) continue;
+            const double r = wave_pack4<false>(sv[4 * g], sv[4 * g + 1], sv[4 * g + 2], sv[4 * g + 3]);
+            if (store) red[wave][4 * g + sub] = r;
+        }
+        if (M & (OP_MOMA | OP_ZSTAT)) {
+            const double r = wave_pack4<true>(acc[A_ZMIN], -acc[A_ZMAX], acc[C_ZMIN], -acc[C_ZMAX]);
+            if (store) red[wave][kRedExt + sub] = r;
         }
         __syncthreads();
         if (tid < kNPart) {
+            const bool mn = tid == A_ZMIN || tid == C_ZMIN, mx = tid == A_ZMAX || tid == C_ZMAX;
             // identity of the unused slots (0, +inf for minima, -inf for maxima)
-            double v = (tid == A_ZMIN || tid == C_ZMIN) ? INFINITY
-                     : (tid == A_ZMAX || tid == C_ZMAX) ? -INFINITY : 0.0;
+            double v = mn ? INFINITY : mx ? -INFINITY : 0.0;
             if (acc_used(M, tid)) {
-                v = red[0][tid];
-                for (int w = 1; w < kBlock / 64; w++) {
-                    if (tid == A_ZMIN || tid == C_ZMIN) v = fmin(v, red[w][tid]);
-                    else if (tid == A_ZMAX || tid == C_ZMAX) v = fmax(v, red[w][tid]);
-                    else v = v + red[w][tid];
+                if (mn || mx) {
+                    const int e = kRedExt + (tid == A_ZMIN ? 0 : tid == A_ZMAX ? 1 : tid == C_ZMIN ? 2 : 3);
+                    v = red[0][e];
+                    for (int w = 1; w < kBlock / 64; w++) v = fmin(v, red[w][e]);
+                    if (mx) v = -v;
+                } else {
+                    const int e = __popc(sums & ((1u << tid) - 1u));
+                    v = red[0][e];
+                    for (int w = 1; w < kBlock / 64; w++) v = v + red[w][e];
                 }
             }
             P.seg_part[(int64_t)tid * P.nseg + (P.seg_rank ? P.seg_rank[s] : s)] = v;
@@ -550,7 +613,8 @@ k_bin(BinParams P)
         for (int j = tid; j < P.nbins; j += kBlock) hist_lds[j] = 0u;
         const double lo = P.edges[2 * b], dz = P.edges[2 * b + 1], inv = 1.0 / dz;
         __syncthreads();
-        for (int64_t i = i0 + tid; i < i1; i += kBlock) {
+        const int64_t step = P.seg_step[s];
+        for (int64_t i = i0 + tid; i < i1; i += step) {
             const int hb = bin_of(P.z[i], lo, dz, inv, P.nbins);
             if (hb >= 0) atomicAdd(&hist_lds[hb], 1u);
         }
@@ -814,42 +878,41 @@ __global__ void __launch_bounds__(kPostBlock) k_post(FinParams F, WakeParams W)
 // Electron side of MPBunch::SSIonBunchInteraction (src/MPBunch.cpp:1165-1206)
 // followed by BunchTransferDueToIon (src/Bunch.cpp:213-220): survivors get
 // px/py += sum over species of 2*N_ion*r_e/gamma * F(x - xbar, y - ybar).
-// Four waves per SIMD (128 VGPRs): the field is compute-bound and the
-// extra waves hide its latency better than the registers they cost
-// (a few spills, in the rarely taken far-field branch).
-__global__ void __launch_bounds__(kBlock, 4)
+// One macroparticle per thread and no loop: the field needs about 50
+// registers, but inside a loop its polynomial constants and far-field branch
+// were hoisted into registers until the kernel spilled at four waves per SIMD;
+// here (54 registers) they stay where they are used and eight waves per SIMD overlap the
+// momenta's memory latency with the field.  The clouds' constants come ready
+// from k_ion_finish and are read as scalars (uniform over a block: an item is
+// up to 256 particles of one bunch).  5.9e7 macroparticles in 480 bunches:
+// 1.54 ms as a strided loop over the pass's segments at four waves per SIMD,
+// 0.70 ms now (4.1 TB/s of the 49 B per macroparticle); 8.4e6: 210 -> 103 us;
+// 18 000: 27.6 -> 6.7 us.  With several species the loop over them is back.
+template <bool ONE>
+__global__ void __launch_bounds__(kBlock)
 k_ion_kick(IonKickParams P)
 {
-    __shared__ BeField sF[CTS_MAX_SPECIES];
-    const int tid = threadIdx.x;
-    // the segments in particle order dealt round-robin to this launch's own
-    // grid (four workgroups per CU, the occupancy the kernel is compiled
-    // for): the workgroups running at one time stream one compact window
-    for (int r = blockIdx.x; r < P.nseg; r += gridDim.x) {
-        const int s = P.seg_order ? P.seg_order[r] : r;
-        const int b = P.seg_bunch[s];
-        const double *c = P.ion_e + (int64_t)b * CTS_MAX_SPECIES * 5;
-        // the clouds' constants, once per segment
-        if (tid < P.nspec) sF[tid] = be_plan(c[5 * tid + 3], c[5 * tid + 4]);
-        __syncthreads();
-        // the momenta are read with the positions, so that one memory
-        // latency per electron, not two, sits in front of the field
-        for (int64_t i = P.seg_begin[s] + tid; i < P.seg_end[s]; i += kBlock) {
-            const uint8_t f = P.flag[i];
-            const double x = P.x[i], y = P.y[i], px0 = P.px[i], py0 = P.py[i];
-            if (f & 3u) continue;
-            double fxs = 0.0, fys = 0.0;
-            for (int p = 0; p < P.nspec; p++) {
-                double fx, fy;
-                be_field(x - c[5 * p + 1], y - c[5 * p + 2], sF[p], fx, fy);
-                fxs = fxs + c[5 * p] * fx;
-                fys = fys + c[5 * p] * fy;
-            }
-            P.px[i] = px0 + fxs;
-            P.py[i] = py0 + fys;
+    const int b = P.item_bunch[blockIdx.x];
+    const int64_t i = P.bunch_off[b] + (int64_t)((int)blockIdx.x - P.item_first[b]) * kBlock + threadIdx.x;
+    if (i >= P.bunch_off[b + 1]) return;
+    const uint8_t f = P.flag[i];
+    const double x = P.x[i], y = P.y[i], px0 = P.px[i], py0 = P.py[i];
+    if (f & 3u) return;
+    const cdptr c = reload((uint64_t)(uintptr_t)(P.ion_e + (int64_t)b * CTS_MAX_SPECIES * 5));
+    const cdptr g = reload((uint64_t)(uintptr_t)(P.ion_f + (int64_t)b * CTS_MAX_SPECIES * kBePlan));
+    double fxs, fys;
+    be_field(x - c[1], y - c[2], be_plan_load(g), fxs, fys);
+    fxs = 0.0 + c[0] * fxs;
+    fys = 0.0 + c[0] * fys;
+    if (!ONE)
+        for (int p = 1; p < P.nspec; p++) {
+            double fx, fy;
+            be_field(x - c[5 * p + 1], y - c[5 * p + 2], be_plan_load(g + p * kBePlan), fx, fy);
+            fxs = fxs + c[5 * p] * fx;
+            fys = fys + c[5 * p] * fy;
         }
-        __syncthreads();
-    }
+    P.px[i] = px0 + fxs;
+    P.py[i] = py0 + fys;
 }
 
 // The same kick with the field surrogate inside its domain and the exact
@@ -866,7 +929,8 @@ k_ion_kick_sur(IonKickParams P)
         const int s = P.seg_order ? P.seg_order[r] : r;
         const int b = P.seg_bunch[s];
         const double *c = P.ion_e + (int64_t)b * CTS_MAX_SPECIES * 5;
-        for (int64_t base = P.seg_begin[s]; base < P.seg_end[s]; base += kBlock) {
+        const int64_t step = P.seg_step[s];
+        for (int64_t base = P.seg_begin[s]; base < P.seg_end[s]; base += step) {
             const int64_t i = base + tid;
             const bool active = i < P.seg_end[s] && (P.flag[i] & 3u) == 0;
             const double x = active ? P.x[i] : 0.0, y = active ? P.y[i] : 0.0;
@@ -1120,6 +1184,10 @@ hipError_t launch_lrwake(const LrwParams &p, hipStream_t st)
 
 // ------------------------------------------------------------ launches
 constexpr uint32_t V_KICK = OP_KICK | OP_MOMB | OP_LRK | OP_WRITE;
+// longitudinal stages alone (a pending wake kick, the RF, drift and energy
+// loss seams): z and delta move, 34 B per macroparticle instead of 98
+constexpr uint32_t V_LONG = OP_KICK | OP_MOMB | OP_RF | OP_DRIFT | OP_U0 | OP_WRITE;
+constexpr uint32_t V_Z = OP_ZSTAT | OP_BIN;  // read-only: the z range, the bins
 constexpr uint32_t V_MOM = OP_MOMA | OP_MOMB | OP_MOMD | OP_ZSTAT | OP_LOSS;
 constexpr uint32_t V_FIX = OP_KICK | OP_MOMB | OP_MAP | OP_SKEW | OP_RF | OP_DRIFT | OP_U0 | OP_SYNRAD |
                            OP_BIN | OP_LOSS | OP_MOMA | OP_MOMD | OP_WRITE | OP_LRC | OP_LRK;
@@ -1332,6 +1400,10 @@ hipError_t launch_pass(const PassParams &p, int nwg, hipStream_t st)
         hipLaunchKernelGGL((k_pass<T_QE, true, 1, 1>), g, b, shm, st, p);
     else if (one_rf && o == T_NOSR)
         hipLaunchKernelGGL((k_pass<T_NOSR, true, 0, 1>), g, b, shm, st, p);
+    else if ((o & ~(V_KICK & ~OP_LRK)) == 0)
+        hipLaunchKernelGGL((k_pass<V_KICK & ~OP_LRK, false, -1, -1>), g, b, shm, st, p);
+    else if ((o & ~V_Z) == 0) hipLaunchKernelGGL((k_pass<V_Z, false, -1, -1>), g, b, shm, st, p);
+    else if ((o & ~V_LONG) == 0) hipLaunchKernelGGL((k_pass<V_LONG, false, -1, -1>), g, b, shm, st, p);
     else if ((o & ~V_KICK) == 0) hipLaunchKernelGGL((k_pass<V_KICK, false, -1, -1>), g, b, shm, st, p);
     else if ((o & OP_BL) && (o & ~V_BLB) == 0) hipLaunchKernelGGL((k_pass<V_BLB, false, -1, -1>), g, b, shm, st, p);
     else if ((o & OP_BLH) && (o & ~V_BLH) == 0) hipLaunchKernelGGL((k_pass<V_BLH, false, -1, -1>), g, b, shm, st, p);
@@ -1350,7 +1422,9 @@ hipError_t launch_ion_kick(const IonKickParams &p, int nwg, hipStream_t st)
         hipLaunchKernelGGL(k_ion_kick_fb, dim3(512), dim3(kBlock), 0, st, p);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_ion_kick, dim3(nwg), dim3(kBlock), 0, st, p);
+    if (p.nitem == 0) return hipSuccess;
+    if (p.nspec == 1) hipLaunchKernelGGL(k_ion_kick<true>, dim3(p.nitem), dim3(kBlock), 0, st, p);
+    else hipLaunchKernelGGL(k_ion_kick<false>, dim3(p.nitem), dim3(kBlock), 0, st, p);
     return hipGetLastError();
 }
 __global__ void k_set_turn(uint32_t *t, uint32_t v)

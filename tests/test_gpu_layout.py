@@ -1,0 +1,72 @@
+"""The default layouts of the streaming pass against an explicit one on the
+same particles, at the edges of the rule that picks them (one bunch of less
+or more than a block, few and many bunches, tiles for many particles):
+coordinates, loss codes and bin counts bit-identical on the fixed grid,
+moments to 1e-12 (partial sums regrouped).  And the electron-side ion kick,
+an item of up to 256 macroparticles per block, at the edges of its items."""
+import numpy as np
+import pytest
+
+from cetasim_amd import configs
+from cetasim_amd.tracker import COORDS, Tracker
+
+import oracle as O
+from test_gpu_train import BBR, ION_TEST, compare_coords, setup_train
+
+pytestmark = pytest.mark.gpu
+
+SZ = configs.BASE["sig"][2]
+
+
+@pytest.mark.parametrize("counts", [[1], [255], [257], [200_001], [1, 300, 256], [3000] * 8, [9_001] * 90,
+                                    [700, 3] * 60, [4_800_000, 5, 70_000]])
+def test_default_layouts_agree(counts):
+    ring, secs, _ = configs.lattice()
+    counts = np.array(counts, np.int64)
+    q, ne = configs.bunch_scalars(counts, ring)
+    rng = np.random.default_rng(8)
+    n = int(counts.sum())
+    sx, sy, sz, sd = configs.BASE["sig"]
+    scale = dict(x=sx, px=sx / 10, y=sy, py=sy / 10, z=sz, dp=sd)
+    parts = {c: rng.standard_normal(n) * scale[c] for c in COORDS}
+    lost = (rng.random(n) < 0.02).astype(np.int32) * 2
+    lost[np.cumsum(counts) - counts] = 0  # every bunch keeps a particle
+    print(f"default layout of {len(counts)} bunches, {n} macroparticles", flush=True)
+    outs = []
+    for lay in (None, (7, 0)):
+        tr = Tracker(ring, secs)
+        tr.set_bunches(counts, q, ne, configs.train_gaps(len(counts), 2, ring.harmonic))
+        tr.upload(parts, lost)
+        tr.set_wake(64, 1, -5 * SZ, 5 * SZ, BBR["rs"], BBR["q"], BBR["fr"])
+        tr.set_synrad(True, 2, 3)
+        if lay:
+            tr.set_layout(*lay)
+        for t in range(2):
+            tr.turn(t)
+        outs.append((tr.wake_state()[0], tr.moments(), tr.download()))
+        tr.close()
+    (h0, m0, d0), (h1, m1, d1) = outs
+    assert np.array_equal(h0, h1) and h0.sum() > 0
+    for c in COORDS + ("lost",):
+        assert np.array_equal(d0[c], d1[c]), c
+    for a, b in zip(m0, m1):
+        assert a["n_alive"] == b["n_alive"] and a["zmin"] == b["zmin"] and a["zmax"] == b["zmax"]
+        if a["n_alive"] > 1:
+            np.testing.assert_allclose(a["c2"], b["c2"], rtol=1e-9, atol=1e-12 * np.max(np.abs(b["c2"])))
+
+
+@pytest.mark.parametrize("nspec", [1, 2])
+def test_ion_kick_items(nspec):
+    counts = [255, 256, 257, 512, 700]
+    ions = dict(ION_TEST, mass_number=[28.0, 18.0][:nspec], cross_section=[2.0e-22, 1.6e-22][:nspec],
+                pressure=[1.0e-5, 0.4e-5][:nspec])
+    ring, secs, counts, gap, q, ne, cfg, tr, bunches, off = setup_train(counts, 6, ions=ions, ne_scale=0.1)
+    ot = O.OracleTrain(ring, secs[0], counts, ne, gap, cfg, ions["seed"])
+    before = np.concatenate([b["px"] for b in bunches])
+    print(f"ion kick items, {nspec} species", flush=True)
+    tr.ion_phase(0)
+    ot.ion_phase(bunches, 0)
+    got = tr.download()
+    compare_coords(got, bunches, off, 1e-12)
+    assert np.max(np.abs(got["px"] - before)) > 1e-8 * np.max(np.abs(before))
+    tr.close()
