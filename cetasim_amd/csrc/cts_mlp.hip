@@ -54,9 +54,27 @@ k_mlp_samples(int64_t n, uint64_t seed, uint32_t tag, float *out, double *exact)
 }
 
 // ------------------------------------------------------------- training
-// One workgroup = one wave; it runs `chunks` batches of 64 samples and
-// accumulates the gradient of the mean squared error of the normalized
-// targets, then writes its partial gradient (+ loss) to part[wg].
+// Gradient of the mean squared error of the normalized targets.  A block of
+// four waves runs `chunks` batches of 64 samples and writes its partial
+// gradient (+ loss) to part[block].  Each wave takes 16 samples of a batch
+// through the network and back; then the sums over the batch's 64 samples are
+// shared out: every wave forms a quarter of dW2 on the matrix cores and one
+// or two of the per-feature sums (lane = feature, samples in order).
+//
+// Register layouts follow the MFMA operands (lane l: lr = l % 16, lg = l / 16):
+//   rows   A operand: sample lr, features 32 kb + 8 lg + i
+//   cols   result: samples 4 lg + t, feature 16 fb + lr
+// H1 is computed in both (three multiply-adds and a GELU per element, and the
+// cols need GELU' anyway), dZ2 passes from cols to rows through LDS, and the
+// split weights of both products stay in registers.
+//
+// What it is bound by: the chain of a batch (record gather, two layers, the
+// sums in order) on one or two waves per SIMD.  One wave per 64-sample batch
+// with every operand staged in 145 KB of LDS, one wave on a compute unit, took
+// 126 us for 512 blocks of two batches; this takes 32 us (about 8 us a batch
+// with two blocks on a compute unit) and gives the same gradients, since every
+// sum keeps its order.  With the waves' sums joined only once, over 32 samples
+// each, 24 us, but the weights of a long training run drift from the others'.
 struct MlpTrainParams {
     const float *params;    // kMlpParams
     const float *samples;   // [n][5]
@@ -70,44 +88,39 @@ struct MlpTrainParams {
     int32_t random;         // 0: samples taken in order (gradient checks)
 };
 
-__global__ void __launch_bounds__(64)
+constexpr int kTrainBlock = 256;
+constexpr int kRow = 68;  // pitch of a row of 64 dwords in LDS
+
+// order between a wave's own LDS writes and reads
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ void __launch_bounds__(kTrainBlock, 2)
 k_mlp_train(MlpTrainParams P)
 {
 #pragma clang fp contract(fast)
-    __shared__ __attribute__((aligned(16))) __bf16 w2h[64 * kPb], w2l[64 * kPb];    // W2[n][k]
-    __shared__ __attribute__((aligned(16))) __bf16 w2th[64 * kPb], w2tl[64 * kPb];  // W2^T[k][n]
-    __shared__ __attribute__((aligned(16))) __bf16 h1h[64 * kPb], h1l[64 * kPb];    // H1[s][k]
-    __shared__ __attribute__((aligned(16))) __bf16 h1th[64 * kPb], h1tl[64 * kPb];  // H1^T[k][s]
-    __shared__ __attribute__((aligned(16))) __bf16 d2h[64 * kPb], d2l[64 * kPb];    // dZ2[s][n]
-    __shared__ __attribute__((aligned(16))) __bf16 d2th[64 * kPb], d2tl[64 * kPb];  // dZ2^T[n][s]
-    __shared__ float z1s[64 * kPf];  // z1, then dz1   [s][k]
-    __shared__ float z2s[64 * kPf];  // z2, then h2    [s][n]
-    __shared__ float xs[64 * 4];
-    __shared__ float dos[64 * 2];
-    const int l = threadIdx.x;
+    // the operands of dW2: dZ2^T[n][s] and H1^T[k][s], split; W2 is staged in
+    // their place at the start
+    __shared__ __attribute__((aligned(16))) __bf16 tr[4][64 * kPb];
+    __bf16 *d2th = tr[0], *d2tl = tr[1], *h1th = tr[2], *h1tl = tr[3];
+    __shared__ __attribute__((aligned(16))) uint32_t dzs[64 * kRow];  // dZ2[s][n] (hi, lo), then dZ1[s][k]
+    __shared__ __attribute__((aligned(16))) float h2s[64 * kRow];     // H2[s][n]
+    __shared__ __attribute__((aligned(16))) float recs[64 * 8];       // a0 a1 a2 valid y0 y1 - -
+    __shared__ float dos[64 * 2];                                     // d loss / d output
+    __shared__ float w1s[64 * 4], w3s[64 * 4];                        // W1[k], b1[k]; b2[n], W3[0][n], W3[1][n]
+    const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
     const int lr = l & 15, lg = l >> 4;
     const float *W = P.params;
+    float *dz1s = reinterpret_cast<float *>(dzs);
 
-    for (int i = l; i < 4096; i += 64) {
-        const int n = i >> 6, k = i & 63;
-        __bf16 hi, lo;
-        split_bf16(W[MP_W2 + i], hi, lo);
-        w2h[n * kPb + k] = hi; w2l[n * kPb + k] = lo;
-        w2th[k * kPb + n] = hi; w2tl[k * kPb + n] = lo;
-    }
-    // per-feature accumulators (lane = feature j) and the dW2 tiles
-    float gw1[3] = {0, 0, 0}, gb1 = 0, gb2 = 0, gw3[2] = {0, 0}, gb3[2] = {0, 0}, loss = 0;
-    v4f gw2[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) gw2[a][b] = (v4f){0, 0, 0, 0};
-    const float w3_0l = W[MP_W3 + l], w3_1l = W[MP_W3 + 64 + l];
-    (void)w3_0l; (void)w3_1l;
-    __syncthreads();
-
-    for (int c = 0; c < P.chunks; c++) {
-        const int64_t gid = ((int64_t)blockIdx.x * P.chunks + c) * 64 + l;
+    // the record of sample gid (lanes below 16 of each wave: 16 wv + l)
+    float rc[5] = {0, 0, 0, 0, 0};
+    bool valid = false;
+    auto fetch = [&](int c) {
+        const int64_t gid = ((int64_t)blockIdx.x * P.chunks + c) * 64 + 16 * wv + l;
         int64_t idx;
         if (P.random) {
             const u32x4 o = philox4x32_10((uint32_t)gid, (uint32_t)(gid >> 32), P.step, 0x4d4c5054u,
@@ -116,160 +129,301 @@ k_mlp_train(MlpTrainParams P)
         } else {
             idx = gid < P.n ? gid : P.n - 1;
         }
+        valid = P.random || gid < P.n;
         const float *rec = P.samples + idx * 5;
-        const float a0 = rec[0], a1 = rec[1], a2 = rec[2];
-        const float y0 = (rec[3] - P.norm[0]) / P.norm[1], y1 = (rec[4] - P.norm[2]) / P.norm[3];
-        const bool valid = P.random || gid < P.n;
-        xs[l * 4 + 0] = a0; xs[l * 4 + 1] = a1; xs[l * 4 + 2] = a2;
-        // layer 1 (lane = sample)
-        for (int k = 0; k < 64; k++) {
-            const float z = W[MP_B1 + k] + W[MP_W1 + 3 * k] * a0 + W[MP_W1 + 3 * k + 1] * a1 + W[MP_W1 + 3 * k + 2] * a2;
-            z1s[l * kPf + k] = z;
-            __bf16 hi, lo;
-            split_bf16(gelu_only(z), hi, lo);
-            h1h[l * kPb + k] = hi; h1l[l * kPb + k] = lo;
-            h1th[k * kPb + l] = hi; h1tl[k * kPb + l] = lo;
-        }
-        __syncthreads();
-        // layer 2: Z2[s][n] = sum_k H1[s][k] W2[n][k]
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+        for (int j = 0; j < 5; j++) rc[j] = rec[j];
+    };
+    if (l < 16) fetch(0);
+
+    // the weights: W2 through LDS into this lane's operands of H1 W2^T and
+    // dZ2 W2 (feature 16 fb + lr, 8 of the other index)
+    float *w2s = reinterpret_cast<float *>(&tr[0][0]);
+    for (int i = tid; i < 4096; i += kTrainBlock) w2s[(i >> 6) * kRow + (i & 63)] = W[MP_W2 + i];
+    if (tid < 64) {
+        for (int j = 0; j < 3; j++) w1s[4 * tid + j] = W[MP_W1 + 3 * tid + j];
+        w1s[4 * tid + 3] = W[MP_B1 + tid];
+        w3s[4 * tid] = W[MP_B2 + tid];
+        w3s[4 * tid + 1] = W[MP_W3 + tid];
+        w3s[4 * tid + 2] = W[MP_W3 + 64 + tid];
+        w3s[4 * tid + 3] = 0.0f;
+    }
+    __syncthreads();
+    v8bf w2h[4][2], w2l[4][2], w2th[4][2], w2tl[4][2];
 #pragma unroll
-            for (int nb = 0; nb < 4; nb++) {
-                v4f acc = {0, 0, 0, 0};
+    for (int fb = 0; fb < 4; fb++)
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++) {
-                    const int ao = (16 * mb + lr) * kPb + 32 * kb + 8 * lg;
-                    const int bo = (16 * nb + lr) * kPb + 32 * kb + 8 * lg;
-                    acc = mfma3(frag(h1h + ao), frag(h1l + ao), frag(w2h + bo), frag(w2l + bo), acc);
-                }
-                const int n = 16 * nb + lr;
+        for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-                for (int t = 0; t < 4; t++) z2s[(16 * mb + 4 * lg + t) * kPf + n] = acc[t] + W[MP_B2 + n];
+            for (int i = 0; i < 8; i++) {
+                __bf16 hi, lo;
+                split_bf16(w2s[(16 * fb + lr) * kRow + 32 * kb + 8 * lg + i], hi, lo);
+                w2h[fb][kb][i] = hi; w2l[fb][kb][i] = lo;
+                split_bf16(w2s[(32 * kb + 8 * lg + i) * kRow + 16 * fb + lr], hi, lo);
+                w2th[fb][kb][i] = hi; w2tl[fb][kb][i] = lo;
             }
-        __syncthreads();
-        // output layer, loss and dZ2 (lane = sample)
-        float o0 = W[MP_B3], o1 = W[MP_B3 + 1];
-        for (int n = 0; n < 64; n++) {
-            const float h = gelu_only(z2s[l * kPf + n]);
-            o0 += W[MP_W3 + n] * h;
-            o1 += W[MP_W3 + 64 + n] * h;
-        }
-        const float e0 = valid ? o0 - y0 : 0.0f, e1 = valid ? o1 - y1 : 0.0f;
-        loss += e0 * e0 + e1 * e1;
-        const float d0 = 2.0f * e0 * P.inv_batch, d1 = 2.0f * e1 * P.inv_batch;
-        dos[l * 2] = d0; dos[l * 2 + 1] = d1;
-        for (int n = 0; n < 64; n++) {
-            float dg;
-            const float h = gelu_f(z2s[l * kPf + n], dg);
-            const float dz = (d0 * W[MP_W3 + n] + d1 * W[MP_W3 + 64 + n]) * dg;
-            __bf16 hi, lo;
-            split_bf16(dz, hi, lo);
-            d2h[l * kPb + n] = hi; d2l[l * kPb + n] = lo;
-            d2th[n * kPb + l] = hi; d2tl[n * kPb + l] = lo;
-            z2s[l * kPf + n] = h;
-        }
-        __syncthreads();
-        // per-feature sums over the samples (lane = feature j)
-        for (int s = 0; s < 64; s++) {
-            const float h = z2s[s * kPf + l];
-            gw3[0] += dos[2 * s] * h;
-            gw3[1] += dos[2 * s + 1] * h;
-            gb2 += (float)d2h[s * kPb + l] + (float)d2l[s * kPb + l];
-        }
-        gb3[0] += d0;
-        gb3[1] += d1;
-        // dH1 = dZ2 W2 -> dZ1 = dH1 * gelu'(z1), in place of z1
+    __syncthreads();
+
+    const float b3 = W[MP_B3 + (lg & 1)];  // output lg of sample lr (lanes below 32)
+    v4f gw2[4];
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+    for (int nb = 0; nb < 4; nb++) gw2[nb] = (v4f){0, 0, 0, 0};
+    float s0 = 0, s1 = 0;       // wave 0: dW3, wave 1: db2, wave 2: dW1[0], [1], wave 3: dW1[2], db1
+    float gb3 = 0, loss = 0;    // sample lr: db3 of output lg, and the loss (lg = 0)
+
+    for (int c = 0; c < P.chunks; c++) {
+        if (l < 16) {
+            float *d = recs + (16 * wv + l) * 8;
+            d[0] = rc[0]; d[1] = rc[1]; d[2] = rc[2];
+            d[3] = valid ? 1.0f : 0.0f;
+            d[4] = (rc[3] - P.norm[0]) / P.norm[1];
+            d[5] = (rc[4] - P.norm[2]) / P.norm[3];
+            if (c + 1 < P.chunks) fetch(c + 1);
+        }
+        wave_sync();
+        // layer 1, rows
+        v8bf ah[2], al[2];
+        {
+            const float4 x = *reinterpret_cast<const float4 *>(recs + (16 * wv + lr) * 8);
 #pragma unroll
-            for (int nb = 0; nb < 4; nb++) {
-                v4f acc = {0, 0, 0, 0};
+            for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++) {
-                    const int ao = (16 * mb + lr) * kPb + 32 * kb + 8 * lg;
-                    const int bo = (16 * nb + lr) * kPb + 32 * kb + 8 * lg;
-                    acc = mfma3(frag(d2h + ao), frag(d2l + ao), frag(w2th + bo), frag(w2tl + bo), acc);
+                for (int i = 0; i < 8; i++) {
+                    const float4 w = *reinterpret_cast<const float4 *>(&w1s[4 * (32 * kb + 8 * lg + i)]);
+                    const float z = w.w + w.x * x.x + w.y * x.y + w.z * x.z;
+                    __bf16 hi, lo;
+                    split_bf16(gelu_only(z), hi, lo);
+                    ah[kb][i] = hi;
+                    al[kb][i] = lo;
                 }
-                const int k = 16 * nb + lr;
+        }
+        // layer 2, cols: Z2[s][n] = sum_k H1[s][k] W2[n][k]
+        float dg2[4][4];
 #pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const int s = 16 * mb + 4 * lg + t;
-                    float dg;
-                    (void)gelu_f(z1s[s * kPf + k], dg);
-                    z1s[s * kPf + k] = acc[t] * dg;
-                }
+        for (int fb = 0; fb < 4; fb++) {
+            v4f acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) acc = mfma3(ah[kb], al[kb], w2h[fb][kb], w2l[fb][kb], acc);
+            const float b2 = w3s[4 * (16 * fb + lr)];
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                h2s[(16 * wv + 4 * lg + t) * kRow + 16 * fb + lr] = gelu_f(acc[t] + b2, dg2[fb][t]);
+        }
+        wave_sync();
+        // the outputs, features in order (lane = sample lr, output lg), the
+        // loss and its derivative
+        if (l < 32) {
+            float o = b3;
+            const float *h = h2s + (16 * wv + lr) * kRow;
+            for (int n = 0; n < 64; n += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>(h + n);
+                o += w3s[4 * n + 1 + lg] * v.x;
+                o += w3s[4 * n + 5 + lg] * v.y;
+                o += w3s[4 * n + 9 + lg] * v.z;
+                o += w3s[4 * n + 13 + lg] * v.w;
             }
-        // dW2 += dZ2^T H1: rows n, columns k, sum over the samples
+            const float *d = recs + (16 * wv + lr) * 8;
+            const float e = d[3] != 0.0f ? o - d[4 + lg] : 0.0f;
+            dos[2 * (16 * wv + lr) + lg] = 2.0f * e * P.inv_batch;
+            gb3 = __builtin_fmaf(2.0f * e, P.inv_batch, gb3);
+            loss += e * e;
+        }
+        wave_sync();
+        // dZ2, cols: to LDS as rows (for dH1) and transposed (for dW2)
+        float dt[4][2];
 #pragma unroll
-        for (int mb = 0; mb < 4; mb++)
+        for (int t = 0; t < 4; t++) {
+            dt[t][0] = dos[2 * (16 * wv + 4 * lg + t)];
+            dt[t][1] = dos[2 * (16 * wv + 4 * lg + t) + 1];
+        }
 #pragma unroll
-            for (int nb = 0; nb < 4; nb++)
+        for (int fb = 0; fb < 4; fb++) {
+            const float4 e = *reinterpret_cast<const float4 *>(&w3s[4 * (16 * fb + lr)]);
+            v4bf vh, vl;
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++) {
-                    const int ao = (16 * mb + lr) * kPb + 32 * kb + 8 * lg;
-                    const int bo = (16 * nb + lr) * kPb + 32 * kb + 8 * lg;
-                    gw2[mb][nb] = mfma3(frag(d2th + ao), frag(d2tl + ao), frag(h1th + bo), frag(h1tl + bo), gw2[mb][nb]);
-                }
+            for (int t = 0; t < 4; t++) {
+                const float dz = (dt[t][0] * e.y + dt[t][1] * e.z) * dg2[fb][t];
+                __bf16 hi, lo;
+                split_bf16(dz, hi, lo);
+                vh[t] = hi;
+                vl[t] = lo;
+                dzs[(16 * wv + 4 * lg + t) * kRow + 16 * fb + lr] =
+                    (uint32_t)__builtin_bit_cast(uint16_t, hi) | ((uint32_t)__builtin_bit_cast(uint16_t, lo) << 16);
+            }
+            *reinterpret_cast<v4bf *>(&d2th[(16 * fb + lr) * kPb + 16 * wv + 4 * lg]) = vh;
+            *reinterpret_cast<v4bf *>(&d2tl[(16 * fb + lr) * kPb + 16 * wv + 4 * lg]) = vl;
+        }
+        wave_sync();
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+            const uint4 *q = reinterpret_cast<const uint4 *>(&dzs[(16 * wv + lr) * kRow + 32 * kb + 8 * lg]);
+            const uint4 q0 = q[0], q1 = q[1];
+            const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                ah[kb][i] = __builtin_bit_cast(__bf16, (uint16_t)(w[i] & 0xffffu));
+                al[kb][i] = __builtin_bit_cast(__bf16, (uint16_t)(w[i] >> 16));
+            }
+        }
+        wave_sync();
+        // H1 again, cols; dH1 = dZ2 W2 -> dZ1 = dH1 GELU'(z1)
+        float4 xt[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) xt[t] = *reinterpret_cast<const float4 *>(recs + (16 * wv + 4 * lg + t) * 8);
+#pragma unroll
+        for (int fb = 0; fb < 4; fb++) {
+            v4f acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) acc = mfma3(ah[kb], al[kb], w2th[fb][kb], w2tl[fb][kb], acc);
+            const float4 w = *reinterpret_cast<const float4 *>(&w1s[4 * (16 * fb + lr)]);
+            v4bf vh, vl;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                float dg;
+                const float z = w.w + w.x * xt[t].x + w.y * xt[t].y + w.z * xt[t].z;
+                __bf16 hi, lo;
+                split_bf16(gelu_f(z, dg), hi, lo);
+                vh[t] = hi;
+                vl[t] = lo;
+                dz1s[(16 * wv + 4 * lg + t) * kRow + 16 * fb + lr] = acc[t] * dg;
+            }
+            *reinterpret_cast<v4bf *>(&h1th[(16 * fb + lr) * kPb + 16 * wv + 4 * lg]) = vh;
+            *reinterpret_cast<v4bf *>(&h1tl[(16 * fb + lr) * kPb + 16 * wv + 4 * lg]) = vl;
+        }
         __syncthreads();
-        for (int s = 0; s < 64; s++) {
-            const float dz = z1s[s * kPf + l];
-            gw1[0] += dz * xs[s * 4 + 0];
-            gw1[1] += dz * xs[s * 4 + 1];
-            gw1[2] += dz * xs[s * 4 + 2];
-            gb1 += dz;
+        // sums over the batch: dW2 += dZ2^T H1, rows n of block wv, ...
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                const int ao = (16 * wv + lr) * kPb + 32 * kb + 8 * lg, bo = (16 * nb + lr) * kPb + 32 * kb + 8 * lg;
+                gw2[nb] = mfma3(frag(d2th + ao), frag(d2tl + ao), frag(h1th + bo), frag(h1tl + bo), gw2[nb]);
+            }
+        // ... and the per-feature sums (lane = feature), samples in order
+        if (wv == 0) {
+#pragma unroll 8
+            for (int s = 0; s < 64; s++) {
+                const float h = h2s[s * kRow + l];
+                s0 += dos[2 * s] * h;
+                s1 += dos[2 * s + 1] * h;
+            }
+        } else if (wv == 1) {
+#pragma unroll 4
+            for (int s = 0; s < 64; s += 4) {
+                const v4bf vh = *reinterpret_cast<const v4bf *>(&d2th[l * kPb + s]);
+                const v4bf vl = *reinterpret_cast<const v4bf *>(&d2tl[l * kPb + s]);
+#pragma unroll
+                for (int t = 0; t < 4; t++) s0 += (float)vh[t] + (float)vl[t];
+            }
+        } else if (wv == 2) {
+#pragma unroll 8
+            for (int s = 0; s < 64; s++) {
+                const float dz = dz1s[s * kRow + l];
+                s0 += dz * recs[8 * s];
+                s1 += dz * recs[8 * s + 1];
+            }
+        } else {
+#pragma unroll 8
+            for (int s = 0; s < 64; s++) {
+                const float dz = dz1s[s * kRow + l];
+                s0 += dz * recs[8 * s + 2];
+                s1 += dz;
+            }
         }
         __syncthreads();
     }
     float *out = P.part + (int64_t)blockIdx.x * (kMlpParams + 1);
-    out[MP_W1 + 3 * l] = gw1[0];
-    out[MP_W1 + 3 * l + 1] = gw1[1];
-    out[MP_W1 + 3 * l + 2] = gw1[2];
-    out[MP_B1 + l] = gb1;
-    out[MP_B2 + l] = gb2;
-    out[MP_W3 + l] = gw3[0];
-    out[MP_W3 + 64 + l] = gw3[1];
 #pragma unroll
-    for (int mb = 0; mb < 4; mb++)
+    for (int nb = 0; nb < 4; nb++)
 #pragma unroll
-        for (int nb = 0; nb < 4; nb++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) out[MP_W2 + (16 * mb + 4 * lg + t) * 64 + 16 * nb + lr] = gw2[mb][nb][t];
-    // db3 and the loss: sums over the lanes (samples)
-    float s0 = gb3[0], s1 = gb3[1], sl = loss;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        s0 += __shfl_xor(s0, o, 64);
-        s1 += __shfl_xor(s1, o, 64);
-        sl += __shfl_xor(sl, o, 64);
+        for (int t = 0; t < 4; t++) out[MP_W2 + (16 * wv + 4 * lg + t) * 64 + 16 * nb + lr] = gw2[nb][t];
+    if (wv == 0) {
+        out[MP_W3 + l] = s0;
+        out[MP_W3 + 64 + l] = s1;
+    } else if (wv == 1) {
+        out[MP_B2 + l] = s0;
+    } else if (wv == 2) {
+        out[MP_W1 + 3 * l] = s0;
+        out[MP_W1 + 3 * l + 1] = s1;
+    } else {
+        out[MP_W1 + 3 * l + 2] = s0;
+        out[MP_B1 + l] = s1;
     }
-    if (l == 0) {
-        out[MP_B3] = s0;
-        out[MP_B3 + 1] = s1;
-        out[kMlpParams] = sl;
+    // db3 and the loss: sums over the samples
+    if (l < 32) {
+        dos[2 * (16 * wv + lr) + lg] = gb3;
+        recs[8 * (16 * wv + lr) + lg] = loss;
+    }
+    __syncthreads();
+    if (wv == 0) {
+        float a0 = dos[2 * l], a1 = dos[2 * l + 1], sl = recs[8 * l] + recs[8 * l + 1];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            a0 += __shfl_xor(a0, o, 64);
+            a1 += __shfl_xor(a1, o, 64);
+            sl += __shfl_xor(sl, o, 64);
+        }
+        if (l == 0) {
+            out[MP_B3] = a0;
+            out[MP_B3 + 1] = a1;
+            out[kMlpParams] = sl;
+        }
     }
 }
 
-// Sum of the workgroup partials (fixed order) and one Adam step.
-__global__ void __launch_bounds__(256)
+// Sum of the workgroup partials (in order) and one Adam step: a block takes 64
+// parameters; its waves bring up to kAdamTile partials to LDS at once, then
+// the first one adds them.  (One thread per parameter walking 512 partials in
+// memory took 118 us, this 6.7.)
+constexpr int kAdamTile = 512;
+__global__ void __launch_bounds__(kAdamBlock)
 k_mlp_adam(float *params, float *m, float *v, const float *part, int nwg, float lr, float b1, float b2,
            float eps, float bc1, float bc2, float *grad_out, float *loss_out)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > kMlpParams) return;
+    __shared__ float tile[kAdamTile][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    const bool in = p <= kMlpParams, mine = wv == 0 && p < kMlpParams;
+    float m0 = 0, v0 = 0, p0 = 0;
+    if (mine) { m0 = m[p]; v0 = v[p]; p0 = params[p]; }
     float g = 0.0f;
-    for (int w = 0; w < nwg; w++) g += part[(int64_t)w * (kMlpParams + 1) + p];
+    for (int w0 = 0; w0 < nwg; w0 += kAdamTile) {
+        constexpr int nw = kAdamBlock / 64, per = kAdamTile / nw;
+        float x[per];
+#pragma unroll
+        for (int j = 0; j < per; j++) {
+            const int w = w0 + wv + j * nw;
+            x[j] = (in && w < nwg) ? part[(int64_t)w * (kMlpParams + 1) + p] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < per; j++) tile[wv + j * nw][lane] = x[j];
+        __syncthreads();
+        if (wv == 0) {
+            const int n = nwg - w0 < kAdamTile ? nwg - w0 : kAdamTile;
+            int j = 0;
+            for (; j + 32 <= n; j += 32) {
+                float y[32];
+#pragma unroll
+                for (int u = 0; u < 32; u++) y[u] = tile[j + u][lane];
+#pragma unroll
+                for (int u = 0; u < 32; u++) g += y[u];
+            }
+            for (; j < n; j++) g += tile[j][lane];
+        }
+        __syncthreads();
+    }
+    if (wv != 0 || p > kMlpParams) return;
     if (p == kMlpParams) {
         if (loss_out) *loss_out = g;
         return;
     }
     if (grad_out) grad_out[p] = g;
     if (lr == 0.0f) return;
-    const float mm = b1 * m[p] + (1.0f - b1) * g;
-    const float vv = b2 * v[p] + (1.0f - b2) * g * g;
+    const float mm = b1 * m0 + (1.0f - b1) * g;
+    const float vv = b2 * v0 + (1.0f - b2) * g * g;
     m[p] = mm;
     v[p] = vv;
-    params[p] -= lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
+    params[p] = p0 - lr * (mm / bc1) / (sqrtf(vv / bc2) + eps);
 }
 
 // Raw network outputs for n feature vectors (tests and validation).
@@ -338,7 +492,7 @@ hipError_t launch_mlp_train(const float *params, const float *samples, int64_t n
     P.params = params; P.samples = samples; P.n = n; P.part = part;
     for (int i = 0; i < 4; i++) P.norm[i] = norm[i];
     P.inv_batch = inv_batch; P.seed = seed; P.step = step; P.chunks = chunks; P.random = random;
-    hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(64), 0, st, P);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(kTrainBlock), 0, st, P);
     return hipGetLastError();
 }
 
@@ -346,8 +500,8 @@ hipError_t launch_mlp_adam(float *params, float *m, float *v, const float *part,
                            float b2, float eps, float bc1, float bc2, float *grad_out, float *loss_out,
                            hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, st, params, m, v, part, nwg,
-                       lr, b1, b2, eps, bc1, bc2, grad_out, loss_out);
+    hipLaunchKernelGGL(k_mlp_adam, dim3(kMlpParams / 64 + 1), dim3(kAdamBlock), 0, st, params, m, v, part,
+                       nwg, lr, b1, b2, eps, bc1, bc2, grad_out, loss_out);
     return hipGetLastError();
 }
 

@@ -38,6 +38,7 @@ constexpr float kSurLnRMin = -3.91202300542814606f;  // ln(0.02)
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 
 // The network's arithmetic is contracted to FMAs (the rest of the library
 // keeps multiply and add separate).
@@ -93,7 +94,7 @@ __device__ __forceinline__ void sur_envelope(float au, float av, float r, float 
 }
 
 constexpr int kPb = 72;  // LDS row pitch of bf16 tiles (144 B): fragment reads spread over banks
-constexpr int kPf = 65;  // LDS row pitch of FP32 rows
+constexpr int kAdamBlock = 1024;
 
 __device__ __forceinline__ v4f mfma3(v8bf ah, v8bf al, v8bf bh, v8bf bl, v4f c)
 {
