@@ -29,7 +29,7 @@
 //
 // Near the beam the kicks take Weideman's rational approximation instead
 // (J. A. C. Weideman, SIAM J. Numer. Anal. 31 (1994) 1497-1518; be_field
-// below), one division and 40 complex multiply-adds per point.  FP64
+// below), one reciprocal and 40 coefficients at two fma each per point.  FP64
 // throughout: the far-field and lower-half-plane forms cancel.
 #pragma once
 
@@ -45,12 +45,16 @@ namespace cts {
 // code, so every translation unit that evaluates the kick field holds its
 // own copy of the table and exports an upload function that fills it;
 // cts_create calls each of them.
+// The kick field's exponential reads its constants from the same table
+// (log2 e, the two parts of ln 2, the Taylor coefficients 1/13! .. 1/0!).
 constexpr int kWeidN = 40;
-static __constant__ double c_weid[kWeidN + 1];  // p's coefficients, highest degree first, then L
+constexpr int kExpAt = kWeidN + 1, kExpDeg = 13;
+constexpr int kFadConst = kExpAt + 3 + kExpDeg + 1;
+static __constant__ double c_weid[kFadConst];  // p's coefficients, highest degree first, then L, then exp's
 
 // Host: the table above.
 struct FadTables {
-    double weid[kWeidN + 1];
+    double weid[kFadConst];
 };
 inline void build_fad_tables(FadTables &t)
 {
@@ -74,6 +78,14 @@ inline void build_fad_tables(FadTables &t)
         t.weid[N - m] = acc / M2;
     }
     t.weid[N] = L;
+    t.weid[kExpAt] = 1.4426950408889634;
+    t.weid[kExpAt + 1] = 0x1.62e42fefa38p-1;     // ln 2 to 42 bits: k times it is exact for |k| < 2^11
+    t.weid[kExpAt + 2] = 0x1.ef35793c7673p-45;   // the rest
+    double f1 = 1.0;
+    for (int n = 0; n <= kExpDeg; n++) {
+        if (n > 0) f1 *= n;
+        t.weid[kExpAt + 3 + kExpDeg - n] = 1.0 / f1;
+    }
 }
 
 constexpr double kIsPi = 0.56418958354775628694807945156;  // 1/sqrt(pi)
@@ -468,55 +480,86 @@ __device__ __forceinline__ void w_weideman(const double *zr, const double *zi, d
     }
 }
 
+// exp(t) for t <= 0: t = k ln 2 + r, |r| <= ln 2 / 2, Taylor's polynomial of
+// degree 13 in r (the next term is below 5e-18), every constant a scalar
+// operand (the library's exp keeps its constants in vector registers across
+// the kick loops).  Below t = -1000 the result is 0 either way.
+__device__ __forceinline__ double exp_neg(double t)
+{
+    const cdptr ce = reload((uint64_t)(uintptr_t)c_weid) + kExpAt;
+    t = fmax(t, -1000.0);
+    const double k = rint(t * ce[0]);
+    const double r = fma(-k, ce[2], fma(-k, ce[1], t));
+    double p = ce[3];
+#pragma unroll
+    for (int n = 1; n <= kExpDeg; n++) p = fma_vvs(r, p, ce[3 + n]);
+    return ldexp(p, (int)k);
+}
+
 // w(z) outside the kick region (x >= 100 or y >= 1000, both >= 0), as
-// faddeeva_w_q1 evaluates it there: erfcx on the imaginary axis, otherwise
+// faddeeva_w_q1 evaluates it there: on the imaginary axis (y >= 1000) erfcx by
+// its continued fraction, otherwise
 // the continued fraction (at most 4 levels for |z|^2 >= 1e4) or the
 // asymptotic form; exp(-z^2) has underflowed.  Few registers, so the kick
 // loops keep their occupancy.
 __device__ __forceinline__ void w_far(double x, double y, double &wr, double &wi)
 {
-    if (x == 0.0) { wr = cts_erfcx(y); wi = 0.0; return; }
     if (std::isinf(x) || std::isinf(y)) { wr = 0.0; wi = 0.0; return; }
+    if (x == 0.0) {
+        double t = y;
+#pragma nounroll
+        for (int k = 24; k >= 1; k--) t = y + (0.5 * k) / t;
+        wr = kIsPi / t;
+        wi = 0.0;
+        return;
+    }
     if (x >= 1e7 || y >= 1e7) { fad_asymptotic(x, y, wr, wi); return; }
     fad_cf(x, y, fad_cf_depth(x * x + y * y), wr, wi);
 }
 
-// ion_field with the beam's constants from be_plan.
+// ion_field with the beam's constants from be_plan (scalars where the caller
+// reads them so).  Both w(z) of the formula run side by side: with the rare
+// far-field branch reduced to short loops and exp's constants as scalars the
+// kernels have the registers for it, and a small launch, which has one wave
+// per SIMD, waits half as long on the recurrences.
 __device__ __forceinline__ void be_field(double x, double y, const BeField &F, double &fx, double &fy)
 {
+    if (F.mode == 2) {
+        gaussian_field(x, y, F.sx, fx, fy);
+    } else {
+        const bool sw = F.mode == 1;
+        const double X = sw ? y : x, Y = sw ? x : y;
+        const double ax = fabs(X), ay = fabs(Y);
+        double zr[2], zi[2], wr[2], wi[2];
+        zr[0] = ax * F.isig;
+        zi[0] = ay * F.isig;
+        zr[1] = F.r * zr[0];
+        zi[1] = zi[0] * F.ir;
+        // Weideman's approximation for both points; a point outside the kick
+        // region (rare: far from the beam) takes the far-field form instead
+        w_weideman<2>(zr, zi, wr, wi);
+        if (!w_kick_region(zr[0], zi[1])) {  // the larger of each
+#pragma nounroll
+            for (int q = 0; q < 2; q++) {
+                const double fr = q ? zr[1] : zr[0], fi = q ? zi[1] : zi[0];
+                if (w_kick_region(fr, fi)) continue;
+                double vr, vi;
+                w_far(fr, fi, vr, vi);
+                if (q) { wr[1] = vr; wi[1] = vi; }
+                else { wr[0] = vr; wi[0] = vi; }
+            }
+        }
+        const double w3 = -exp_neg(-(ax * ax) * F.hx - (ay * ay) * F.hy);
+        const double w0r = F.coeff * (wr[0] + w3 * wr[1]);
+        const double w0i = F.coeff * (wi[0] + w3 * wi[1]);
+        const double fX = X <= 0 ? -w0i : w0i, fY = Y <= 0 ? -w0r : w0r;
+        fx = sw ? fY : fX;
+        fy = sw ? fX : fY;
+    }
     if (fabs(x) * F.isx + fabs(y) * F.isy < 1.0E-5) {
         fx = 0;
         fy = 0;
-        return;
     }
-    if (F.mode == 2) {
-        gaussian_field(x, y, F.sx, fx, fy);
-        return;
-    }
-    const bool sw = F.mode == 1;
-    const double X = sw ? y : x, Y = sw ? x : y;
-    const double ax = fabs(X), ay = fabs(Y);
-    double zr[2], zi[2], wr[2], wi[2];
-    zr[0] = ax * F.isig;
-    zi[0] = ay * F.isig;
-    zr[1] = F.r * zr[0];
-    zi[1] = zi[0] * F.ir;
-    // Weideman's approximation for both points; a point outside the kick
-    // region (rare: far from the beam) takes the far-field form instead
-    // one point after the other: four waves per SIMD interleave enough
-    // work, and the single recurrence needs fewer registers (fewer spills
-    // in the ion turn's passage loop) than the two side by side
-#pragma nounroll
-    for (int q = 0; q < 2; q++) w_weideman<1>(zr + q, zi + q, wr + q, wi + q);
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-        if (!w_kick_region(zr[q], zi[q])) w_far(zr[q], zi[q], wr[q], wi[q]);
-    const double w3 = -exp(-(ax * ax) * F.hx - (ay * ay) * F.hy);
-    const double w0r = F.coeff * (wr[0] + w3 * wr[1]);
-    const double w0i = F.coeff * (wi[0] + w3 * wi[1]);
-    const double fX = X <= 0 ? -w0i : w0i, fY = Y <= 0 ? -w0r : w0r;
-    fx = sw ? fY : fX;
-    fy = sw ? fX : fY;
 }
 
 // Bunch::GaussianField (src/Bunch.cpp:202-211)
@@ -524,7 +567,7 @@ __device__ inline void gaussian_field(double posx, double posy, double sx, doubl
 {
     const double r2 = posx * posx + posy * posy;
     const double sigma2 = sx * sx;
-    const double e = 1 - exp(-r2 / 2 / sigma2);
+    const double e = 1 - exp_neg(-r2 / 2 / sigma2);
     fx = -posx / r2 * e;
     fy = -posy / r2 * e;
 }

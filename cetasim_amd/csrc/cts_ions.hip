@@ -450,7 +450,7 @@ k_compact_scatter(IonCompactParams P)
 // this translation unit's copy of the Faddeeva tables
 hipError_t upload_faddeeva_tables_ions(const FadTables &t)
 {
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, (kWeidN + 1) * sizeof(double));
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, kFadConst * sizeof(double));
 }
 
 // wave_bound: a host bound of the segment's waves; the kernel reads the

@@ -17,7 +17,7 @@ namespace cts {
 
 hipError_t upload_faddeeva_tables(const FadTables &t)
 {
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, (kWeidN + 1) * sizeof(double));
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, kFadConst * sizeof(double));
 }
 
 // Streaming (nontemporal) global accesses.

@@ -527,7 +527,7 @@ hipError_t launch_mlp_field_error(const float *W, const double *exact, int64_t n
 
 hipError_t upload_faddeeva_tables_mlp(const FadTables &t)
 {
-    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, (kWeidN + 1) * sizeof(double));
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_weid), t.weid, kFadConst * sizeof(double));
 }
 
 }  // namespace cts
