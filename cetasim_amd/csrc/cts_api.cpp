@@ -84,7 +84,8 @@ struct IonIp {
     double *d_coeff = nullptr, *d_dt = nullptr;  // [nb][CTS_MAX_SPECIES], [nb]
     unsigned long long *d_acc = nullptr;  // kIonReplicas + 1 copies of [nspec][nb][kIonAcc][3]
     uint32_t *d_wcnt = nullptr;  // [nspec][wstride]: survivors per wave of a segment
-    uint32_t *d_wofs = nullptr;  // [wstride]: their prefix sums
+    uint32_t *d_wcoarse = nullptr;  // [2][nspec][cstride]: survivors of kIonCoarse cohorts, by segment parity
+    int64_t cstride = 0;
     std::vector<double> q;       // host copy of d_q: [nb][nspec] macro-ion charge per passage
 };
 
@@ -159,6 +160,7 @@ struct cts_handle {
     int32_t *d_item_bunch = nullptr, *d_item_first = nullptr;
     int nitem = 0;
     double *d_ion_bview = nullptr;
+    double *d_ion_bplan = nullptr;  // the bunches' field constants ([nb][kBePlan])
     std::vector<IonIp> ips;
     // d_cur holds the moments of the present coordinates
     bool cur_valid = false;
@@ -301,7 +303,7 @@ void free_bunch_state(cts_handle *h)
                     h->d_seg_begin, h->d_seg_end, h->d_bunch_off, h->d_bunch_count,
                     h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part, h->d_shift,
                     h->d_cur, h->d_hist, h->d_sigz, h->d_zrange, h->d_noise, h->d_ion_e, h->d_ion_bview,
-                    h->d_ion_f, h->d_item_bunch, h->d_item_first,
+                    h->d_ion_f, h->d_ion_bplan, h->d_item_bunch, h->d_item_first,
                     h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev,
                     h->d_edges_now, h->d_table, h->d_scale,
                     h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order, h->d_seg_step};
@@ -315,7 +317,7 @@ void free_bunch_state(cts_handle *h)
     h->d_seg_begin = h->d_seg_end = h->d_bunch_off = h->d_bunch_count = nullptr;
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = nullptr;
     h->d_seg_part = h->d_shift = h->d_sigz = h->d_zrange = h->d_noise = h->d_ion_e = h->d_ion_bview = nullptr;
-    h->d_ion_f = nullptr;
+    h->d_ion_f = h->d_ion_bplan = nullptr;
     h->d_item_bunch = h->d_item_first = nullptr;
     h->d_cur = h->d_hist = nullptr;
     h->d_bhist = nullptr;
@@ -896,7 +898,7 @@ void free_ion_ip(IonIp &I)
             if (I.d_alive[b][p]) (void)hipFree(I.d_alive[b][p]);
         }
     void *ptrs[] = {I.d_len, I.d_nalive, I.d_mean, I.d_smax, I.d_q, I.d_cloud, I.d_coeff, I.d_dt, I.d_acc,
-                    I.d_wcnt, I.d_wofs};
+                    I.d_wcnt, I.d_wcoarse};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     I = IonIp{};
@@ -949,14 +951,25 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
     const cts_section &S = h->secs[k];
     const int64_t nacc = (int64_t)Ip.nspec * h->nb * kIonAcc * 3;
     int64_t *len0 = Ip.d_len + 2 * CTS_MAX_SPECIES;
+    const int64_t ncoarse = Ip.nspec * Ip.cstride;  // of one segment parity
     {
+        IonPrepParams pp;
+        pp.cur = h->d_cur;
+        pp.beta_x = S.beta_x; pp.beta_y = S.beta_y;
+        pp.bview = h->d_ion_bview; pp.bplan = h->d_ion_bplan; pp.size_max = Ip.d_smax;
+        pp.fb_count = h->d_fb_count;
+        pp.len = Ip.d_len + Ip.buf * CTS_MAX_SPECIES;
+        pp.len0 = len0;
+        pp.wcoarse = Ip.d_wcoarse;
+        pp.ncoarse = (int32_t)(2 * ncoarse);
+        pp.nb = h->nb; pp.nspec = Ip.nspec;
         TimedScope ts(h, "ion_prep");
-        HIPCHK(launch_ion_prep(h->d_cur, h->nb, S.beta_x, S.beta_y, h->d_ion_bview, Ip.d_smax, h->d_fb_count,
-                               Ip.d_len + Ip.buf * CTS_MAX_SPECIES, len0, Ip.nspec, h->stream));
+        HIPCHK(launch_ion_prep(pp, h->stream));
     }
     IonTurnParams P;
     std::memset(&P, 0, sizeof P);
     P.bview = h->d_ion_bview;
+    P.bplan = h->d_ion_bplan;
     P.size_max = Ip.d_smax;
     P.coeffI = Ip.d_coeff;
     P.dt = Ip.d_dt;
@@ -964,6 +977,7 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
     P.acc_stride = nacc;
     P.wcnt = Ip.d_wcnt;
     P.wcnt_stride = Ip.wstride;
+    P.wcoarse_stride = Ip.cstride;
     P.sur_params = nullptr;
     if (h->sur && (h->sur_mode & 1)) sur_export(h->sur, &P.sur_params, &P.sur_norm);
     P.loss_boundary = I.loss_boundary;
@@ -994,7 +1008,9 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
             P.vy[p] = Ip.d_ion[buf][p][3];
             P.alive[p] = Ip.d_alive[buf][p];
         }
+        const int par = ja / kIonSegment % 2;
         P.len = Ip.d_len + buf * CTS_MAX_SPECIES;
+        P.wcoarse = Ip.d_wcoarse + par * ncoarse;
         P.j_begin = ja;
         P.j_end = jb;
         const int64_t waves = (ub + 63) / 64 + (int64_t)(jb - ja) * P.w_new;
@@ -1003,24 +1019,29 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
             HIPCHK(launch_ion_turn(P, Ip.nspec, waves, h->stream));
         }
         ub = std::min<int64_t>(ub + (int64_t)(jb - ja) * I.n_new, Ip.cap);
+        IonCompactParams c;
+        std::memset(&c, 0, sizeof c);
         for (int p = 0; p < Ip.nspec; p++) {
-            IonCompactParams c;
-            c.x = Ip.d_ion[buf][p][0]; c.y = Ip.d_ion[buf][p][1];
-            c.vx = Ip.d_ion[buf][p][2]; c.vy = Ip.d_ion[buf][p][3];
-            c.alive = Ip.d_alive[buf][p];
-            c.ox = Ip.d_ion[1 - buf][p][0]; c.oy = Ip.d_ion[1 - buf][p][1];
-            c.ovx = Ip.d_ion[1 - buf][p][2]; c.ovy = Ip.d_ion[1 - buf][p][3];
-            c.oalive = Ip.d_alive[1 - buf][p];
-            c.len = Ip.d_len + buf * CTS_MAX_SPECIES + p;
-            c.new_len = Ip.d_len + (1 - buf) * CTS_MAX_SPECIES + p;
-            c.wcnt = Ip.d_wcnt + p * Ip.wstride;
-            c.wofs = Ip.d_wofs;
-            c.cap = Ip.cap;
-            c.n_new = I.n_new;
-            c.w_new = P.w_new;
-            c.nseg = jb - ja;
+            c.x[p] = P.x[p]; c.y[p] = P.y[p]; c.vx[p] = P.vx[p]; c.vy[p] = P.vy[p];
+            c.alive[p] = P.alive[p];
+            c.ox[p] = Ip.d_ion[1 - buf][p][0]; c.oy[p] = Ip.d_ion[1 - buf][p][1];
+            c.ovx[p] = Ip.d_ion[1 - buf][p][2]; c.ovy[p] = Ip.d_ion[1 - buf][p][3];
+            c.oalive[p] = Ip.d_alive[1 - buf][p];
+        }
+        c.len = P.len;
+        c.new_len = Ip.d_len + (1 - buf) * CTS_MAX_SPECIES;
+        c.wcnt = Ip.d_wcnt;
+        c.wcnt_stride = Ip.wstride;
+        c.wcoarse = P.wcoarse;
+        c.wcoarse_next = Ip.d_wcoarse + (1 - par) * ncoarse;
+        c.wcoarse_stride = Ip.cstride;
+        c.cap = Ip.cap;
+        c.n_new = I.n_new;
+        c.w_new = P.w_new;
+        c.nseg = jb - ja;
+        {
             TimedScope ts(h, "ion_compact");
-            HIPCHK(launch_ion_compact(c, waves, h->stream));
+            HIPCHK(launch_ion_compact(c, Ip.nspec, waves, h->stream));
         }
         Ip.buf = 1 - buf;
     }
@@ -1210,7 +1231,8 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
         }
         h->nitem = first[nb];
         if ((rc = dalloc(&h->d_item_bunch, bunch.size())) || (rc = dalloc(&h->d_item_first, first.size())) ||
-            (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)))
+            (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)) ||
+            (rc = dalloc(&h->d_ion_bplan, (size_t)nb * kBePlan)))
             return rc;
         HIPCHK(hipMemcpy(h->d_item_bunch, bunch.data(), bunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(h->d_item_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -2180,6 +2202,7 @@ int cts_set_ions_ip(cts_handle *h, int32_t k, const cts_ion_config *cfg)
     Ip.cfg = *cfg;
     Ip.cap = cap;
     Ip.wstride = wstride;
+    Ip.cstride = wstride / (kIonCoarse * kIonCohort) + 1;
     auto fail_free = [&](int code) {
         free_ion_ip(Ip);
         return code;
@@ -2196,7 +2219,8 @@ int cts_set_ions_ip(cts_handle *h, int32_t k, const cts_ion_config *cfg)
         (rc = dalloc(&Ip.d_cloud, (size_t)h->nb * CTS_MAX_SPECIES * 6)) ||
         (rc = dalloc(&Ip.d_coeff, (size_t)h->nb * CTS_MAX_SPECIES)) || (rc = dalloc(&Ip.d_dt, (size_t)h->nb)) ||
         (rc = dalloc(&Ip.d_acc, (size_t)(kIonReplicas + 1) * cfg->nspec * h->nb * kIonAcc * 3)) ||
-        (rc = dalloc(&Ip.d_wcnt, (size_t)(cfg->nspec * wstride))) || (rc = dalloc(&Ip.d_wofs, (size_t)wstride)))
+        (rc = dalloc(&Ip.d_wcnt, (size_t)(cfg->nspec * wstride))) ||
+        (rc = dalloc(&Ip.d_wcoarse, (size_t)(2 * cfg->nspec * Ip.cstride))))
         return fail_free(rc);
     // per bunch: ion kick coefficient 2 N_e r_e (m_e / m_u) / A c
     // (src/MPBunch.cpp:1117) and drift time C / h * gap / c

@@ -148,6 +148,7 @@ struct IonTurnParams {
     uint8_t *alive[CTS_MAX_SPECIES];
     const int64_t *len;      // [nspec] ions of the current buffer (compacted, all alive)
     const double *bview;     // [nb][4] bunch xbar, ybar, rmsRx, rmsRy
+    const double *bplan;     // [nb][kBePlan] the bunches' field constants
     const double *size_max;  // [2] largest rmsRx, rmsRy over the bunches
     const double *coeffI;    // [nb][CTS_MAX_SPECIES] 2 N_e r_e (m_e/m_u) / A c
     const double *dt;        // [nb] C / h * gap / c
@@ -159,6 +160,8 @@ struct IonTurnParams {
     int64_t acc_stride;
     uint32_t *wcnt;          // [nspec][wcnt_stride]: survivors of each wave
     int64_t wcnt_stride;
+    uint32_t *wcoarse;       // [nspec][wcoarse_stride]: survivors of kIonCoarse cohorts each, zero at the start
+    int64_t wcoarse_stride;
     const float *sur_params; // field surrogate (null: exact field)
     SurNorm sur_norm;
     double loss_boundary, ap_x, ap_y;
@@ -188,19 +191,33 @@ struct IonFinishParams {
 };
 constexpr int kIonAcc = 6;  // n, sum dx, sum dy, sum dx^2, sum dy^2, n kept
 
-// Stable compaction of one species after a segment, wave by wave in the
-// segment's wave order (old ions, then each passage's new ones: slot order).
+// Stable compaction after a segment, wave by wave in the segment's wave order
+// (old ions, then each passage's new ones: slot order).
 struct IonCompactParams {
-    const double *x, *y, *vx, *vy;
-    const uint8_t *alive;
-    double *ox, *oy, *ovx, *ovy;
-    uint8_t *oalive;
-    const int64_t *len;      // compacted ions of the source buffer before the segment
-    int64_t *new_len;        // ions of the destination buffer
-    const uint32_t *wcnt;    // survivors of every wave of the segment
-    uint32_t *wofs;          // their exclusive prefix sums
+    const double *x[CTS_MAX_SPECIES], *y[CTS_MAX_SPECIES], *vx[CTS_MAX_SPECIES], *vy[CTS_MAX_SPECIES];
+    const uint8_t *alive[CTS_MAX_SPECIES];
+    double *ox[CTS_MAX_SPECIES], *oy[CTS_MAX_SPECIES], *ovx[CTS_MAX_SPECIES], *ovy[CTS_MAX_SPECIES];
+    uint8_t *oalive[CTS_MAX_SPECIES];
+    const int64_t *len;      // [nspec] compacted ions of the source buffer before the segment
+    int64_t *new_len;        // [nspec] ions of the destination buffer
+    const uint32_t *wcnt;    // [nspec][wcnt_stride] survivors of every wave of the segment
+    const uint32_t *wcoarse; // [nspec][wcoarse_stride] survivors of kIonCoarse cohorts each
+    uint32_t *wcoarse_next;  // the next segment's, cleared
+    int64_t wcnt_stride, wcoarse_stride;
     int64_t cap;
     int32_t n_new, w_new, nseg;
+};
+
+// Bunch views, field constants and largest sizes from the last moments.
+struct IonPrepParams {
+    const cts_moments *cur;
+    double beta_x, beta_y;
+    double *bview, *bplan, *size_max;
+    uint32_t *fb_count;      // cleared (null: none)
+    const int64_t *len;
+    int64_t *len0;           // ions at the start of the turn
+    uint32_t *wcoarse;       // both buffers of coarse counts, cleared
+    int32_t ncoarse, nb, nspec;
 };
 
 struct BinParams {
@@ -372,16 +389,14 @@ hipError_t launch_finalize(const FinParams &p, hipStream_t st);
 hipError_t launch_post(const FinParams &f, const WakeParams &w, hipStream_t st);
 hipError_t launch_wake_table(const WakeTableParams &p, int ntables, hipStream_t st);
 hipError_t launch_wake(const WakeParams &p, int nb, hipStream_t st);
-hipError_t launch_ion_prep(const cts_moments *cur, int nb, double beta_x, double beta_y, double *bview,
-                           double *size_max, uint32_t *fb_count, const int64_t *len, int64_t *len0, int nspec,
-                           hipStream_t st);
+hipError_t launch_ion_prep(const IonPrepParams &p, hipStream_t st);
 // out[i] = sum over the kIonReplicas copies (stride n) of acc[i]; the
 // copies are left at zero
 hipError_t launch_ion_reduce(unsigned long long *acc, int64_t n, unsigned long long *out, hipStream_t st);
 hipError_t launch_ion_turn(const IonTurnParams &p, int nspec, int64_t wave_bound, hipStream_t st);
 hipError_t launch_ion_finish(const IonFinishParams &p, hipStream_t st);
 // wave_bound: a host bound of the segment's waves
-hipError_t launch_ion_compact(const IonCompactParams &p, int64_t wave_bound, hipStream_t st);
+hipError_t launch_ion_compact(const IonCompactParams &p, int nspec, int64_t wave_bound, hipStream_t st);
 constexpr int kBlMaxLds = 4096;  // beam-loaded cavities x (bins + 1): the per-bin kicks in LDS (32 KB)
 constexpr int kIonTurnMaxBlocks = 4096;  // grid bound of an ion segment or compaction (blocks stride over the waves)
 #ifndef CTS_ION_REPLICAS
@@ -396,10 +411,17 @@ constexpr int kIonSegment = CTS_ION_SEGMENT;  // bunch passages per ion segment
 #define CTS_ION_COHORT 4
 #endif
 #ifndef CTS_ION_WAVES_PER_EU
-#define CTS_ION_WAVES_PER_EU 4
+#define CTS_ION_WAVES_PER_EU 5
+#endif
+#ifndef CTS_ION_PACK
+#define CTS_ION_PACK 4
 #endif
 constexpr int kIonCohort = CTS_ION_COHORT;      // waves of an ion-turn block, walking the passages together
 constexpr int kIonBlock = 64 * kIonCohort;
+constexpr int kIonPack = CTS_ION_PACK;          // passages between two packings of a cohort (a power of two)
+constexpr int kIonCoarse = 64;                  // cohorts of a coarse survivor count
+constexpr int kIonPrepBlock = 512;
+constexpr int kCompactBlock = 1024;
 constexpr int kIonWavesPerEU = CTS_ION_WAVES_PER_EU;  // occupancy the ion-turn kernel is compiled for
 hipError_t launch_qe_debug(const float2 *tab, uint64_t seed, uint32_t turn, uint64_t base, int64_t n, double *out,
                            hipStream_t st);

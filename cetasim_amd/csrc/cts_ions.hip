@@ -20,6 +20,8 @@
 // associative, so the result does not depend on the order in which waves
 // finish.  A second small kernel turns them into each passage's moments and
 // electron-side kick parameters, in passage order.
+#include <type_traits>
+
 #include "cts_internal.hpp"
 
 namespace cts {
@@ -94,35 +96,45 @@ __device__ __forceinline__ bool ion_wave_slot(int w, int w_old, int64_t len, int
 // waves of the segment at a time (striding over the grid).  Wave w <
 // w_old holds the compacted ions of slots [64 w, 64 w + 64), from the
 // segment's first passage; the other waves hold the new ions of passage j0
-// (slot len + (j0 - j_begin) n_new + t), which join at their passage.  The
-// cohort walks the passages in step; after each passage, when the ions
-// still alive in the waves already walking fit into fewer waves, they are
-// packed (in wave and lane order) into the first of them through LDS, so
-// the lanes that evaluate the field stay mostly occupied as ions are lost.
-// Every ion sees the same operations in the same order as passage by
-// passage.  The cloud moments of each passage are summed per wave with DPP
-// moves and ballots into LDS, added over the cohort's waves in wave order
-// and turned into fixed-point limbs once per cohort (integer atomics, so
-// the sums do not depend on the order in which blocks finish); each block
-// adds its sums to one copy of the global sums at the end.  SUR: the
-// bunch's field at the ion from the surrogate inside its domain, the exact
+// (slot len + (j0 - j_begin) n_new + t), which join at their passage.  Every
+// kIonPack passages the cohort's waves meet: when the ions still alive in the
+// waves already walking fit into fewer of them, they are packed (in wave and
+// lane order) into the first ones through LDS, so the lanes that evaluate the
+// field stay mostly occupied as ions are lost; in between every wave walks on
+// its own.  Every ion sees the same operations in the same order as passage by
+// passage.  The bunch's data and field constants are read as scalars.  The
+// cloud moments of each passage are summed per wave (four sums at once,
+// wave_pack4; the counts by ballots) into LDS, added over the cohort's waves
+// in wave order and turned into fixed-point limbs once per cohort (integer
+// atomics, so the sums do not depend on the order in which blocks finish);
+// each block adds its sums to one copy of the global sums at the end.  SUR:
+// the bunch's field at the ion from the surrogate inside its domain, the exact
 // field elsewhere.
+//
+// Bound by FP64 vector work and what is left of its latency: about 390 vector
+// instructions per wave and passage (two w(z) of 40 coefficients at two fma
+// each are 148 of them), 17 ps per ion and passage on 5e5 ions that outlive
+// the train (22 ps with a barrier pair every passage, the sums by DPP moves and
+// the constants in LDS).  Packing every 1, 2, 4, 8 passages: 2.24, 2.11, 2.00,
+// 1.97 ms per turn there, and 1.49, 1.40, 1.38, 1.41 on a train whose ions live
+// 12 passages; cohorts of 2 and 8 waves 2.14 and 2.31, five or six waves per
+// SIMD alike.
 template <bool SUR>
-__global__ void __launch_bounds__(kIonBlock, kIonWavesPerEU)
+__global__ void __launch_bounds__(kIonBlock, SUR ? 3 : kIonWavesPerEU)
 k_ion_turn(IonTurnParams P)
 {
-    __shared__ __attribute__((aligned(16))) MlpLds L;
-    __shared__ double sbv[kIonSegment][4], scI[kIonSegment], sdt[kIonSegment];
-    __shared__ BeField sF[kIonSegment];
+    struct NoNet {};
+    __shared__ __attribute__((aligned(16))) std::conditional_t<SUR, MlpLds, NoNet> L;
     __shared__ unsigned long long sacc[kIonSegment * kIonAcc * 3];
-    __shared__ double wpart[kIonCohort][kIonSegment][kIonAcc];  // per wave, per passage
-    __shared__ double rp[4][kIonBlock];                          // packing: x, y, vx, vy
-    __shared__ int32_t rs[kIonBlock], ro[kIonBlock];             // packing: slot, first wave
-    __shared__ int32_t wn[kIonCohort];                           // alive ions of each wave (-1: not walking)
-    __shared__ uint32_t wkept[kIonCohort];                       // survivors of each first wave
+    __shared__ double wpart[kIonCohort][kIonSegment][4];  // per wave, per passage: the sums
+    __shared__ uint32_t wcount[kIonCohort][kIonSegment];  // alive before | kept << 16
+    __shared__ double rp[4][kIonBlock];                   // packing: x, y, vx, vy
+    __shared__ int32_t rs[kIonBlock], ro[kIonBlock];      // packing: slot, first wave
+    __shared__ int32_t wn[kIonCohort];                    // alive ions of each wave (-1: not walking)
+    __shared__ uint32_t wkept[kIonCohort];                // survivors of each first wave
     __shared__ int32_t s_qmin;
     const int p = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t len = P.len[p];
     // waves: the ions alive at the start of the segment (compacted), then
     // the new ions of every passage of the segment
@@ -131,13 +143,7 @@ k_ion_turn(IonTurnParams P)
     const int total = w_old + nseg * P.w_new;
     const int ncoh = (total + kIonCohort - 1) / kIonCohort;
     if ((int)blockIdx.x >= ncoh) return;  // whole block idle (uniform)
-    if (SUR) load_mlp_lds(L, P.sur_params, tid, kIonBlock);
-    for (int i = tid; i < nseg * 4; i += kIonBlock) sbv[i >> 2][i & 3] = P.bview[4 * P.j_begin + i];
-    for (int i = tid; i < nseg; i += kIonBlock) {
-        scI[i] = P.coeffI[(P.j_begin + i) * CTS_MAX_SPECIES + p];
-        sdt[i] = P.dt[P.j_begin + i];
-        sF[i] = be_plan(P.bview[4 * (P.j_begin + i) + 2], P.bview[4 * (P.j_begin + i) + 3]);
-    }
+    if constexpr (SUR) load_mlp_lds(L, P.sur_params, tid, kIonBlock);
     for (int i = tid; i < nseg * kIonAcc * 3; i += kIonBlock) sacc[i] = 0ull;
     const uint32_t turn = P.turn_dev ? *P.turn_dev + P.turn : P.turn;
     double *X = P.x[p], *Y = P.y[p], *VX = P.vx[p], *VY = P.vy[p];
@@ -147,6 +153,11 @@ k_ion_turn(IonTurnParams P)
     const double bx = P.ap_x > lbx ? lbx : P.ap_x;
     const double by = P.ap_y > lby ? lby : P.ap_y;
     const uint64_t below = (1ull << lane) - 1ull;
+    // the scalars of passage j: bunch view, field constants, kick, drift
+    const cdptr bview = reload((uint64_t)(uintptr_t)(P.bview + 4 * P.j_begin));
+    const cdptr bplan = reload((uint64_t)(uintptr_t)(P.bplan + (int64_t)kBePlan * P.j_begin));
+    const cdptr coeff = reload((uint64_t)(uintptr_t)(P.coeffI + (int64_t)CTS_MAX_SPECIES * P.j_begin + p));
+    const cdptr drift = reload((uint64_t)(uintptr_t)(P.dt + P.j_begin));
     for (int c = blockIdx.x; c < ncoh; c += gridDim.x) {
         const int w = c * kIonCohort + wv;
         // slot: this lane's ion in the buffer (-1: none); q0: the wave's
@@ -164,8 +175,8 @@ k_ion_turn(IonTurnParams P)
             if (w < w_old) {
                 x = X[slot]; y = Y[slot]; vx = VX[slot]; vy = VY[slot];
             } else {
-                ion_generate(P.seed, turn, (uint32_t)(P.j_begin + q0), p, (uint32_t)t, sbv[q0][0], sbv[q0][1],
-                             sbv[q0][2], sbv[q0][3], x, y);
+                ion_generate(P.seed, turn, (uint32_t)(P.j_begin + q0), p, (uint32_t)t, bview[4 * q0], bview[4 * q0 + 1],
+                             bview[4 * q0 + 2], bview[4 * q0 + 3], x, y);
             }
             A[slot] = 0;  // survivors set it again at the end
         }
@@ -173,55 +184,56 @@ k_ion_turn(IonTurnParams P)
         int32_t first = wv;  // the wave the ion started in
         bool alive = false;  // walking and not lost
         if (tid == 0) s_qmin = nseg;
-        for (int i = tid; i < kIonCohort * kIonSegment * kIonAcc; i += kIonBlock) (&wpart[0][0][0])[i] = 0.0;
+        for (int i = tid; i < kIonCohort * kIonSegment * 4; i += kIonBlock) (&wpart[0][0][0])[i] = 0.0;
+        for (int i = tid; i < kIonCohort * kIonSegment; i += kIonBlock) (&wcount[0][0])[i] = 0u;
         if (tid < kIonCohort) wkept[tid] = 0u;
         __syncthreads();
         const bool any_mine = __any(mine);
         if (lane == 0 && any_mine) atomicMin(&s_qmin, q0);
         __syncthreads();
-        for (int q = s_qmin; q < nseg; q++) {
+        const int qfirst = __builtin_amdgcn_readfirstlane(s_qmin);
+        for (int q = qfirst; q < nseg; q++) {
             // a wave's new ions join at their passage (wave-uniform)
             if (q == q0) alive = myslot >= 0;
-            const bool walking = q0 <= q;
-            if (__any(alive)) {
-                const double xm = sbv[q][0], ym = sbv[q][1];
-                const double dx = x - xm, dy = y - ym;
+            const uint64_t am0 = __ballot(alive);
+            if (am0) {
+                const double dx = x - bview[4 * q], dy = y - bview[4 * q + 1];
                 double fx = 0.0, fy = 0.0;
-                if (SUR) {
-                    const bool ok = sur_field(L, P.sur_norm, alive, dx, dy, sbv[q][2], sbv[q][3], fx, fy);
-                    if (alive && !ok) be_field(dx, dy, sF[q], fx, fy);
+                const BeField F = be_plan_load(bplan + q * kBePlan);
+                if constexpr (SUR) {
+                    const bool ok = sur_field(L, P.sur_norm, alive, dx, dy, bview[4 * q + 2], bview[4 * q + 3], fx, fy);
+                    if (alive && !ok) be_field(dx, dy, F, fx, fy);
                 } else if (alive) {
-                    be_field(dx, dy, sF[q], fx, fy);
+                    be_field(dx, dy, F, fx, fy);
                 }
                 bool keep = false;
                 if (alive) {
-                    const double cI = scI[q];
+                    const double cI = coeff[q * CTS_MAX_SPECIES], dt = drift[q];
                     vx += cI * fx;
                     vy += cI * fy;
-                    x += vx * sdt[q];
-                    y += vy * sdt[q];
+                    x += vx * dt;
+                    y += vy * dt;
                     keep = !(fabs(x) > bx || fabs(y) > by);
                 }
                 // the cloud as the bunch finds it (before the kick), and the
-                // ions kept: counts by ballot, sums by DPP reductions
-                const double c0 = (double)__popcll(__ballot(alive));
-                double cs[4] = {alive ? dx : 0.0, alive ? dy : 0.0, alive ? dx * dx : 0.0, alive ? dy * dy : 0.0};
-                wave_sum4_dpp(cs);
-                const double c1 = cs[0], c2 = cs[1], c3 = cs[2], c4 = cs[3];
-                const double c5 = (double)__popcll(__ballot(keep));
-                if (lane == 0) {
-                    double *o = wpart[wv][q];
-                    o[0] = c0; o[1] = c1; o[2] = c2; o[3] = c3; o[4] = c4; o[5] = c5;
-                }
+                // ions kept
+                const double s = wave_pack4<false>(alive ? dx : 0.0, alive ? dy : 0.0, alive ? dx * dx : 0.0,
+                                                   alive ? dy * dy : 0.0);
+                if ((lane & 15) == 0) wpart[wv][q][pack4_value(lane >> 4)] = s;
+                const uint64_t km = __ballot(keep);
+                if (lane == 0) wcount[wv][q] = (uint32_t)__popcll(am0) | ((uint32_t)__popcll(km) << 16);
                 alive = keep;
             }
+            if (((q - qfirst) & (kIonPack - 1)) != kIonPack - 1) continue;
             // pack the walking waves' ions into as few of them as hold them
+            const bool walking = q0 <= q;
             const uint64_t am = __ballot(alive);
             if (lane == 0) wn[wv] = walking ? __popcll(am) : -1;
             __syncthreads();
             int nalive = 0, busy = 0, base = 0, rank = 0;
+#pragma unroll
             for (int k = 0; k < kIonCohort; k++) {
-                const int n = wn[k];
+                const int n = __builtin_amdgcn_readfirstlane(wn[k]);
                 if (n < 0) continue;
                 if (k < wv) { base += n; rank++; }
                 nalive += n;
@@ -256,14 +268,26 @@ k_ion_turn(IonTurnParams P)
         }
         __syncthreads();
         if (tid < kIonCohort && c * kIonCohort + tid < total) P.wcnt[p * P.wcnt_stride + c * kIonCohort + tid] = wkept[tid];
-        // the cohort's passage sums: over its waves in wave order, then to
-        // fixed point (limb k of value v of passage q per thread)
-        for (int i = tid; i < nseg * kIonAcc * 3; i += kIonBlock) {
-            const int q = i / (kIonAcc * 3), v = (i / 3) % kIonAcc, kk = i % 3;
+        if (tid == 0) {
+            uint32_t n = 0;
+            for (int k = 0; k < kIonCohort; k++) n += wkept[k];
+            if (n) atomicAdd(&P.wcoarse[p * P.wcoarse_stride + c / kIonCoarse], n);
+        }
+        // the cohort's passage sums over its waves in wave order, then to
+        // fixed point (limb k of value v of passage q per thread); a count n
+        // is n 2^16 in the highest limb
+        for (int i = tid; i < nseg * 4 * 3; i += kIonBlock) {
+            const int q = i / 12, v = (i / 3) % 4, kk = i % 3;
             double sv = 0.0;
             for (int k = 0; k < kIonCohort; k++) sv += wpart[k][q][v];
             const long long l = fx_limb(sv, kk);
-            if (l != 0) atomicAdd(&sacc[(q * kIonAcc + v) * 3 + kk], (unsigned long long)l);
+            if (l != 0) atomicAdd(&sacc[(q * kIonAcc + 1 + v) * 3 + kk], (unsigned long long)l);
+        }
+        for (int i = tid; i < nseg * 2; i += kIonBlock) {
+            const int q = i >> 1, v = i & 1;
+            uint32_t n = 0;
+            for (int k = 0; k < kIonCohort; k++) n += v ? wcount[k][q] >> 16 : wcount[k][q] & 0xffffu;
+            if (n) atomicAdd(&sacc[(q * kIonAcc + 5 * v) * 3 + 2], (unsigned long long)n << 16);
         }
         __syncthreads();
     }
@@ -349,33 +373,36 @@ k_ion_finish(IonFinishParams P)
 // from the last moment record (rmsRx = sqrt(emitX * betaX[k]),
 // src/MPBunch.cpp:481-482), and their maxima (MPGetBeamInfo,
 // src/MPBeam.cpp:2203-2258).
-__global__ void __launch_bounds__(256)
-k_ion_prep(const cts_moments *cur, int nb, double beta_x, double beta_y, double *bview, double *size_max,
-           uint32_t *fb_count, const int64_t *len, int64_t *len0, int nspec)
+__global__ void __launch_bounds__(kIonPrepBlock)
+k_ion_prep(IonPrepParams P)
 {
-    if (threadIdx.x == 0 && fb_count) *fb_count = 0u;
-    if ((int)threadIdx.x < nspec) len0[threadIdx.x] = len[threadIdx.x];
-    __shared__ double mx[256], my[256];
+    __shared__ double red[2][kIonPrepBlock / 64];
+    const int tid = threadIdx.x;
+    if (tid == 0 && P.fb_count) *P.fb_count = 0u;
+    if (tid < P.nspec) P.len0[tid] = P.len[tid];
+    for (int i = tid; i < P.ncoarse; i += kIonPrepBlock) P.wcoarse[i] = 0u;
     double ax = -INFINITY, ay = -INFINITY;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-        const double *c = cur[b].c2;
-        const double rx = sqrt(sqrt(c[0] * c[2] - c[1] * c[1]) * beta_x);
-        const double ry = sqrt(sqrt(c[3] * c[5] - c[4] * c[4]) * beta_y);
-        bview[4 * b + 0] = cur[b].mean[0];
-        bview[4 * b + 1] = cur[b].mean[2];
-        bview[4 * b + 2] = rx;
-        bview[4 * b + 3] = ry;
+    for (int b = tid; b < P.nb; b += kIonPrepBlock) {
+        const double *c = P.cur[b].c2;
+        const double rx = sqrt(sqrt(c[0] * c[2] - c[1] * c[1]) * P.beta_x);
+        const double ry = sqrt(sqrt(c[3] * c[5] - c[4] * c[4]) * P.beta_y);
+        double *v = P.bview + 4 * b;
+        v[0] = P.cur[b].mean[0];
+        v[1] = P.cur[b].mean[2];
+        v[2] = rx;
+        v[3] = ry;
+        be_plan_store(be_plan(rx, ry), P.bplan + (int64_t)b * kBePlan);
         ax = fmax(ax, rx);
         ay = fmax(ay, ry);
     }
-    mx[threadIdx.x] = ax;
-    my[threadIdx.x] = ay;
+    ax = wave_max(ax);
+    ay = wave_max(ay);
+    if ((tid & 63) == 0) { red[0][tid >> 6] = ax; red[1][tid >> 6] = ay; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = mx[0], c = my[0];
-        for (int t = 1; t < (int)blockDim.x; t++) { a = fmax(a, mx[t]); c = fmax(c, my[t]); }
-        size_max[0] = a;
-        size_max[1] = c;
+    if (tid < 2) {
+        double a = red[tid][0];
+        for (int w = 1; w < kIonPrepBlock / 64; w++) a = fmax(a, red[tid][w]);
+        P.size_max[tid] = a;
     }
 }
 
@@ -392,58 +419,57 @@ k_ion_reduce(unsigned long long *acc, int64_t n, unsigned long long *out)
     out[i] = s;
 }
 
-// Stable compaction of one species' cloud into the other buffer after a
-// segment.  Pass 1 (one block): exclusive prefix sums of the survivors of
-// the segment's waves.  Pass 2: every wave moves its survivors to their
-// places, in the waves' order (old ions, then each passage's new ones), so
-// the slot order is kept.
-__global__ void __launch_bounds__(1024)
-k_compact_scan(IonCompactParams P)
+// Stable compaction of the clouds into the other buffer after a segment, one
+// launch for all species (grid.y).  A wave's survivors go behind those of the
+// waves before it (old ions, then each passage's new ones, so the slot order
+// is kept): a block of 16 waves adds the coarse counts (kIonCoarse cohorts
+// each, left by k_ion_turn) up to its group and the waves' counts within it.
+// As a scan of one block and a second launch, for each species, the two took
+// 9 us after every segment, however small.
+__global__ void __launch_bounds__(kCompactBlock)
+k_ion_compact(IonCompactParams P)
 {
-    __shared__ uint32_t s[1024];
-    const int64_t len = *P.len;
+    constexpr int W = kCompactBlock / 64, G = kIonCoarse * kIonCohort;  // waves of a block, of a coarse count
+    __shared__ uint32_t red[W], cnt[W];
+    const int p = blockIdx.y;
+    const int64_t len = P.len[p];
     const int w_old = (int)((len + 63) / 64);
     const int total = w_old + P.nseg * P.w_new;
-    const int per = (total + 1023) / 1024;
-    const int a = min((int)threadIdx.x * per, total), b = min(a + per, total);
-    uint32_t c = 0;
-    for (int w = a; w < b; w++) c += P.wcnt[w];
-    s[threadIdx.x] = c;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const uint32_t v = (int)threadIdx.x >= o ? s[threadIdx.x - o] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint32_t run = s[threadIdx.x] - c;
-    for (int w = a; w < b; w++) {
-        const uint32_t n = P.wcnt[w];
-        P.wofs[w] = run;
-        run += n;
-    }
-    if (threadIdx.x == 1023) *P.new_len = (int64_t)s[1023];
-}
-
-__global__ void __launch_bounds__(256)
-k_compact_scatter(IonCompactParams P)
-{
-    const int64_t len = *P.len;
-    const int w_old = (int)((len + 63) / 64);
-    const int total = w_old + P.nseg * P.w_new;
-    const int lane = threadIdx.x & 63;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
-    for (int w = blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += gridDim.x * 4) {
-        int q0, t;
-        int64_t i;
-        const bool mine = ion_wave_slot(w, w_old, len, P.n_new, P.w_new, P.cap, lane, i, q0, t);
-        const bool on = mine && P.alive[i];
-        const uint64_t m = __ballot(on);
-        if (on) {
-            const uint64_t d = P.wofs[w] + (uint64_t)__popcll(m & below);
-            P.ox[d] = P.x[i]; P.oy[d] = P.y[i]; P.ovx[d] = P.vx[i]; P.ovy[d] = P.vy[i];
-            P.oalive[d] = 1;
+    const uint32_t *wcnt = P.wcnt + p * P.wcnt_stride, *coarse = P.wcoarse + p * P.wcoarse_stride;
+    // the other buffer of coarse counts, for the next segment
+    if (blockIdx.x == 0)
+        for (int i = tid; i < P.wcoarse_stride; i += kCompactBlock) P.wcoarse_next[p * P.wcoarse_stride + i] = 0u;
+    if (total == 0 && blockIdx.x == 0 && tid == 0) P.new_len[p] = 0;
+    for (int w0 = blockIdx.x * W; w0 < total; w0 += gridDim.x * W) {
+        const int g = w0 / G;
+        uint32_t c = 0;
+        for (int i = tid; i < g; i += kCompactBlock) c += coarse[i];
+        for (int i = g * G + tid; i < w0; i += kCompactBlock) c += wcnt[i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        const int w = w0 + wv;
+        const uint32_t mine_cnt = w < total ? wcnt[w] : 0u;
+        if (lane == 0) { red[wv] = c; cnt[wv] = mine_cnt; }
+        __syncthreads();
+        uint32_t base = 0;
+        for (int k = 0; k < W; k++) base += red[k] + (k < wv ? cnt[k] : 0u);
+        if (w == total - 1 && lane == 0) P.new_len[p] = (int64_t)(base + mine_cnt);
+        if (w < total && mine_cnt) {
+            int q0, t;
+            int64_t i;
+            const bool mine = ion_wave_slot(w, w_old, len, P.n_new, P.w_new, P.cap, lane, i, q0, t);
+            const bool on = mine && P.alive[p][i];
+            const uint64_t m = __ballot(on);
+            if (on) {
+                const uint64_t d = base + (uint64_t)__popcll(m & below);
+                P.ox[p][d] = P.x[p][i]; P.oy[p][d] = P.y[p][i];
+                P.ovx[p][d] = P.vx[p][i]; P.ovy[p][d] = P.vy[p][i];
+                P.oalive[p][d] = 1;
+            }
         }
+        __syncthreads();
     }
 }
 
@@ -474,11 +500,9 @@ hipError_t launch_ion_finish(const IonFinishParams &p, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_ion_prep(const cts_moments *cur, int nb, double bx, double by, double *bview, double *size_max,
-                           uint32_t *fb_count, const int64_t *len, int64_t *len0, int nspec, hipStream_t st)
+hipError_t launch_ion_prep(const IonPrepParams &p, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_ion_prep, dim3(1), dim3(256), 0, st, cur, nb, bx, by, bview, size_max, fb_count, len,
-                       len0, nspec);
+    hipLaunchKernelGGL(k_ion_prep, dim3(1), dim3(kIonPrepBlock), 0, st, p);
     return hipGetLastError();
 }
 
@@ -488,13 +512,13 @@ hipError_t launch_ion_reduce(unsigned long long *acc, int64_t n, unsigned long l
     return hipGetLastError();
 }
 
-hipError_t launch_ion_compact(const IonCompactParams &p, int64_t wave_bound, hipStream_t st)
+hipError_t launch_ion_compact(const IonCompactParams &p, int nspec, int64_t wave_bound, hipStream_t st)
 {
-    int64_t blocks = (wave_bound + 3) / 4;
+    constexpr int W = kCompactBlock / 64;
+    int64_t blocks = (wave_bound + W - 1) / W;
     if (blocks > kIonTurnMaxBlocks) blocks = kIonTurnMaxBlocks;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_compact_scan, dim3(1), dim3(1024), 0, st, p);
-    hipLaunchKernelGGL(k_compact_scatter, dim3((unsigned)blocks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(k_ion_compact, dim3((unsigned)blocks, (unsigned)nspec), dim3(kCompactBlock), 0, st, p);
     return hipGetLastError();
 }
 

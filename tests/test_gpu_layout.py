@@ -70,3 +70,27 @@ def test_ion_kick_items(nspec):
     compare_coords(got, bunches, off, 1e-12)
     assert np.max(np.abs(got["px"] - before)) > 1e-8 * np.max(np.abs(before))
     tr.close()
+
+
+@pytest.mark.parametrize("nspec,n_new,nb", [(2, 3000, 40), (1, 17_000, 3)])
+def test_cloud_of_many_waves(nspec, n_new, nb):
+    """Clouds over several coarse survivor counts (256 waves each) and, with
+    40 bunches, a compaction between two segments: the cloud in slot order."""
+    ions = dict(ION_TEST, mass_number=[28.0, 18.0][:nspec], cross_section=[2.0e-22, 1.6e-22][:nspec],
+                pressure=[1.0e-5, 0.4e-5][:nspec], n_new=n_new, max_ions=400_000)
+    counts = [400 + 3 * (b % 5) for b in range(nb)]
+    ring, secs, counts, gap, q, ne, cfg, tr, bunches, off = setup_train(counts, 14, ions=ions, ne_scale=0.1,
+                                                                       gap=[2] * nb)
+    ot = O.OracleTrain(ring, secs[0], counts, ne, gap, cfg, ions["seed"])
+    print(f"cloud of {nspec} x {n_new * nb} ions", flush=True)
+    tr.ion_phase(0)
+    exp = ot.ion_phase(bunches, 0)
+    got = tr.ion_passages()
+    np.testing.assert_allclose(got[:, :nspec, 5], exp[:, :nspec, 0], rtol=1e-12)
+    np.testing.assert_allclose(got[:, :nspec, 1:5], exp[:, :nspec, 1:5], rtol=1e-9, atol=1e-18)
+    for sp in range(nspec):
+        cloud, ec = tr.ion_cloud(sp), ot.cloud.species(sp)
+        assert len(cloud["x"]) == len(ec["x"]) > 30_000
+        for c in ("x", "y", "vx", "vy"):
+            np.testing.assert_allclose(cloud[c], ec[c], rtol=1e-9, atol=1e-9 * np.max(np.abs(ec[c])))
+    tr.close()
