@@ -142,7 +142,7 @@ struct cts_handle {
     int hist_parity = 0;
     int32_t *d_counts = nullptr;
     double *d_kick = nullptr, *d_poten = nullptr, *d_edges_prev = nullptr, *d_edges_now = nullptr;
-    double *d_table = nullptr, *d_scale = nullptr;
+    double *d_table = nullptr, *d_scale = nullptr, *d_terms = nullptr;
     bool kick_pending = false;
 
     // synrad
@@ -159,6 +159,9 @@ struct cts_handle {
     // items of the electron-side kick (kBlock particles of one bunch each)
     int32_t *d_item_bunch = nullptr, *d_item_first = nullptr;
     int nitem = 0;
+    // blocks of the binning over the reference's edges
+    int32_t *d_bin_bunch = nullptr, *d_bin_first = nullptr;
+    int nbin_item = 0;
     double *d_ion_bview = nullptr;
     double *d_ion_bplan = nullptr;  // the bunches' field constants ([nb][kBePlan])
     std::vector<IonIp> ips;
@@ -214,7 +217,8 @@ struct cts_handle {
     struct KeepBl { bool on = false; cts_beam_loading_config cfg{}; } keep_bl;
 
     // graph replays of two consecutive turns (cts_run_turns): the turn is
-    // read from d_turn, which the graph advances by 2; one instance per
+    // read from d_turn[0], which the graph advances by 2 at its end, and left
+    // by the pass in d_turn[1] for the kernels behind it; one instance per
     // (wake buffer parity, ion buffer) at capture
     uint32_t *d_turn = nullptr;
     bool capturing = false;
@@ -304,8 +308,9 @@ void free_bunch_state(cts_handle *h)
                     h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part, h->d_shift,
                     h->d_cur, h->d_hist, h->d_sigz, h->d_zrange, h->d_noise, h->d_ion_e, h->d_ion_bview,
                     h->d_ion_f, h->d_ion_bplan, h->d_item_bunch, h->d_item_first,
+                    h->d_bin_bunch, h->d_bin_first,
                     h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev,
-                    h->d_edges_now, h->d_table, h->d_scale,
+                    h->d_edges_now, h->d_table, h->d_scale, h->d_terms,
                     h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order, h->d_seg_step};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -318,11 +323,11 @@ void free_bunch_state(cts_handle *h)
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = nullptr;
     h->d_seg_part = h->d_shift = h->d_sigz = h->d_zrange = h->d_noise = h->d_ion_e = h->d_ion_bview = nullptr;
     h->d_ion_f = h->d_ion_bplan = nullptr;
-    h->d_item_bunch = h->d_item_first = nullptr;
+    h->d_item_bunch = h->d_item_first = h->d_bin_bunch = h->d_bin_first = nullptr;
     h->d_cur = h->d_hist = nullptr;
     h->d_bhist = nullptr;
     h->d_counts = nullptr;
-    h->d_kick = h->d_poten = h->d_edges_prev = h->d_edges_now = h->d_table = h->d_scale = nullptr;
+    h->d_kick = h->d_poten = h->d_edges_prev = h->d_edges_now = h->d_table = h->d_scale = h->d_terms = nullptr;
     h->d_fb_count = nullptr;
     h->d_fb_list = nullptr;
 }
@@ -524,6 +529,7 @@ PassParams base_pass(cts_handle *h, uint32_t ops, int k)
     }
     if (h->capturing) {
         p.turn_dev = h->d_turn;
+        p.turn_copy = h->d_turn + 1;
         p.turn = (uint32_t)h->cap_off;
     }
     return p;
@@ -552,8 +558,7 @@ FinParams base_fin(cts_handle *h, uint32_t ops, int slot, int prev_slot)
     f.nseg = h->nseg;
     f.lr_cen = h->d_lrw_cen;
     if (h->capturing) {
-        f.turn_dev = h->d_turn;
-        f.turn_off = h->cap_off;
+        f.turn_dev = h->d_turn + 1;
         f.hist_cap = h->hist_cap;
     }
     return f;
@@ -579,8 +584,6 @@ int run_finalize(cts_handle *h, const FinParams &f)
 
 int slot_of(cts_handle *h, int turn) { return (h->hist_cap > 0 && turn >= 0) ? turn % h->hist_cap : -1; }
 
-// Wake stage after the histogram is complete: reference-edge mode needs
-// the per-bunch table for this turn's bin width first.
 WakeParams wake_params(cts_handle *h)
 {
     WakeParams w;
@@ -599,19 +602,20 @@ WakeParams wake_params(cts_handle *h)
     return w;
 }
 
+WakeTableParams table_params(cts_handle *h)
+{
+    WakeTableParams t;
+    std::memset(&t, 0, sizeof t);
+    t.terms = h->d_terms;
+    t.table = h->d_table;
+    t.nbins = h->nbins;
+    t.nres = h->nres;
+    for (int r = 0; r < h->nres; r++) { t.rs[r] = h->rs[r]; t.q[r] = h->q[r]; t.omega[r] = h->omega[r]; }
+    return t;
+}
+
 int run_wake(cts_handle *h)
 {
-    if (h->wake_mode == 0) {
-        WakeTableParams t;
-        std::memset(&t, 0, sizeof t);
-        t.edges = h->d_edges_now;
-        t.table = h->d_table;
-        t.nbins = h->nbins;
-        t.nres = h->nres;
-        for (int r = 0; r < h->nres; r++) { t.rs[r] = h->rs[r]; t.q[r] = h->q[r]; t.omega[r] = h->omega[r]; }
-        TimedScope ts(h, "wake_table");
-        HIPCHK(launch_wake_table(t, h->nb, h->stream));
-    }
     WakeParams w = wake_params(h);
     TimedScope ts(h, "wake");
     HIPCHK(launch_wake(w, h->nb, h->stream));
@@ -619,17 +623,28 @@ int run_wake(cts_handle *h)
     return CTS_OK;
 }
 
-int run_bin(cts_handle *h)
+// Reference-edge mode after the pass: the moments of `f` (null: the edges in
+// d_edges_now are final), the bins over this turn's edges and every bunch's
+// lag table for its bin width.
+int run_close(cts_handle *h, const FinParams *f)
 {
-    BinParams b;
+    CloseParams c;
+    std::memset(&c, 0, sizeof c);
+    if (f) c.f = *f;
+    c.fin = f != nullptr;
+    c.edges_given = f == nullptr;
+    c.edges_now = h->d_edges_now;
+    c.nb = h->nb;
+    c.tables = h->nb;
+    c.t = table_params(h);
+    BinParams &b = c.b;
     b.z = h->d_z;
-    b.seg_begin = h->d_seg_begin; b.seg_end = h->d_seg_end;
-    b.seg_bunch = h->d_seg_bunch; b.wg_seg = h->d_wg_seg; b.seg_step = h->d_seg_step;
-    b.edges = h->d_edges_now;
+    b.bunch_off = h->d_bunch_off;
+    b.item_bunch = h->d_bin_bunch; b.item_first = h->d_bin_first;
     b.bunch_hist = h->d_bhist + (size_t)h->hist_parity * h->nb * h->nbins;
     b.nbins = h->nbins;
-    TimedScope ts(h, "bin");
-    HIPCHK(launch_bin(b, h->nwg, h->stream));
+    TimedScope ts(h, "close");
+    HIPCHK(launch_close(c, h->nbin_item, h->stream));
     return CTS_OK;
 }
 
@@ -706,12 +721,12 @@ int reset_status(cts_handle *h)
     return CTS_OK;
 }
 
-// Workgroups of the streaming pass that the device holds at one time: three
-// of 256 threads per compute unit (the turn's variants use 130 to 152
-// registers).  The default layouts cut the particles for exactly that many,
-// so that no workgroup waits for a second round: with 1024 on 256 compute
-// units the 480-bunch train's pass took 1.50 ms, with 768 1.33 ms.
-constexpr int kPassPerCu = 3;
+// Binning blocks of a bunch: each adds its whole histogram to the bunch's at
+// the end, so more of them soon cost more in atomics than they bin (1.3e6
+// macroparticles, k_close by blocks: 32 27 us, 64 18, 128 14.9, 256 15.3,
+// 1024 29), and a small bunch takes one per 4096 (6e4 with 1024 bins: 15
+// blocks 32 us, 59 44, 118 66).
+constexpr int64_t kBinBlocks = 128, kBinMin = 4096;
 
 struct Seg {
     int64_t begin, end;
@@ -1138,14 +1153,14 @@ int cts_create(const cts_ring *ring, const cts_section *secs, int32_t nsec, cts_
     if (e == hipSuccess) e = upload_faddeeva_tables_ions(ft);
     if (e == hipSuccess) e = hipMalloc((void **)&h->d_status, sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemset(h->d_status, 0, sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&h->d_turn, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void **)&h->d_turn, 2 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc((void **)&h->d_ntab, 2 * kNormTab * sizeof(float2));
     if (e == hipSuccess) {
         std::vector<float2> tab(2 * kNormTab);
         build_normal_tables(tab.data());
         e = hipMemcpy(h->d_ntab, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = hipMemset(h->d_turn, 0, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(h->d_turn, 0, 2 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc((void **)&h->h_status, sizeof(uint32_t), hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&h->status_ev, hipEventDisableTiming);
     if (e == hipSuccess) {
@@ -1221,22 +1236,30 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
         (rc = dalloc(&h->d_ion_e, (size_t)nb * CTS_MAX_SPECIES * 5)) || (rc = dalloc(&h->d_ion_bview, (size_t)nb * 4)))
         return rc;
     if ((rc = layout_segments(h, h->wg_target, h->tile))) return rc;
-    {
+    // items of kernels that split the bunches themselves: the electron-side
+    // ion kick (a block of particles each) and the binning
+    const auto cut_items = [&](auto items_of, int32_t **d_bunch, int32_t **d_first, int *count) -> int {
         std::vector<int32_t> first(nb + 1, 0), bunch;
         for (int b = 0; b < nb; b++) {
-            const int64_t items = (counts[b] + kBlock - 1) / kBlock;
+            const int64_t items = items_of(counts[b]);
             if (first[b] + items > INT32_MAX / 2) return fail(CTS_ERR_ARG, "cts_set_bunches: too many particles");
             first[b + 1] = first[b] + (int32_t)items;
             bunch.insert(bunch.end(), (size_t)items, b);
         }
-        h->nitem = first[nb];
-        if ((rc = dalloc(&h->d_item_bunch, bunch.size())) || (rc = dalloc(&h->d_item_first, first.size())) ||
-            (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)) ||
-            (rc = dalloc(&h->d_ion_bplan, (size_t)nb * kBePlan)))
-            return rc;
-        HIPCHK(hipMemcpy(h->d_item_bunch, bunch.data(), bunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(h->d_item_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    }
+        *count = first[nb];
+        int r;
+        if ((r = dalloc(d_bunch, bunch.size())) || (r = dalloc(d_first, first.size()))) return r;
+        HIPCHK(hipMemcpy(*d_bunch, bunch.data(), bunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(*d_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        return CTS_OK;
+    };
+    const auto kick_items = [](int64_t n) { return (n + kBlock - 1) / kBlock; };
+    const auto bin_items = [](int64_t n) { return std::min<int64_t>(kBinBlocks, (n + kBinMin - 1) / kBinMin); };
+    if ((rc = cut_items(kick_items, &h->d_item_bunch, &h->d_item_first, &h->nitem)) ||
+        (rc = cut_items(bin_items, &h->d_bin_bunch, &h->d_bin_first, &h->nbin_item)) ||
+        (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)) ||
+        (rc = dalloc(&h->d_ion_bplan, (size_t)nb * kBePlan)))
+        return rc;
     HIPCHK(hipMemcpy(h->d_bunch_off, h->offsets.data(), (nb + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_count, h->counts.data(), nb * sizeof(int64_t), hipMemcpyHostToDevice));
     h->kick_pending = false;
@@ -1361,11 +1384,11 @@ int cts_set_wake(cts_handle *h, int32_t nbins, int32_t mode, double grid_lo, dou
     if ((rc = flush_kick(h))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     void *old[] = {h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev, h->d_edges_now,
-                   h->d_table, h->d_scale};
+                   h->d_table, h->d_scale, h->d_terms};
     for (void *p : old)
         if (p) (void)hipFree(p);
     h->d_bhist = nullptr; h->d_counts = nullptr;
-    h->d_kick = h->d_poten = h->d_edges_prev = h->d_edges_now = h->d_table = h->d_scale = nullptr;
+    h->d_kick = h->d_poten = h->d_edges_prev = h->d_edges_now = h->d_table = h->d_scale = h->d_terms = nullptr;
     h->nbins = (nres > 0) ? nbins : 0;
     h->wake_mode = mode;
     h->grid_lo = grid_lo;
@@ -1382,8 +1405,10 @@ int cts_set_wake(cts_handle *h, int32_t nbins, int32_t mode, double grid_lo, dou
     if ((rc = dalloc(&h->d_bhist, (size_t)2 * nb * n)) || (rc = dalloc(&h->d_counts, (size_t)nb * n)) ||
         (rc = dalloc(&h->d_kick, (size_t)nb * n)) || (rc = dalloc(&h->d_poten, (size_t)nb * n)) ||
         (rc = dalloc(&h->d_edges_prev, (size_t)nb * 2)) || (rc = dalloc(&h->d_edges_now, (size_t)nb * 2)) ||
-        (rc = dalloc(&h->d_table, (size_t)(mode == 0 ? nb : 1) * (2 * n - 1))) || (rc = dalloc(&h->d_scale, nb)))
+        (rc = dalloc(&h->d_table, (size_t)(mode == 0 ? nb : 1) * (2 * n - 1))) || (rc = dalloc(&h->d_scale, nb)) ||
+        (rc = dalloc(&h->d_terms, (size_t)2 * nres * kWakeSteps)))
         return rc;
+    HIPCHK(launch_wake_terms(table_params(h), h->d_terms, h->stream));
     // scale of srWakePoten: (-1)*e*q/E (src/MPBunch.cpp:1996-1998)
     std::vector<double> sc(nb);
     for (int b = 0; b < nb; b++) sc[b] = (-1) * kEcharge * h->macro_charge[b] / h->ring.energy;
@@ -1394,14 +1419,13 @@ int cts_set_wake(cts_handle *h, int32_t nbins, int32_t mode, double grid_lo, dou
         for (int b = 0; b < nb; b++) { ed[2 * b] = grid_lo; ed[2 * b + 1] = dz; }
         HIPCHK(hipMemcpy(h->d_edges_now, ed.data(), ed.size() * sizeof(double), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(h->d_edges_prev, ed.data(), ed.size() * sizeof(double), hipMemcpyHostToDevice));
-        WakeTableParams t;
-        std::memset(&t, 0, sizeof t);
-        t.edges = h->d_edges_now;  // bunch 0's width is the grid's
-        t.table = h->d_table;
-        t.nbins = n;
-        t.nres = nres;
-        for (int r = 0; r < nres; r++) { t.rs[r] = h->rs[r]; t.q[r] = h->q[r]; t.omega[r] = h->omega[r]; }
-        HIPCHK(launch_wake_table(t, 1, h->stream));
+        CloseParams c;  // the one lag table, at the grid's width (bunch 0's)
+        std::memset(&c, 0, sizeof c);
+        c.edges_given = 1;
+        c.edges_now = h->d_edges_now;
+        c.tables = 1;
+        c.t = table_params(h);
+        HIPCHK(launch_close(c, 0, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
     return CTS_OK;
@@ -1462,8 +1486,8 @@ static int run_lrwake(cts_handle *h, int32_t turn)
     L.fix_dp = h->nbins > 0 ? 0 : 1;  // with a short-range wake the dp moments close in the next pass
     L.turn = (uint32_t)turn;
     if (h->capturing) {
-        L.turn_dev = h->d_turn;
-        L.turn = (uint32_t)h->cap_off;
+        L.turn_dev = h->d_turn + 1;
+        L.turn = 0;
     }
     L.status = h->d_status;
     TimedScope ts(h, "lrwake");
@@ -1561,19 +1585,19 @@ static int turn_body(cts_handle *h, int32_t turn)
     // finalize: dp part of the previous record (MOMB), this turn's record
     FinParams f = base_fin(h, ops & (OP_MOMB | OP_MOMA | OP_MOMD | OP_LOSS | OP_ZSTAT | OP_LRC), slot_of(h, turn),
                            slot_of(h, h->last_turn));
+    if (h->capturing && h->cap_off == 1) f.advance = h->d_turn;
     if (wake && h->wake_mode == 1) {
         // fixed grid: moments and wake in one launch
         TimedScope ts(h, "post");
         HIPCHK(launch_post(f, wake_params(h), h->stream));
         h->hist_parity = 1 - h->hist_parity;
         h->kick_pending = true;
-    } else {
-        if ((rc = run_finalize(h, f))) return rc;
-        if (wake) {
-            if ((rc = run_bin(h))) return rc;
-            if ((rc = run_wake(h))) return rc;
-            h->kick_pending = true;
-        }
+    } else if (wake) {
+        if ((rc = run_close(h, &f))) return rc;
+        if ((rc = run_wake(h))) return rc;
+        h->kick_pending = true;
+    } else if ((rc = run_finalize(h, f))) {
+        return rc;
     }
     if (h->bbi_on && (rc = run_bbi(h))) return rc;
     if (h->lrw_T > 0 && (rc = run_lrwake(h, turn))) return rc;
@@ -1616,10 +1640,6 @@ static int capture_pair(cts_handle *h, hipGraphExec_t *out)
         for (int off = 0; off < 2 && rc == CTS_OK; off++) {
             h->cap_off = off;
             rc = turn_body(h, last_turn + 1 + off);
-        }
-        if (rc == CTS_OK) {
-            e = launch_advance_turn(h->d_turn, 2u, h->stream);
-            if (e != hipSuccess) rc = fail(CTS_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
         }
         const hipError_t e2 = hipStreamEndCapture(h->stream, &g);
         if (rc == CTS_OK && e2 != hipSuccess)
@@ -1881,9 +1901,9 @@ int cts_sr_wake(cts_handle *h, const double *sigma_z_stale)
         // length of the last MPBeamRMSCal (src/MPBunch.cpp:1900-1908)
         PassParams p = base_pass(h, OP_ZSTAT, 0);
         if ((rc = run_pass(h, p, "zstat"))) return rc;
-        FinParams f = base_fin(h, OP_ZSTAT, -1, -1);
-        if ((rc = run_finalize(h, f))) return rc;
+        const FinParams f = base_fin(h, OP_ZSTAT, -1, -1);
         if (sigma_z_stale) {
+            if ((rc = run_finalize(h, f))) return rc;
             std::vector<double> zr(2 * h->nb), ed(2 * h->nb);
             HIPCHK(hipMemcpyAsync(zr.data(), h->d_zrange, zr.size() * sizeof(double), hipMemcpyDeviceToHost,
                                   h->stream));
@@ -1896,7 +1916,7 @@ int cts_sr_wake(cts_handle *h, const double *sigma_z_stale)
             }
             HIPCHK(hipMemcpy(h->d_edges_now, ed.data(), ed.size() * sizeof(double), hipMemcpyHostToDevice));
         }
-        if ((rc = run_bin(h))) return rc;
+        if ((rc = run_close(h, sigma_z_stale ? nullptr : &f))) return rc;
     } else {
         PassParams p = base_pass(h, OP_BIN, 0);
         if ((rc = run_pass(h, p, "bin"))) return rc;

@@ -17,6 +17,12 @@ namespace cts {
 constexpr int kBlock = 256;
 constexpr int kPostWaves = 8;  // waves of a block that closes a turn (moments of a bunch, or 64 wake bins)
 constexpr int kPostBlock = 64 * kPostWaves;
+// Workgroups of the streaming pass that the device holds at one time: three
+// of 256 threads per compute unit (the turn's variants use 130 to 152
+// registers).  The default layouts cut the particles for exactly that many,
+// so that no workgroup waits for a second round: with 1024 on 256 compute
+// units the 480-bunch train's pass took 1.50 ms, with 768 1.33 ms.
+constexpr int kPassPerCu = 3;
 constexpr uint32_t kNewLost = 0x80u;
 
 enum : uint32_t {
@@ -92,6 +98,7 @@ struct PassParams {
     // turn_dev is set (graph replays read the turn from device memory)
     uint32_t turn;
     const uint32_t *turn_dev;
+    uint32_t *turn_copy;  // graph replays: the turn, for the kernels that close it (null: none)
     uint64_t seed;
     const float2 *ntab;  // normal tables (NormalTab layout: sc then lg)
     const double *lr_kick;  // [nb][3] long-range wake kick (px, py, dp) of OP_LRK
@@ -222,9 +229,10 @@ struct IonPrepParams {
 
 struct BinParams {
     const double *z;
-    const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg, *seg_step;
-    const double *edges;
+    const int64_t *bunch_off;
+    // blocks that share a bunch's particles: the bunch of every one, and
+    // every bunch's first
+    const int32_t *item_bunch, *item_first;
     uint32_t *bunch_hist;
     int32_t nbins;
 };
@@ -242,10 +250,12 @@ struct FinParams {
     double *zrange;     // survivors' z range (GetZMinMax, without the pad)
     double *edges_now;
     uint32_t *status;
-    // history slots from the device turn counter (graph replays):
-    // slot = t % hist_cap, prev_slot = (t - 1) % hist_cap, t = *turn_dev + turn_off
+    // history slots from the turn that the pass left (graph replays):
+    // slot = t % hist_cap, prev_slot = (t - 1) % hist_cap, t = *turn_dev; the
+    // last turn of a replay sets the counter of the next one (advance)
     const uint32_t *turn_dev;
-    int32_t turn_off, hist_cap;
+    uint32_t *advance;
+    int32_t hist_cap;
     double *lr_cen;       // [nb][3] post-map centroids (OP_LRC)
 };
 
@@ -357,11 +367,21 @@ struct BlWalkParams {
 hipError_t launch_bl_walk(const BlWalkParams &p, hipStream_t st);
 void lrwake_yokoya(double rx, double ry, double out[5]);
 
+constexpr int kWakeSteps = 1000;  // of the pseudo-Green function's Riemann sum
 struct WakeTableParams {
-    const double *edges;  // per table: {lo, dz}
+    const double *terms;  // [nres][kWakeSteps]{z, cos - sin / sq} (k_wake_terms)
     double *table;
     int32_t nbins, nres;
     double rs[CTS_MAX_RES], q[CTS_MAX_RES], omega[CTS_MAX_RES];
+};
+
+// k_close: the end of a turn with the reference's edges.
+struct CloseParams {
+    FinParams f;
+    BinParams b;
+    WakeTableParams t;
+    const double *edges_now;
+    int32_t fin, edges_given, tables, tab_blocks, nb;  // close the moments; edges_now is final; lag tables
 };
 
 struct WakeParams {
@@ -380,14 +400,14 @@ struct WakeParams {
 hipError_t launch_pass(const PassParams &p, int nwg, hipStream_t st);
 // Host: the NormalTab contents (2 * kNormTab float2, sc then lg).
 void build_normal_tables(float2 *out);
-// device turn counter of graph replays: *t = v, and *t += by
+// device turn counter of graph replays: *t = v
 hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st);
-hipError_t launch_advance_turn(uint32_t *t, uint32_t by, hipStream_t st);
-hipError_t launch_bin(const BinParams &p, int nwg, hipStream_t st);
+hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_t st);
+// nitem: binning blocks (0: none)
+hipError_t launch_close(CloseParams c, int nitem, hipStream_t st);
 hipError_t launch_ion_kick(const IonKickParams &p, int nwg, hipStream_t st);
 hipError_t launch_finalize(const FinParams &p, hipStream_t st);
 hipError_t launch_post(const FinParams &f, const WakeParams &w, hipStream_t st);
-hipError_t launch_wake_table(const WakeTableParams &p, int ntables, hipStream_t st);
 hipError_t launch_wake(const WakeParams &p, int nb, hipStream_t st);
 hipError_t launch_ion_prep(const IonPrepParams &p, hipStream_t st);
 // out[i] = sum over the kIonReplicas copies (stride n) of acc[i]; the

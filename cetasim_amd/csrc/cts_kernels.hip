@@ -229,8 +229,8 @@ __host__ __device__ constexpr uint32_t pass_writes(uint32_t M)
 // pass is not short of loads in flight)
 constexpr int kPassDepth = 1;
 
-template <uint32_t M, bool EXACT, int NOISE, int NRF>
-__global__ void __launch_bounds__(kBlock)
+template <uint32_t M, uint32_t RT, int NOISE, int NRF>
+__global__ void __launch_bounds__(kBlock, M != RT ? kPassPerCu : 1)
 k_pass(PassParams P)
 {
     extern __shared__ double smem_d[];
@@ -239,14 +239,16 @@ k_pass(PassParams P)
     double *bl_lds = smem_d + P.nbins + (P.nbins + 1) / 2;                // bl_nbl * (bl_nbins + 1)
     __shared__ double red[kBlock / 64][kRedExt + 4];
 
-    // EXACT variants run exactly the stages in M (no runtime stage tests);
-    // NOISE >= 0 fixes the noise source at compile time
-    const uint32_t ops = EXACT ? M : (P.ops & M);
+    // the stages in M run without a test, those also in RT only when the
+    // launch asks for them; NOISE >= 0 fixes the noise source at compile time
+    const uint32_t ops = (M & ~RT) | (P.ops & RT);
     const int noise_mode = NOISE >= 0 ? NOISE : P.noise_mode;
     const int n_rf = NRF >= 0 ? NRF : P.n_rf;
     const int tid = threadIdx.x;
     const int s_first = P.wg_seg[blockIdx.x], s_last = P.wg_seg[blockIdx.x + 1];
     const uint32_t turn = P.turn_dev ? *P.turn_dev + P.turn : P.turn;
+    // the kernels that close the turn read its number here
+    if (P.turn_copy && blockIdx.x == 0 && tid == 0) *P.turn_copy = turn;
     __shared__ NormalTab ntab;
     if ((ops & OP_SYNRAD) && noise_mode == 2) {
         load_normal_tab(ntab, P.ntab, tid, kBlock);
@@ -597,36 +599,6 @@ k_pass(PassParams P)
     }
 }
 
-// ------------------------------------------------------------ binning
-// Histogram pass for the reference's bin edges, which depend on the
-// survivors' z range after the pass (src/MPBunch.cpp:1900-1919).
-__global__ void __launch_bounds__(kBlock)
-k_bin(BinParams P)
-{
-    extern __shared__ double smem_d[];
-    uint32_t *hist_lds = reinterpret_cast<uint32_t *>(smem_d);
-    const int tid = threadIdx.x;
-    const int s_first = P.wg_seg[blockIdx.x], s_last = P.wg_seg[blockIdx.x + 1];
-    for (int s = s_first; s < s_last; s++) {
-        const int b = P.seg_bunch[s];
-        const int64_t i0 = P.seg_begin[s], i1 = P.seg_end[s];
-        for (int j = tid; j < P.nbins; j += kBlock) hist_lds[j] = 0u;
-        const double lo = P.edges[2 * b], dz = P.edges[2 * b + 1], inv = 1.0 / dz;
-        __syncthreads();
-        const int64_t step = P.seg_step[s];
-        for (int64_t i = i0 + tid; i < i1; i += step) {
-            const int hb = bin_of(P.z[i], lo, dz, inv, P.nbins);
-            if (hb >= 0) atomicAdd(&hist_lds[hb], 1u);
-        }
-        __syncthreads();
-        for (int j = tid; j < P.nbins; j += kBlock) {
-            const uint32_t c = hist_lds[j];
-            if (c) atomicAdd(&P.bunch_hist[(int64_t)b * P.nbins + j], c);
-        }
-        __syncthreads();
-    }
-}
-
 // ----------------------------------------------------------- finalize
 // Per bunch: fold the segment partials and write the moment record.  One
 // block of kPostWaves waves per bunch: a wave folds four of the values at
@@ -645,6 +617,66 @@ __device__ __forceinline__ bool part_needed(uint32_t ops, int j)
                                         : (ops & OP_LRC) != 0;
 }
 
+// values j0 .. j0 + 3 of the stages in `ops`, over segments s0 .. s1 - 1, by
+// one wave
+__device__ __forceinline__ void fold_parts(const FinParams &P, int s0, int s1, int j0, uint32_t ops, double *tot)
+{
+    const int lane = threadIdx.x & 63;
+    if (j0 >= kNPart) return;
+    double v[4], v0[4];
+    bool need[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int j = j0 + u;
+        need[u] = j < kNPart && part_needed(ops, j);
+        v0[u] = (j == A_ZMIN || j == C_ZMIN) ? INFINITY : (j == A_ZMAX || j == C_ZMAX) ? -INFINITY : 0.0;
+        v[u] = v0[u];
+    }
+    // sixteen loads in flight: four segments of four values
+    for (int s = s0 + lane; s < s1; s += 4 * 64) {
+        double x[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                x[u][q] = v0[u];
+                if (need[u] && s + 64 * q < s1) x[u][q] = P.seg_part[(int64_t)(j0 + u) * P.nseg + s + 64 * q];
+            }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int j = j0 + u;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (j == A_ZMIN || j == C_ZMIN) v[u] = fmin(v[u], x[u][q]);
+                else if (j == A_ZMAX || j == C_ZMAX) v[u] = fmax(v[u], x[u][q]);
+                else v[u] += x[u][q];
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int j = j0 + u;
+        if (!need[u]) continue;
+        double r;
+        if (j == A_ZMIN || j == C_ZMIN) r = wave_min(v[u]);
+        else if (j == A_ZMAX || j == C_ZMAX) r = wave_max(v[u]);
+        else r = wave_sum_dpp(v[u]);
+        if (lane == 0) tot[j] = r;
+    }
+}
+
+// The reference's bin edges from the survivors' z range and rms after the
+// pass (src/MPBunch.cpp:1900-1908): {lo, width}.
+__device__ __forceinline__ void ref_edges(const double *tot, int nbins, double &sig, double &lo, double &dz)
+{
+    const double n = tot[C_N];
+    const double mz = tot[C_SZ] / n;
+    sig = sqrt(tot[C_QZZ] / n - mz * mz);
+    const double zMin = tot[C_ZMIN] - 1.e-6, zMax = tot[C_ZMAX] + 1.e-6;
+    lo = zMin - 2 * sig;
+    dz = (zMax + 2 * sig - lo) / nbins;
+}
+
 __device__ __forceinline__ void finalize_body(const FinParams &P, int b)
 {
     __shared__ double tot[kNPart + 2];
@@ -657,55 +689,14 @@ __device__ __forceinline__ void finalize_body(const FinParams &P, int b)
     if (tid < 20) old = curd[tid];
     if (tid < 7) sh_l = tid == 0 ? 0.0 : sh[tid - 1];
     if (tid >= 32 && tid < 35) sh_r = sh[2 * (tid - 32)];
-    for (int j0 = 4 * wave; j0 < kNPart; j0 += 4 * kPostWaves) {
-        double v[4], v0[4];
-        bool need[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int j = j0 + u;
-            need[u] = j < kNPart && part_needed(P.ops, j);
-            v0[u] = (j == A_ZMIN || j == C_ZMIN) ? INFINITY : (j == A_ZMAX || j == C_ZMAX) ? -INFINITY : 0.0;
-            v[u] = v0[u];
-        }
-        // sixteen loads in flight: four segments of four values
-        for (int s = s0 + lane; s < s1; s += 4 * 64) {
-            double x[4][4];
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    x[u][q] = v0[u];
-                    if (need[u] && s + 64 * q < s1) x[u][q] = P.seg_part[(int64_t)(j0 + u) * P.nseg + s + 64 * q];
-                }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = j0 + u;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    if (j == A_ZMIN || j == C_ZMIN) v[u] = fmin(v[u], x[u][q]);
-                    else if (j == A_ZMAX || j == C_ZMAX) v[u] = fmax(v[u], x[u][q]);
-                    else v[u] += x[u][q];
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int j = j0 + u;
-            if (!need[u]) continue;
-            double r;
-            if (j == A_ZMIN || j == C_ZMIN) r = wave_min(v[u]);
-            else if (j == A_ZMAX || j == C_ZMAX) r = wave_max(v[u]);
-            else r = wave_sum_dpp(v[u]);
-            if (lane == 0) tot[j] = r;
-        }
-    }
+    fold_parts(P, s0, s1, 4 * wave, P.ops, tot);
     __syncthreads();
     if (wave != 0) return;
 
     const double ncount = (double)P.bunch_count[b];
     int32_t slot = P.slot, prev_slot = P.prev_slot;
     if (P.turn_dev && P.hist_cap > 0) {
-        const uint32_t t = *P.turn_dev + (uint32_t)P.turn_off;
+        const uint32_t t = *P.turn_dev;
         slot = (int32_t)(t % (uint32_t)P.hist_cap);
         prev_slot = t >= 1u ? (int32_t)((t - 1u) % (uint32_t)P.hist_cap) : -1;
     }
@@ -758,34 +749,44 @@ __device__ __forceinline__ void finalize_body(const FinParams &P, int b)
         if (((P.ops & OP_MOMA) && lane >= 1 && lane <= 5) || ((momb || momd) && lane == 6)) sh[lane - 1] = rec;
     }
     if ((P.ops & OP_ZSTAT) && lane == 63) {
-        const double n = tot[C_N];
-        const double mz = tot[C_SZ] / n;
-        const double sig = sqrt(tot[C_QZZ] / n - mz * mz);
+        double sig, lo, dz;
+        ref_edges(tot, P.nbins, sig, lo, dz);
         P.sigz_stale[b] = sig;
         P.zrange[2 * b] = tot[C_ZMIN];
         P.zrange[2 * b + 1] = tot[C_ZMAX];
         if (P.nbins > 0 && P.ref_edges) {
-            const double zMin = tot[C_ZMIN] - 1.e-6, zMax = tot[C_ZMAX] + 1.e-6;
-            const double lo = zMin - 2 * sig, hi = zMax + 2 * sig;
             P.edges_now[2 * b] = lo;
-            P.edges_now[2 * b + 1] = (hi - lo) / P.nbins;
+            P.edges_now[2 * b + 1] = dz;
         }
     }
+    // graph replays: the next replay's first turn
+    if (P.advance && b == 0 && lane == 0) *P.advance = *P.turn_dev + 1u;
 }
 
 // ---------------------------------------------------------- wake table
 // W[l] = longitudinal BBR pseudo-Green function at tau = (l-(nbins-1))*dt
 // (src/WakeFunction.cpp:558-652); one wave per lag, each lane sums a strided
-// share of the 1000-step Riemann sum.  grid = (ceil(nlag*64/256), ntables).
-__global__ void __launch_bounds__(kBlock)
-k_wake_table(WakeTableParams P)
+// share of the 1000-step Riemann sum.  The factors that do not depend on the
+// lag come from k_wake_terms ({z, cos - sin / sq} per step), which leaves an
+// exponential per step.
+__global__ void __launch_bounds__(kBlock) k_wake_terms(WakeTableParams P, double *terms)
 {
-    const int nlag = 2 * P.nbins - 1;
-    const int lag = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+    const int j = blockIdx.x * kBlock + threadIdx.x, r = blockIdx.y;
+    if (j >= kWakeSteps) return;
+    const double sigmat = 1.e-3 / kClight, sigmaz = sigmat * kClight;
+    const double Q = P.q[r], vz = P.omega[r] * sigmaz / kClight;
+    const double dz = 3 * vz / (2 * Q) / kWakeSteps;
+    const double sq = sqrt(4 * Q * Q - 1);
+    const double z = j * dz;
+    double s, c;
+    sincos(z * sq, &s, &c);
+    terms[2 * ((int64_t)r * kWakeSteps + j)] = z;
+    terms[2 * ((int64_t)r * kWakeSteps + j) + 1] = c - s / sq;
+}
+
+__device__ __forceinline__ double wake_lag(const WakeTableParams &P, double dt, int lag)
+{
     const int lane = threadIdx.x & 63;
-    const int t = blockIdx.y;
-    if (lag >= nlag) return;
-    const double dt = P.edges[2 * t + 1] / kClight;
     const double tau = (lag - (P.nbins - 1)) * dt;
     const double sigmat = 1.e-3 / kClight;
     const double u = tau / sigmat;
@@ -794,22 +795,112 @@ k_wake_table(WakeTableParams P)
     for (int r = 0; r < P.nres; r++) {
         const double Q = P.q[r];
         const double vz = P.omega[r] * sigmaz / kClight;
-        const double zMax = 3 * vz / (2 * Q);
-        const double dz = zMax / 1000;
-        const double sq = sqrt(4 * Q * Q - 1);
+        const double dz = 3 * vz / (2 * Q) / kWakeSteps;
+        const double *t = P.terms + 2 * (int64_t)r * kWakeSteps;
         double sum = 0.0;
-        for (int j = lane; j < 1000; j += 64) {
-            const double z = j * dz;
-            const double a = u + 2 * Q / vz * z;
-            const double term0 = -1 / 2.0 * (a * a) - z;
-            double s, c;
-            sincos(z * sq, &s, &c);
-            sum += exp(term0) * (c - s / sq) * dz;
+        for (int j0 = lane; j0 < kWakeSteps; j0 += 4 * 64) {
+            double2 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int j = j0 + 64 * q;
+                v[q] = *reinterpret_cast<const double2 *>(t + 2 * (j < kWakeSteps ? j : 0));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const double a = u + 2 * Q / vz * v[q].x;
+                const double term0 = -1 / 2.0 * (a * a) - v[q].x;
+                if (j0 + 64 * q < kWakeSteps) sum += exp_neg(term0) * v[q].y * dz;
+            }
         }
         sum = wave_sum(sum);
         total += (sqrt(2. / kPi) * P.rs[r] * kClight / sigmaz) * sum;
     }
-    if (lane == 0) P.table[(int64_t)t * nlag + lag] = total;
+    return total;
+}
+
+// The wake of the reference's edges, up to its bins and table, in one launch
+// after the pass: per bunch a block that closes the moments (finalize_body)
+// and blocks of the lag table, then blocks that bin the particles
+// (src/MPBunch.cpp:1915-1919).  Each of them forms the bunch's edges itself
+// from the pass's partial sums, with the same operations, so none waits for
+// another.  As three launches (moments, bins, table) they took 6.5, 20.6 and
+// 7.7 us on 1.3e6 macroparticles, together 12.3; at 2e4, where the gaps
+// between launches count, 16.5 and 7.3; with 1024 bins (a table of 2047 lags)
+// 73 and 29.  edges_given: edges_now holds them (the seam with the host's
+// bunch lengths, and the fixed grid's table).
+__global__ void __launch_bounds__(kPostBlock) k_close(CloseParams C)
+{
+    extern __shared__ double smem_d[];
+    __shared__ double tot[kNPart + 2], ed[2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const FinParams &F = C.f;
+    const int nfin = C.fin ? C.nb : 0, ntab = C.tables * C.tab_blocks;
+    int blk = blockIdx.x;
+    if (blk < nfin) {
+        finalize_body(F, blk);
+        return;
+    }
+    blk -= nfin;
+    const auto edges = [&](int b) {
+        if (!C.edges_given) {
+            const int s0 = F.bunch_seg[b], s1 = F.bunch_seg[b + 1];
+            if (wave < 2) fold_parts(F, s0, s1, wave == 0 ? C_N - 1 : C_N + 3, OP_ZSTAT, tot);
+        }
+        __syncthreads();
+        if (tid == 0) {
+            if (C.edges_given) {
+                ed[0] = C.edges_now[2 * b];
+                ed[1] = C.edges_now[2 * b + 1];
+            } else {
+                double sig;
+                ref_edges(tot, C.t.nbins, sig, ed[0], ed[1]);
+            }
+        }
+        __syncthreads();
+    };
+    if (blk < ntab) {
+        const int t = blk / C.tab_blocks, lag = (blk - t * C.tab_blocks) * kPostWaves + wave;
+        const int nlag = 2 * C.t.nbins - 1;
+        edges(t);
+        if (lag >= nlag) return;
+        const double w = wake_lag(C.t, ed[1] / kClight, lag);
+        if (lane == 0) C.t.table[(int64_t)t * nlag + lag] = w;
+        return;
+    }
+    blk -= ntab;
+    // a block bins an equal share of one bunch
+    uint32_t *hist_lds = reinterpret_cast<uint32_t *>(smem_d);
+    const BinParams &B = C.b;
+    const int b = B.item_bunch[blk];
+    const int64_t n = B.bunch_off[b + 1] - B.bunch_off[b];
+    const int nblk = B.item_first[b + 1] - B.item_first[b];
+    const int64_t per = ((n + nblk - 1) / nblk + kPostBlock - 1) / kPostBlock * kPostBlock;
+    const int64_t i0 = (int64_t)(blk - B.item_first[b]) * per, i1 = min(n, i0 + per);
+    const double *z0 = B.z + B.bunch_off[b];
+    constexpr int U = 4;  // loads in flight per thread
+    double z[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int64_t k = i0 + tid + u * kPostBlock;
+        z[u] = k < i1 ? z0[k] : INFINITY;
+    }
+    for (int j = tid; j < B.nbins; j += kPostBlock) hist_lds[j] = 0u;
+    edges(b);
+    const double lo = ed[0], dz = ed[1], inv = 1.0 / dz;
+    for (int64_t i = i0 + tid; i < i1; i += U * kPostBlock) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int hb = bin_of(z[u], lo, dz, inv, B.nbins);
+            if (hb >= 0) atomicAdd(&hist_lds[hb], 1u);
+            const int64_t k = i + (u + U) * kPostBlock;
+            z[u] = k < i1 ? z0[k] : INFINITY;
+        }
+    }
+    __syncthreads();
+    for (int j = tid; j < B.nbins; j += kPostBlock) {
+        const uint32_t c = hist_lds[j];
+        if (c) atomicAdd(&B.bunch_hist[(int64_t)b * B.nbins + j], c);
+    }
 }
 
 // --------------------------------------------------------------- wake
@@ -1200,13 +1291,19 @@ constexpr uint32_t V_BLB = V_FIX | V_REF | OP_BL;
 constexpr uint32_t V_BLH = OP_KICK | OP_MAP | OP_SKEW | OP_LRK | OP_BLH;  // bins for the cavity walk
 constexpr uint32_t V_ALL = 0xffffffffu;
 
-// stage sets of the fused turn in its steady state
-constexpr uint32_t T_QE = OP_KICK | OP_MOMB | OP_MAP | OP_RF | OP_DRIFT | OP_U0 | OP_SYNRAD | OP_BIN |
-                          OP_LOSS | OP_MOMA | OP_WRITE;
-constexpr uint32_t T_NOSR = OP_KICK | OP_MOMB | OP_MAP | OP_RF | OP_DRIFT | OP_U0 | OP_BIN | OP_LOSS |
-                            OP_MOMA | OP_WRITE;
-constexpr uint32_t T_QE_LR = T_QE | OP_LRC | OP_LRK;  // with the long-range wake
-constexpr uint32_t T_QE_BL = T_QE | OP_BL;            // a beam-loaded cavity in place of the ideal one
+// Stage sets of the fused turn: every stage a turn of the kind runs is compiled
+// in without a test; the wake kick and the moments it completes stay optional,
+// since a turn after a flush has none (it ran the general variant: 1.40 ms
+// against 1.19 on the 480-bunch train).
+constexpr uint32_t T_SR = OP_KICK | OP_MOMB | OP_MAP | OP_RF | OP_DRIFT | OP_U0 | OP_SYNRAD | OP_LOSS | OP_MOMA | OP_WRITE;
+constexpr uint32_t T_OPT = OP_KICK | OP_MOMB;
+constexpr uint32_t T_QE = T_SR | OP_BIN;      // fixed-grid wake
+constexpr uint32_t T_QE_REF = T_SR | OP_ZSTAT;  // the reference's edges
+constexpr uint32_t T_QE_NW = T_SR | OP_MOMD;  // no wake: the moments close now
+constexpr uint32_t T_NOSR = T_QE & ~OP_SYNRAD;
+constexpr uint32_t T_NOSR_REF = T_QE_REF & ~OP_SYNRAD;
+constexpr uint32_t T_QE_LR = T_QE | OP_LRC | OP_LRK;            // with the long-range wake
+constexpr uint32_t T_QE_BL = T_QE | OP_BL | OP_LRC | OP_LRK;    // a beam-loaded cavity in place of the ideal one
 
 // ---------------------------------------------------------- cavity walk
 // One turn of MPBeam::BeamMomtumUpdateDueToRFTest (src/MPBeam.cpp:2624-2706)
@@ -1389,30 +1486,29 @@ hipError_t launch_pass(const PassParams &p, int nwg, hipStream_t st)
     const size_t shm = (o & (OP_BL | OP_BLH)) ? ((size_t)p.nbins + (p.nbins + 1) / 2 + bl) * sizeof(double)
                                               : (size_t)p.nbins * (sizeof(double) + sizeof(uint32_t));
     const dim3 g(nwg), b(kBlock);
-    const bool one_rf = p.n_rf == 1;
-    if (one_rf && o == T_QE && p.noise_mode == 2)
-        hipLaunchKernelGGL((k_pass<T_QE, true, 2, 1>), g, b, shm, st, p);
-    else if (one_rf && o == T_QE_LR && p.noise_mode == 2)
-        hipLaunchKernelGGL((k_pass<T_QE_LR, true, 2, 1>), g, b, shm, st, p);
-    else if (p.n_rf == 0 && o == T_QE_BL && p.noise_mode == 2)
-        hipLaunchKernelGGL((k_pass<T_QE_BL, true, 2, 0>), g, b, shm, st, p);
-    else if (one_rf && o == T_QE && p.noise_mode == 1)
-        hipLaunchKernelGGL((k_pass<T_QE, true, 1, 1>), g, b, shm, st, p);
-    else if (one_rf && o == T_NOSR)
-        hipLaunchKernelGGL((k_pass<T_NOSR, true, 0, 1>), g, b, shm, st, p);
-    else if ((o & ~(V_KICK & ~OP_LRK)) == 0)
-        hipLaunchKernelGGL((k_pass<V_KICK & ~OP_LRK, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_Z) == 0) hipLaunchKernelGGL((k_pass<V_Z, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_LONG) == 0) hipLaunchKernelGGL((k_pass<V_LONG, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_KICK) == 0) hipLaunchKernelGGL((k_pass<V_KICK, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & OP_BL) && (o & ~V_BLB) == 0) hipLaunchKernelGGL((k_pass<V_BLB, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & OP_BLH) && (o & ~V_BLH) == 0) hipLaunchKernelGGL((k_pass<V_BLH, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & OP_MAP) && (o & ~V_BLA) == 0)
-        hipLaunchKernelGGL((k_pass<V_BLA, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_MOM) == 0) hipLaunchKernelGGL((k_pass<V_MOM, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_FIX) == 0) hipLaunchKernelGGL((k_pass<V_FIX, false, -1, -1>), g, b, shm, st, p);
-    else if ((o & ~V_REF) == 0) hipLaunchKernelGGL((k_pass<V_REF, false, -1, -1>), g, b, shm, st, p);
-    else hipLaunchKernelGGL((k_pass<V_ALL, false, -1, -1>), g, b, shm, st, p);
+    const bool one_rf = p.n_rf == 1, draws = p.noise_mode == 2;
+    const auto is = [o](uint32_t M, uint32_t RT) { return (o & ~RT) == (M & ~RT) && (o & ~M) == 0; };
+#define CTS_PASS(M, RT, NOISE, NRF) hipLaunchKernelGGL((k_pass<(M), (RT), NOISE, NRF>), g, b, shm, st, p)
+    if (one_rf && draws && is(T_QE, T_OPT)) CTS_PASS(T_QE, T_OPT, 2, 1);
+    else if (one_rf && draws && is(T_QE_REF, T_OPT)) CTS_PASS(T_QE_REF, T_OPT, 2, 1);
+    else if (one_rf && draws && is(T_QE_NW, T_OPT | OP_MOMD)) CTS_PASS(T_QE_NW, T_OPT | OP_MOMD, 2, 1);
+    else if (one_rf && draws && is(T_QE_LR, T_OPT | OP_LRK)) CTS_PASS(T_QE_LR, T_OPT | OP_LRK, 2, 1);
+    else if (p.n_rf == 0 && draws && is(T_QE_BL, T_OPT | OP_LRC | OP_LRK)) CTS_PASS(T_QE_BL, T_OPT | OP_LRC | OP_LRK, 2, 0);
+    else if (one_rf && p.noise_mode == 1 && is(T_QE, T_OPT)) CTS_PASS(T_QE, T_OPT, 1, 1);
+    else if (one_rf && is(T_NOSR, T_OPT)) CTS_PASS(T_NOSR, T_OPT, 0, 1);
+    else if (one_rf && is(T_NOSR_REF, T_OPT)) CTS_PASS(T_NOSR_REF, T_OPT, 0, 1);
+    else if ((o & ~(V_KICK & ~OP_LRK)) == 0) CTS_PASS(V_KICK & ~OP_LRK, V_KICK, -1, -1);
+    else if ((o & ~V_Z) == 0) CTS_PASS(V_Z, V_Z, -1, -1);
+    else if ((o & ~V_LONG) == 0) CTS_PASS(V_LONG, V_LONG, -1, -1);
+    else if ((o & ~V_KICK) == 0) CTS_PASS(V_KICK, V_KICK, -1, -1);
+    else if ((o & OP_BL) && (o & ~V_BLB) == 0) CTS_PASS(V_BLB, V_BLB, -1, -1);
+    else if ((o & OP_BLH) && (o & ~V_BLH) == 0) CTS_PASS(V_BLH, V_BLH, -1, -1);
+    else if ((o & OP_MAP) && (o & ~V_BLA) == 0) CTS_PASS(V_BLA, V_BLA, -1, -1);
+    else if ((o & ~V_MOM) == 0) CTS_PASS(V_MOM, V_MOM, -1, -1);
+    else if ((o & ~V_FIX) == 0) CTS_PASS(V_FIX, V_FIX, -1, -1);
+    else if ((o & ~V_REF) == 0) CTS_PASS(V_REF, V_REF, -1, -1);
+    else CTS_PASS(V_ALL, V_ALL, -1, -1);
+#undef CTS_PASS
     return hipGetLastError();
 }
 hipError_t launch_ion_kick(const IonKickParams &p, int nwg, hipStream_t st)
@@ -1431,23 +1527,21 @@ __global__ void k_set_turn(uint32_t *t, uint32_t v)
 {
     if (threadIdx.x == 0) *t = v;
 }
-__global__ void k_advance_turn(uint32_t *t, uint32_t by)
-{
-    if (threadIdx.x == 0) *t += by;
-}
 hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st)
 {
     hipLaunchKernelGGL(k_set_turn, dim3(1), dim3(64), 0, st, t, v);
     return hipGetLastError();
 }
-hipError_t launch_advance_turn(uint32_t *t, uint32_t by, hipStream_t st)
+hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_advance_turn, dim3(1), dim3(64), 0, st, t, by);
+    hipLaunchKernelGGL(k_wake_terms, dim3((kWakeSteps + kBlock - 1) / kBlock, p.nres), dim3(kBlock), 0, st, p, terms);
     return hipGetLastError();
 }
-hipError_t launch_bin(const BinParams &p, int nwg, hipStream_t st)
+hipError_t launch_close(CloseParams c, int nitem, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_bin, dim3(nwg), dim3(kBlock), (size_t)p.nbins * sizeof(uint32_t), st, p);
+    c.tab_blocks = (2 * c.t.nbins - 1 + kPostWaves - 1) / kPostWaves;
+    const int64_t grid = (int64_t)(c.fin ? c.nb : 0) + (int64_t)c.tables * c.tab_blocks + nitem;
+    hipLaunchKernelGGL(k_close, dim3((unsigned)grid), dim3(kPostBlock), (size_t)c.t.nbins * sizeof(uint32_t), st, c);
     return hipGetLastError();
 }
 hipError_t launch_finalize(const FinParams &p, hipStream_t st)
@@ -1459,13 +1553,6 @@ hipError_t launch_post(const FinParams &f, const WakeParams &w, hipStream_t st)
 {
     const dim3 g(1 + (w.nbins + 63) / 64, f.nb);
     hipLaunchKernelGGL(k_post, g, dim3(kPostBlock), wake_lds(w.nbins), st, f, w);
-    return hipGetLastError();
-}
-hipError_t launch_wake_table(const WakeTableParams &p, int ntables, hipStream_t st)
-{
-    const int nlag = 2 * p.nbins - 1;
-    const int blocks = (nlag * 64 + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_wake_table, dim3(blocks, ntables), dim3(kBlock), 0, st, p);
     return hipGetLastError();
 }
 hipError_t launch_wake(const WakeParams &p, int nb, hipStream_t st)

@@ -433,8 +433,9 @@ int cts_eigen_emit(cts_handle *h, double *out);
 int cts_sync(cts_handle *h);
 
 /* Kernel timing with HIP events on the handle's stream.  name is one of
- * "pass", "finalize", "wake_table", "bin", "ion"; avg_ms is the mean
- * duration of the launches recorded since timing was switched on. */
+ * "pass", "post", "finalize", "close", "wake", "kick", "moments", "ion_prep",
+ * "ion_turn", "ion_compact", "ion_kick", ...; avg_ms is the mean duration of
+ * the launches recorded since timing was switched on. */
 int cts_set_timing(cts_handle *h, int32_t on);
 int cts_kernel_time(cts_handle *h, const char *name, double *avg_ms, int64_t *launches);
 
