@@ -565,23 +565,26 @@ k_pass(PassParams P)
             if (store) red[wave][kRedExt + sub] = r;
         }
         __syncthreads();
-        if (tid < kNPart) {
-            const bool mn = tid == A_ZMIN || tid == C_ZMIN, mx = tid == A_ZMAX || tid == C_ZMAX;
-            // identity of the unused slots (0, +inf for minima, -inf for maxima)
-            double v = mn ? INFINITY : mx ? -INFINITY : 0.0;
+        // partial sums by the first wave, the two z ranges by the second (one
+        // value per lane without a select between them: with both in one
+        // branch per lane the compiler lost the sign of a maximum)
+        double *part = P.seg_part + (P.seg_rank ? P.seg_rank[s] : s);
+        if (tid < kNPart && tid != A_ZMIN && tid != A_ZMAX && tid != C_ZMIN && tid != C_ZMAX) {
+            double v = 0.0;
             if (acc_used(M, tid)) {
-                if (mn || mx) {
-                    const int e = kRedExt + (tid == A_ZMIN ? 0 : tid == A_ZMAX ? 1 : tid == C_ZMIN ? 2 : 3);
-                    v = red[0][e];
-                    for (int w = 1; w < kBlock / 64; w++) v = fmin(v, red[w][e]);
-                    if (mx) v = -v;
-                } else {
-                    const int e = __popc(sums & ((1u << tid) - 1u));
-                    v = red[0][e];
-                    for (int w = 1; w < kBlock / 64; w++) v = v + red[w][e];
-                }
+                const int e = __popc(sums & ((1u << tid) - 1u));
+                v = red[0][e];
+                for (int w = 1; w < kBlock / 64; w++) v = v + red[w][e];
             }
-            P.seg_part[(int64_t)tid * P.nseg + (P.seg_rank ? P.seg_rank[s] : s)] = v;
+            part[(int64_t)tid * P.nseg] = v;
+        }
+        if (tid >= 64 && tid < 68) {
+            static_assert(A_ZMAX == A_ZMIN + 1 && C_ZMAX == C_ZMIN + 1, "two ranges");
+            const int q = tid - 64;  // A min, -(A max), C min, -(C max); infinite where unused
+            double v = INFINITY;
+            if (M & (OP_MOMA | OP_ZSTAT))
+                for (int w = 0; w < kBlock / 64; w++) v = fmin(v, red[w][kRedExt + q]);
+            part[(int64_t)(A_ZMIN + (q & 1) + (q >> 1) * (C_ZMIN - A_ZMIN)) * P.nseg] = copysign(1.0, 0.5 - (q & 1)) * v;
         }
         if (use_hist) {
             for (int j = tid; j < P.nbins; j += kBlock) {

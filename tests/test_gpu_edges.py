@@ -45,11 +45,13 @@ def test_reference_edges(nbins, counts, layout):
     z_map = tr.download()["z"]
     tr.turn(1)
     cnt, edges, kick = tr.wake_state()
+    mom = tr.moments()
     off = np.concatenate([[0], np.cumsum(counts)])
     z_all = tr.download()["z"]
     rs, qq, om = (np.array(BBR[c], float) for c in ("rs", "q", "fr"))
     for b in range(nb):
         z = z_all[off[b]:off[b + 1]]
+        assert mom[b]["zmin"] == z.min() and mom[b]["zmax"] == z.max()
         sig = np.std(z_map[off[b]:off[b + 1]])
         lo, hi = z.min() - 1e-6 - 2 * sig, z.max() + 1e-6 + 2 * sig
         assert abs(edges[b, 0] - lo) <= 1e-11 * (hi - lo)
