@@ -190,7 +190,8 @@ struct cts_handle {
     BbiTable bbi;
     uint32_t *d_bbi_hist = nullptr;                 // [nb][n]
     unsigned long long *d_bbi_dsum = nullptr;       // [nb][n][4] (dipolar planes)
-    double *d_bbi_prof = nullptr, *d_bbi_wake = nullptr;  // [3][nb][n], [5][nb][n]
+    double *d_bbi_prof = nullptr, *d_bbi_wake = nullptr, *d_bbi_kick = nullptr;  // [3][nb][n], [5][nb][n] twice
+    int *d_bbi_range = nullptr;                     // [nb][2]
     double *d_bbi_g = nullptr, *d_bbi_scale = nullptr;    // [n], [nb]
 
     // beam-loaded cavities (cts_set_beam_loading)
@@ -271,12 +272,14 @@ void free_bl_state(cts_handle *h)
 
 void free_bbi_state(cts_handle *h)
 {
-    void *ptrs[] = {h->d_bbi_hist, h->d_bbi_prof, h->d_bbi_wake, h->d_bbi_g, h->d_bbi_scale, h->d_bbi_dsum};
+    void *ptrs[] = {h->d_bbi_hist, h->d_bbi_prof, h->d_bbi_wake, h->d_bbi_g, h->d_bbi_scale, h->d_bbi_dsum,
+                    h->d_bbi_kick, h->d_bbi_range};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     h->d_bbi_hist = nullptr;
     h->d_bbi_dsum = nullptr;
-    h->d_bbi_prof = h->d_bbi_wake = h->d_bbi_g = h->d_bbi_scale = nullptr;
+    h->d_bbi_prof = h->d_bbi_wake = h->d_bbi_kick = h->d_bbi_g = h->d_bbi_scale = nullptr;
+    h->d_bbi_range = nullptr;
     h->bbi_on = false;
     h->bbi = BbiTable{};
 }
@@ -285,14 +288,17 @@ BbiParams bbi_params(cts_handle *h)
 {
     BbiParams p{};
     p.n = h->bbi.n; p.is = h->bbi.is; p.ie = h->bbi.ie; p.nb = h->nb; p.td = h->bbi.td; p.nw = h->bbi.nw;
-    p.zmin = h->bbi.zmin; p.dz = h->bbi.dz; p.half = h->bbi.half; p.bx = h->bbi.bx; p.by = h->bbi.by;
+    p.zmin = h->bbi.zmin; p.dz = h->bbi.dz; p.inv_dz = 1.0 / p.dz; p.half = h->bbi.half; p.bx = h->bbi.bx; p.by = h->bbi.by;
     for (int q = 0; q < 5; q++) p.planes[q] = h->bbi.planes[q];
     p.energy = h->ring.energy; p.beta2 = std::pow(h->ring.rbeta, 2);
-    p.seg_begin = h->d_seg_begin; p.seg_end = h->d_seg_end;
-    p.seg_bunch = h->d_seg_bunch; p.wg_seg = h->d_wg_seg; p.seg_step = h->d_seg_step;
+    p.bunch_off = h->d_bunch_off;
+    p.item_bunch = h->d_bin_bunch; p.item_first = h->d_bin_first;
+    p.kick_bunch = h->d_item_bunch; p.kick_first = h->d_item_first;
+    p.cur = h->d_cur;
     p.x = h->d_x; p.y = h->d_y; p.z = h->d_z;
     p.px = h->d_px; p.py = h->d_py; p.dp = h->d_dp; p.flag = h->d_flag;
     p.hist = h->d_bbi_hist; p.dsum = h->d_bbi_dsum; p.prof = h->d_bbi_prof; p.wake = h->d_bbi_wake;
+    p.kick = h->d_bbi_kick; p.range = h->d_bbi_range;
     p.g = h->d_bbi_g; p.scale = h->d_bbi_scale;
     for (int j = 0; j < kBbiTaps; j++) p.taps[j] = h->bbi.taps[j];
     return p;
@@ -725,8 +731,9 @@ int reset_status(cts_handle *h)
 // the end, so more of them soon cost more in atomics than they bin (1.3e6
 // macroparticles, k_close by blocks: 32 27 us, 64 18, 128 14.9, 256 15.3,
 // 1024 29), and a small bunch takes one per 4096 (6e4 with 1024 bins: 15
-// blocks 32 us, 59 44, 118 66).
-constexpr int64_t kBinBlocks = 128, kBinMin = 4096;
+// blocks 32 us, 59 44, 118 66); a large one takes more of them, up to 16384
+// each.
+constexpr int64_t kBinBlocks = 128, kBinMin = 4096, kBinMax = 16384;
 
 struct Seg {
     int64_t begin, end;
@@ -1254,7 +1261,9 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
         return CTS_OK;
     };
     const auto kick_items = [](int64_t n) { return (n + kBlock - 1) / kBlock; };
-    const auto bin_items = [](int64_t n) { return std::min<int64_t>(kBinBlocks, (n + kBinMin - 1) / kBinMin); };
+    const auto bin_items = [](int64_t n) {
+        return std::min(std::max(kBinBlocks, n / kBinMax), (n + kBinMin - 1) / kBinMin);
+    };
     if ((rc = cut_items(kick_items, &h->d_item_bunch, &h->d_item_first, &h->nitem)) ||
         (rc = cut_items(bin_items, &h->d_bin_bunch, &h->d_bin_first, &h->nbin_item)) ||
         (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)) ||
@@ -1504,14 +1513,14 @@ int run_bbi(cts_handle *h)
     const BbiParams p = bbi_params(h);
     {
         TimedScope ts(h, "bbi_bin");
-        HIPCHK(launch_bbi_bin(p, h->nwg, h->stream));
+        HIPCHK(launch_bbi_bin(p, h->nbin_item, h->stream));
     }
     {
         TimedScope ts(h, "bbi_wake");
         HIPCHK(launch_bbi_wake(p, h->stream));
     }
     TimedScope ts(h, "bbi_kick");
-    HIPCHK(launch_bbi_kick(p, h->nwg, h->stream));
+    HIPCHK(launch_bbi_kick(p, h->nitem, h->stream));
     h->kick_pending = true;
     return CTS_OK;
 }
@@ -2023,7 +2032,8 @@ int cts_set_bbimp(cts_handle *h, const cts_bbimp_config *cfg)
     const bool dip = h->bbi.planes[1] || h->bbi.planes[2];
     const size_t ng = h->bbi.g.size();
     if ((rc = dalloc(&h->d_bbi_hist, (size_t)nb * n)) || (rc = dalloc(&h->d_bbi_prof, 3 * (size_t)nb * n)) ||
-        (rc = dalloc(&h->d_bbi_wake, 5 * (size_t)nb * n)) || (rc = dalloc(&h->d_bbi_g, ng)) ||
+        (rc = dalloc(&h->d_bbi_wake, 5 * (size_t)nb * n)) ||
+        (rc = dalloc(&h->d_bbi_kick, 5 * (size_t)nb * n)) || (rc = dalloc(&h->d_bbi_range, 2 * (size_t)nb)) || (rc = dalloc(&h->d_bbi_g, ng)) ||
         (rc = dalloc(&h->d_bbi_scale, (size_t)nb)) || (dip && (rc = dalloc(&h->d_bbi_dsum, 4 * (size_t)nb * n)))) {
         free_bbi_state(h);
         return rc;
@@ -2039,6 +2049,7 @@ int cts_set_bbimp(cts_handle *h, const cts_bbimp_config *cfg)
     HIPCHK(hipMemset(h->d_bbi_hist, 0, (size_t)nb * n * sizeof(uint32_t)));
     if (dip) HIPCHK(hipMemset(h->d_bbi_dsum, 0, 4 * (size_t)nb * n * sizeof(unsigned long long)));
     HIPCHK(hipMemset(h->d_bbi_wake, 0, 5 * (size_t)nb * n * sizeof(double)));
+    HIPCHK(hipMemset(h->d_bbi_kick, 0, 5 * (size_t)nb * n * sizeof(double)));
     HIPCHK(hipMemset(h->d_bbi_prof, 0, 3 * (size_t)nb * n * sizeof(double)));
     h->bbi_on = true;
     cts_handle::KeepBbi k;

@@ -12,11 +12,11 @@
 // computed once on the host.  The transverse planes multiply the spectrum by
 // i Z and keep the + sign; the quadrupolar ones use the charge profile, the
 // dipolar ones the x- and y-weighted profiles (sum of charge times x per
-// bin).  Per turn: an LDS histogram per workgroup segment (with the
+// bin).  Per turn: LDS histograms of shares of the bunches (with the
 // dipolar planes, the per-bin sums of x and y as two-limb fixed-point
-// integers, so they do not depend on the order of the atomics), one block
-// per bunch for the smoothing and the convolutions, and a kick sweep.  The
-// smoothing is GSL's gsl_filter_gaussian (GSL 2.8, the version the
+// integers, so they do not depend on the order of the atomics), a block per
+// profile for the smoothing, a block per 256 bins and plane for the
+// convolutions, and a kick with a particle per thread.  The smoothing is GSL's gsl_filter_gaussian (GSL 2.8, the version the
 // reference builds against) with K = 51, alpha = 10 and
 // GSL_FILTER_END_PADVALUE: y_i = sum_j w_j x_{clamp(i + j - 25)},
 // w_j = exp(-alpha^2 ((j - 25)/25)^2 / 2) normalised to sum 1, followed by
@@ -29,12 +29,7 @@
 // way, takes the mean x and y of each bin, and sums the wake table over the
 // bins behind each one: V_i = -sum_{j >= i} w[j - i] rho_j (the dipolar
 // planes rho_j <x>_j).  No transform: the sums run over the bins where rho
-// is nonzero (zeros add nothing), one block per bunch.
-//
-// A bunch fills a small part of the grid, so the binning histograms each
-// workgroup segment over the range of bins its particles reach, in LDS
-// windows of up to kBbiWin bins: one sweep over the segment finds the
-// range, one sweep per window bins it.
+// is nonzero (zeros add nothing).
 #include <climits>
 #include <cmath>
 #include <string>
@@ -160,17 +155,23 @@ namespace {
 
 // bin of z as the reference indexes it, (int)((z - zmin + dz/2)/dz) in the
 // frequency domain, (int)((z - zmin)/dz) in the time domain, or -1 off the
-// grid (the reference does not test the range)
+// grid (the reference does not test the range).  With the reciprocal, and
+// the division where the two could truncate apart.
+__device__ __forceinline__ double bbi_pos(double z, const BbiParams &P)
+{
+    const double d = z - P.zmin + P.half;
+    double q = d * P.inv_dz;
+    if (fabs(q - rint(q)) < 1e-9) q = d / P.dz;
+    return q;
+}
 __device__ __forceinline__ int bbi_bin(double z, const BbiParams &P)
 {
-    const double q = (z - P.zmin + P.half) / P.dz;
+    const double q = bbi_pos(z, P);
     return (q > -1.0 && q < (double)P.n) ? (int)q : -1;
 }
 
 // survivors before this turn's loss marking
 __device__ __forceinline__ bool bbi_alive(uint8_t f) { return (f & 3u) == 0u || (f & kNewLost); }
-
-constexpr int kUnroll = 4;  // particles per thread per step of the sweeps
 
 // a coordinate as two integer limbs, v ~ hi 2^-30 + lo 2^-62, hi =
 // floor(v 2^30), 0 <= lo <= 2^32: the limb sums of up to 2^31 values with
@@ -193,124 +194,158 @@ __device__ __forceinline__ double fx2_value(unsigned long long hi, unsigned long
 // LDS of the binning: counts, then (dipolar planes) four limb sums per bin
 __host__ __device__ constexpr int bbi_count_words(bool dip) { return dip ? ((kBbiDipWin + 1) & ~1) : kBbiWin; }
 
-__global__ void __launch_bounds__(kBlock) k_bbi_bin(BbiParams P)
+// Binning, a share of one bunch per block, bound by the time its few loads
+// and LDS atomics take one after another.  The window is the bins of the
+// survivors' z range, which the turn's moments hold (no sweep for the range);
+// a macroparticle marked lost this turn may lie outside and goes to the
+// bunch's sums directly.  A bunch fills few bins, so the window is kept in as
+// many copies as fit, up to one per wave: the atomics of different waves do
+// not meet.  With one window of the whole grid per workgroup of the pass 37 us
+// on 60 bunches of 6e4 with both dipolar planes, 27 now (blocks of 512
+// threads 29, of 1024 40); without the planes 15 (512: 16, 1024: 22).
+__global__ void __launch_bounds__(kBbiBinBlock) k_bbi_bin(BbiParams P)
 {
     extern __shared__ __attribute__((aligned(16))) uint32_t hl[];
-    __shared__ int krange[2];
-    const int tid = threadIdx.x;
+    constexpr int U = 4, kCopies = kBbiBinBlock / 64;
+    const int tid = threadIdx.x, b = P.item_bunch[blockIdx.x];
+    if (P.scale[b] == 0.0) return;  // uniform
     const bool dipx = P.planes[1] != 0, dipy = P.planes[2] != 0, dip = dipx || dipy;
-    // dipolar sums [window][4]: x hi, x lo, y hi, y lo (8-byte aligned after the counts)
+    const int64_t first = P.bunch_off[b], n = P.bunch_off[b + 1] - first;
+    const int nblk = P.item_first[b + 1] - P.item_first[b];
+    const int64_t per = (n + nblk - 1) / nblk;
+    const int64_t i0 = first + (int64_t)(blockIdx.x - P.item_first[b]) * per, i1 = min(first + n, i0 + per);
+    if (i0 >= i1) return;
+    const auto edge = [&](double z) {
+        const double q = bbi_pos(z, P);
+        return q > 0.0 ? (q < (double)P.n ? (int)q : P.n - 1) : 0;
+    };
+    const int klo = edge(P.cur[b].zmin), khi = max(klo, edge(P.cur[b].zmax)), R = khi - klo + 1;
+    const int cap = dip ? kBbiDipWin : kBbiWin, W = min(R, cap), nc = min(kCopies, cap / W);
+    // [copy][bin] counts; [copy][limb][bin] x hi, x lo, y hi, y lo
+    const int copy = tid / 64 % nc;
+    uint32_t *hc = hl + copy * W;
     unsigned long long *ds = reinterpret_cast<unsigned long long *>(hl + bbi_count_words(dip));
-    for (int s = P.wg_seg[blockIdx.x]; s < P.wg_seg[blockIdx.x + 1]; s++) {
-        const int b = P.seg_bunch[s];
-        if (P.scale[b] == 0.0) continue;  // uniform: the whole block skips
-        const int64_t e = P.seg_end[s], step = P.seg_step[s];
-        // the range of bins the segment's counted particles reach; a grid
-        // that fits one window is taken whole (no sweep for the range)
-        const bool whole = P.n <= (dip ? kBbiDipWin : kBbiWinCopies);
-        if (tid == 0) { krange[0] = whole ? 0 : INT_MAX; krange[1] = whole ? P.n - 1 : -1; }
+    unsigned long long *dc = ds + (size_t)copy * 4 * W;
+    uint32_t *gh = P.hist + (int64_t)b * P.n;
+    unsigned long long *gd = P.dsum + (int64_t)b * 4 * P.n;  // not read without the dipolar planes
+    for (int w0 = klo; w0 <= khi; w0 += W) {
+        const int wn = min(W, khi - w0 + 1);
+        for (int j = tid; j < nc * W; j += kBbiBinBlock) hl[j] = 0u;
+        if (dip)
+            for (int j = tid; j < 4 * nc * W; j += kBbiBinBlock) ds[j] = 0ull;
         __syncthreads();
-        int rlo = INT_MAX, rhi = -1;
-        for (int64_t i0 = P.seg_begin[s] + tid; !whole && i0 < e; i0 += kUnroll * step) {
-            double zz[kUnroll];
-            uint8_t ff[kUnroll];
+        for (int64_t i = i0 + tid; i < i1; i += U * kBbiBinBlock) {
+            double zz[U], xx[U], yy[U];
+            uint8_t ff[U];
 #pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + u * step;
-                ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
-                zz[u] = i < e ? P.z[i] : 0.0;
+            for (int u = 0; u < U; u++) {
+                const int64_t k = min(i + u * kBbiBinBlock, i1 - 1);
+                ff[u] = P.flag[k];
+                zz[u] = P.z[k];
+                xx[u] = dipx ? P.x[k] : 0.0;
+                yy[u] = dipy ? P.y[k] : 0.0;
             }
 #pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const int k = bbi_alive(ff[u]) ? bbi_bin(zz[u], P) : -1;
-                if (k >= 0) { rlo = min(rlo, k); rhi = max(rhi, k); }
-            }
-        }
-        if (rhi >= 0) { atomicMin(&krange[0], rlo); atomicMax(&krange[1], rhi); }
-        __syncthreads();
-        const int klo = krange[0], khi = krange[1];
-        __syncthreads();  // krange is reset by the next segment
-        if (khi < klo) continue;
-        // narrow ranges: one copy of the counts per wave (a bunch fills few
-        // bins, so the waves' atomics would collide on one copy)
-        const int nc = (!dip && khi - klo < kBbiWinCopies) ? kBlock / 64 : 1;
-        const int W = dip ? kBbiDipWin : (nc > 1 ? kBbiWinCopies : kBbiWin);
-        uint32_t *mine = hl + (tid / 64 % nc) * W;
-        for (int w0 = klo; w0 <= khi; w0 += W) {
-            const int wn = min(W, khi - w0 + 1);
-            for (int j = tid; j < nc * W; j += kBlock) hl[j] = 0u;
-            if (dip)
-                for (int j = tid; j < 4 * wn; j += kBlock) ds[j] = 0ull;
-            __syncthreads();
-            // four particles per thread in flight: all loads before any use
-            for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * step) {
-                double zz[kUnroll], xx[kUnroll], yy[kUnroll];
-                uint8_t ff[kUnroll];
-#pragma unroll
-                for (int u = 0; u < kUnroll; u++) {
-                    const int64_t i = i0 + u * step;
-                    ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
-                    zz[u] = i < e ? P.z[i] : 0.0;
-                    xx[u] = (i < e && dipx) ? P.x[i] : 0.0;
-                    yy[u] = (i < e && dipy) ? P.y[i] : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < kUnroll; u++) {
-                    if (!bbi_alive(ff[u])) continue;
-                    const int k = bbi_bin(zz[u], P) - w0;
-                    if (k < 0 || k >= wn) continue;
-                    atomicAdd(&mine[k], 1u);
+            for (int u = 0; u < U; u++) {
+                if (i + u * kBbiBinBlock >= i1 || !bbi_alive(ff[u])) continue;
+                const int k = bbi_bin(zz[u], P), kw = k - w0;
+                unsigned long long xh, xl, yh, yl;
+                if (dipx) fx2_split(xx[u], xh, xl);
+                if (dipy) fx2_split(yy[u], yh, yl);
+                if (kw >= 0 && kw < wn) {
+                    atomicAdd(&hc[kw], 1u);
                     if (dipx) {
-                        unsigned long long hi, lo;
-                        fx2_split(xx[u], hi, lo);
-                        atomicAdd(&ds[4 * k], hi);
-                        atomicAdd(&ds[4 * k + 1], lo);
+                        atomicAdd(&dc[kw], xh);
+                        atomicAdd(&dc[W + kw], xl);
                     }
                     if (dipy) {
-                        unsigned long long hi, lo;
-                        fx2_split(yy[u], hi, lo);
-                        atomicAdd(&ds[4 * k + 2], hi);
-                        atomicAdd(&ds[4 * k + 3], lo);
+                        atomicAdd(&dc[2 * W + kw], yh);
+                        atomicAdd(&dc[3 * W + kw], yl);
+                    }
+                } else if (w0 == klo && k >= 0 && (k < klo || k > khi)) {
+                    atomicAdd(&gh[k], 1u);
+                    if (dipx) {
+                        atomicAdd(&gd[4 * k], xh);
+                        atomicAdd(&gd[4 * k + 1], xl);
+                    }
+                    if (dipy) {
+                        atomicAdd(&gd[4 * k + 2], yh);
+                        atomicAdd(&gd[4 * k + 3], yl);
                     }
                 }
             }
-            __syncthreads();
-            for (int j = tid; j < wn; j += kBlock) {
-                uint32_t c = 0;
-                for (int q = 0; q < nc; q++) c += hl[q * W + j];
-                if (c) atomicAdd(&P.hist[(int64_t)b * P.n + w0 + j], c);
-            }
-            if (dip)
-                for (int j = tid; j < 4 * wn; j += kBlock) {
-                    const unsigned long long v = ds[j];
-                    if (v) atomicAdd(&P.dsum[((int64_t)b * P.n + w0) * 4 + j], v);
-                }
-            __syncthreads();
         }
+        __syncthreads();
+        for (int j = tid; j < wn; j += kBbiBinBlock) {
+            uint32_t c = 0;
+            for (int q = 0; q < nc; q++) c += hl[q * W + j];
+            if (c) atomicAdd(&gh[w0 + j], c);
+        }
+        if (dip)
+            for (int j = tid; j < 4 * wn; j += kBbiBinBlock) {
+                unsigned long long v = 0;
+                for (int q = 0; q < nc; q++) v += ds[(4 * q + (j & 3)) * W + (j >> 2)];
+                if (v) atomicAdd(&gd[4 * (int64_t)w0 + j], v);
+            }
+        __syncthreads();
     }
 }
 
-// The smoothed profile over [is, ie) of one bunch from its raw profile
-// raw(i) (the reference's GetSmoothedBunchProfileGassionFilter), raw values
-// elsewhere; written to prof[0, n).  raw vanishes outside [lo, hi], so the
-// smoothed values vanish outside [lo - 25, hi + 25]: only those are formed.
-template <typename Raw>
-__device__ void bbi_smooth(const BbiParams &P, Raw raw, double *prof, double (*red)[kBlock], int lo, int hi)
+// One profile of one bunch (blockIdx.y: charge, x- and y-weighted): the
+// smoothed values over [is, ie) (the reference's
+// GetSmoothedBunchProfileGassionFilter), raw ones elsewhere; the time
+// domain's other two are the mean x and y per bin.  The raw profile vanishes
+// outside the bins that hold particles, [lo, hi], so the smoothed one does
+// outside [lo - 25, hi + 25]: only those are formed, from LDS tiles.  One
+// block per bunch did this and the convolutions in 60.9 us on 60 bunches of
+// 1200 bins; the two launches take 17.5.
+__global__ void __launch_bounds__(kBlock) k_bbi_prof(BbiParams P)
 {
-    const int tid = threadIdx.x;
-    const int nr = P.ie - P.is, half = (kBbiTaps - 1) / 2;
+    constexpr int T = 1024, half = (kBbiTaps - 1) / 2;
+    __shared__ double tile[T + 2 * half], red[2][kBlock];
+    __shared__ int krange[2];
+    const int b = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+    if (r > 0 && !P.planes[r]) return;
+    const double sc = P.scale[b];
+    if (sc == 0.0) return;  // the tables stay zero
+    const uint32_t *cnt = P.hist + (int64_t)b * P.n;
+    const unsigned long long *ds = P.dsum + (int64_t)b * 4 * P.n + 2 * (r - 1);  // read for r > 0
+    double *prof = P.prof + ((int64_t)r * P.nb + b) * P.n;
+    if (tid == 0) { krange[0] = INT_MAX; krange[1] = -1; }
+    __syncthreads();
+    {
+        int lo = INT_MAX, hi = -1;
+#pragma unroll 8
+        for (int j = tid; j < P.n; j += kBlock)
+            if (cnt[j]) { lo = min(lo, j); hi = max(hi, j); }
+        if (hi >= 0) { atomicMin(&krange[0], lo); atomicMax(&krange[1], hi); }
+    }
+    __syncthreads();
+    const bool any = krange[1] >= krange[0];
+    const int lo = any ? krange[0] : 0, hi = any ? krange[1] : -1;
+    if (r == 0 && tid == 0) { P.range[2 * b] = lo; P.range[2 * b + 1] = hi; }
+    if (P.td && r > 0) {
+        for (int j = tid; j < P.n; j += kBlock)
+            prof[j] = cnt[j] ? fx2_value(ds[4 * j], ds[4 * j + 1]) / cnt[j] : 0.0;
+        return;
+    }
+    const auto raw = [&](int i) { return r == 0 ? (double)cnt[i] * sc : sc * fx2_value(ds[4 * i], ds[4 * i + 1]); };
     const int a = max(P.is, lo - half), e = min(P.ie, hi + half + 1);
     double s0 = 0, s1 = 0;
-    for (int i = a + tid; i < e; i += kBlock) {
-        double y = 0;
-        for (int j = 0; j < kBbiTaps; j++) {
-            int k = i - P.is + j - half;
-            k = k < 0 ? 0 : (k >= nr ? nr - 1 : k);
-            y += P.taps[j] * raw(P.is + k);
+    for (int t0 = a; t0 < e; t0 += T) {
+        const int tn = min(T, e - t0);
+        __syncthreads();  // the tile before
+        for (int m = tid; m < tn + 2 * half; m += kBlock)
+            tile[m] = raw(min(max(t0 - half + m, P.is), P.ie - 1));
+        __syncthreads();
+        for (int i = tid; i < tn; i += kBlock) {
+            double y = 0;
+#pragma unroll
+            for (int j = 0; j < kBbiTaps; j++) y += P.taps[j] * tile[i + j];
+            s0 += tile[i + half];
+            s1 += y;
+            prof[t0 + i] = y;  // scaled below by the same thread
         }
-        s0 += raw(i);
-        s1 += y;
-        prof[i] = y;
     }
     red[0][tid] = s0;
     red[1][tid] = s1;
@@ -319,179 +354,112 @@ __device__ void bbi_smooth(const BbiParams &P, Raw raw, double *prof, double (*r
         if (tid < w) { red[0][tid] += red[0][tid + w]; red[1][tid] += red[1][tid + w]; }
         __syncthreads();
     }
-    const double r = red[1][0] != 0.0 ? red[0][0] / red[1][0] : 0.0;
-    __syncthreads();  // red is reused by the next profile
-    for (int i = tid; i < P.n; i += kBlock) {
-        if (i >= a && i < e) prof[i] *= r;
-        else if (i >= P.is && i < P.ie) prof[i] = 0.0;
-        else prof[i] = raw(i);
-    }
-    __syncthreads();
+    const double f = red[1][0] != 0.0 ? red[0][0] / red[1][0] : 0.0;
+    for (int i = a + tid; i < e; i += kBlock) prof[i] *= f;
+    for (int i = tid; i < P.n; i += kBlock)
+        if (i < a || i >= e) prof[i] = (i >= P.is && i < P.ie) ? 0.0 : raw(i);
 }
 
-// one block per bunch: the profiles, their smoothing, the induced voltages;
-// the histogram and dipolar sums of the bunch are cleared for the next turn
-// (fills, no memset node)
+// The induced voltage of one plane (blockIdx.z) on 256 bins of one bunch:
+// frequency domain, longitudinal V = -IDFT(I Z) and transverse
+// V = +IDFT(I i Z), circular convolutions of the profile (dipolar planes: the
+// weighted ones); time domain, V_i = -sum_{j >= i} w[j - i] rho_j (dipolar
+// planes rho_j <x>_j) over the rows of the wake (src/MPBunch.cpp:2100-2111).
+// Both sum over the nonzero part of the profile in the order of its bins, with
+// tiles of profile and weights in LDS.  The voltage over energy, beta^2 (and
+// beta function, where the kick has it first) goes to the kick's own table:
+// no division per macroparticle.  Clears the bins' sums for the next turn
+// (stores, no memset node).
 __global__ void __launch_bounds__(kBlock) k_bbi_wake(BbiParams P)
 {
-    __shared__ double red[2][kBlock];
-    __shared__ int krange[2];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const int64_t nbn = (int64_t)P.nb * P.n;
-    uint32_t *cnt = P.hist + (int64_t)b * P.n;
-    unsigned long long *ds = P.dsum ? P.dsum + (int64_t)b * 4 * P.n : nullptr;
-    double *prof[3] = {P.prof + (int64_t)b * P.n, P.prof + nbn + (int64_t)b * P.n,
-                       P.prof + 2 * nbn + (int64_t)b * P.n};
-    const double sc = P.scale[b];
-    if (sc == 0.0) {
-        for (int j = tid; j < P.n; j += kBlock) {
-            for (int q = 0; q < 5; q++) P.wake[((int64_t)q * P.nb + b) * P.n + j] = 0.0;
-            for (int r = 0; r < 3; r++) prof[r][j] = 0.0;
-            cnt[j] = 0u;
-            if (ds)
-                for (int c = 0; c < 4; c++) ds[4 * j + c] = 0ull;
-        }
-        return;
+    constexpr int T = 256;
+    __shared__ double pr[T], gt[T + kBlock];
+    const int b = blockIdx.x, q = blockIdx.z, tid = threadIdx.x;
+    const int o0 = blockIdx.y * kBlock, o = o0 + tid, n = P.n;
+    if (P.scale[b] == 0.0) return;  // the tables stay zero
+    const int lo = P.range[2 * b], hi = P.range[2 * b + 1];
+    if (q == 0 && o < n) {
+        P.hist[(int64_t)b * n + o] = 0u;
+        if (P.dsum)
+            for (int c = 0; c < 4; c++) P.dsum[((int64_t)b * n + o) * 4 + c] = 0ull;
     }
-    // the bins holding particles
-    if (tid == 0) { krange[0] = INT_MAX; krange[1] = -1; }
-    __syncthreads();
-    {
-        int lo = INT_MAX, hi = -1;
-        for (int j = tid; j < P.n; j += kBlock)
-            if (cnt[j]) { lo = min(lo, j); hi = max(hi, j); }
-        if (hi >= 0) { atomicMin(&krange[0], lo); atomicMax(&krange[1], hi); }
-    }
-    __syncthreads();
-    const bool any = krange[1] >= krange[0];
-    const int lo = any ? krange[0] : 0, hi = any ? krange[1] : -1;
+    if (!P.planes[q]) return;
+    const int half = (kBbiTaps - 1) / 2;
     // every nonzero value of a profile lies in [plo, phi]
-    const int plo = max(0, lo - (kBbiTaps - 1) / 2), phi = min(P.n - 1, hi + (kBbiTaps - 1) / 2);
-    const int src[5] = {0, 1, 2, 0, 0};
-    if (!P.td) {
-        bbi_smooth(P, [&](int i) { return (double)cnt[i] * sc; }, prof[0], red, lo, hi);
-        if (P.planes[1])
-            bbi_smooth(P, [&](int i) { return sc * fx2_value(ds[4 * i], ds[4 * i + 1]); }, prof[1], red, lo, hi);
-        if (P.planes[2])
-            bbi_smooth(P, [&](int i) { return sc * fx2_value(ds[4 * i + 2], ds[4 * i + 3]); }, prof[2], red, lo, hi);
-        // longitudinal V = -IDFT(I Z); transverse V = +IDFT(I i Z), the
-        // dipolar planes from the weighted profiles: circular convolutions
-        // over the nonzero part of the profile, in the order of i
-        for (int q = 0; q < 5; q++) {
-            if (!P.planes[q]) continue;
-            const double *g = P.g + (int64_t)q * P.n;
-            const double *pr = prof[src[q]];
-            double *wake = P.wake + ((int64_t)q * P.nb + b) * P.n;
-            for (int j = tid; j < P.n; j += kBlock) {
-                double v = 0;
-                int m = j - plo;  // (j - i) mod n for i = plo, plo + 1, ...
-                if (m < 0) m += P.n;
-                for (int i = plo; i <= phi; i++) {
-                    v += pr[i] * g[m];
-                    m = m == 0 ? P.n - 1 : m - 1;
-                }
-                wake[j] = q == 0 ? -v : v;
-            }
-        }
-    } else {
-        // charge per bin, smoothed over the whole grid (src/MPBunch.cpp:
-        // 2048-2056); the mean x and y of each bin (2058-2082)
-        bbi_smooth(P, [&](int i) { return (double)cnt[i] * sc; }, prof[0], red, lo, hi);
-        for (int r = 1; r < 3; r++) {
-            if (!P.planes[r]) continue;
-            for (int j = tid; j < P.n; j += kBlock)
-                prof[r][j] = cnt[j] ? fx2_value(ds[4 * j + 2 * (r - 1)], ds[4 * j + 2 * (r - 1) + 1]) / cnt[j] : 0.0;
+    const int plo = max(0, lo - half), phi = min(n - 1, hi + half);
+    const double *g = P.g + (int64_t)q * (P.td ? P.nw : n);
+    const double *rho = P.prof + ((P.td || q > 2 ? 0 : (int64_t)q * P.nb) + b) * n;
+    const double *avg = P.td && (q == 1 || q == 2) ? P.prof + ((int64_t)q * P.nb + b) * n : nullptr;
+    double v = 0;
+    // a tile of sources can matter to the time domain's bins only where
+    // 0 <= j - i < nw for some pair
+    const int s_first = P.td ? max(plo, o0) : plo;
+    const int s_last = P.td ? (int)min((int64_t)phi, (int64_t)o0 + kBlock - 1 + P.nw - 1) : phi;
+    for (int s0 = s_first; s0 <= s_last; s0 += T) {
+        const int sn = min(T, s_last - s0 + 1);
+        __syncthreads();  // the tiles before
+        if (tid < sn) pr[tid] = avg ? rho[s0 + tid] * avg[s0 + tid] : rho[s0 + tid];
+        // gt[k]: weight of the source sl of the tile in the bin ol of the
+        // block at k = ol - sl + T - 1
+        for (int k = tid; k < T + kBlock - 1; k += kBlock) {
+            const int d = o0 - s0 + k - (T - 1);  // bin - source
+            if (P.td) gt[k] = (d <= 0 && -d < P.nw) ? g[-d] : 0.0;
+            else gt[k] = g[((d % n) + n) % n];
         }
         __syncthreads();
-        // V_i = -sum_{j >= i} w[j - i] rho_j (the dipolar planes rho_j <x>_j),
-        // j over the rows of the wake and the nonzero profile (2100-2111)
-        for (int q = 0; q < 5; q++) {
-            if (!P.planes[q]) continue;
-            const double *w = P.g + (int64_t)q * P.nw;
-            const double *rho = prof[0];
-            const double *avg = (q == 1 || q == 2) ? prof[q] : nullptr;
-            double *wake = P.wake + ((int64_t)q * P.nb + b) * P.n;
-            for (int i = tid; i < P.n; i += kBlock) {
-                double v = 0;
-                const int j1 = (int)min((int64_t)phi, (int64_t)i + P.nw - 1);
-                if (avg)
-                    for (int j = max(i, plo); j <= j1; j++) v -= w[j - i] * rho[j] * avg[j];
-                else
-                    for (int j = max(i, plo); j <= j1; j++) v -= w[j - i] * rho[j];
-                wake[i] = v;
-            }
-        }
+        const double *w = gt + tid + T - 1;
+#pragma unroll 8
+        for (int sl = 0; sl < sn; sl++) v = fma(pr[sl], w[-sl], v);
     }
-    __syncthreads();
-    for (int j = lo + tid; j <= hi; j += kBlock) {
-        cnt[j] = 0u;
-        if (ds)
-            for (int c = 0; c < 4; c++) ds[4 * j + c] = 0ull;
-    }
+    if (o >= n) return;
+    if (P.td || q == 0) v = -v;
+    const int64_t at = ((int64_t)q * P.nb + b) * n + o;
+    P.wake[at] = v;
+    double k = v / P.energy / P.beta2;
+    if (q == 1 || (q == 3 && P.td)) k = k / P.bx;
+    if (q == 2 || (q == 4 && P.td)) k = k / P.by;
+    P.kick[at] = k;
 }
 
+// A block of up to 256 macroparticles of one bunch, one per thread with all
+// its loads issued at once (the kick moves 42 to 74 bytes of each and little
+// else; with four per thread in a loop and the divisions by energy, beta^2
+// and the beta functions 59.4 us on 60 bunches of 6e4, now 42).
 __global__ void __launch_bounds__(kBlock) k_bbi_kick(BbiParams P)
 {
-    const int tid = threadIdx.x;
+    const int b = P.kick_bunch[blockIdx.x];
+    const int64_t i = P.bunch_off[b] + (int64_t)(blockIdx.x - P.kick_first[b]) * kBlock + threadIdx.x;
+    if (i >= P.bunch_off[b + 1] || P.scale[b] == 0.0) return;
+    const bool dx = P.planes[1] != 0, dy = P.planes[2] != 0, qx = P.planes[3] != 0, qy = P.planes[4] != 0;
+    const uint8_t f = P.flag[i];
+    const double z = P.z[i];
+    double d = 0, px = 0, py = 0, x = 0, y = 0;
+    if (P.planes[0]) d = P.dp[i];
+    if (dx || qx) px = P.px[i];
+    if (dy || qy) py = P.py[i];
+    if (qx) x = P.x[i];
+    if (qy) y = P.y[i];
+    if (!bbi_alive(f)) return;
+    const int k = bbi_bin(z, P);
+    if (k < 0) return;
     const int64_t nbn = (int64_t)P.nb * P.n;
-    const bool tx = P.planes[1] || P.planes[3], ty = P.planes[2] || P.planes[4];
-    for (int s = P.wg_seg[blockIdx.x]; s < P.wg_seg[blockIdx.x + 1]; s++) {
-        const int b = P.seg_bunch[s];
-        if (P.scale[b] == 0.0) continue;
-        const double *wz = P.wake + (int64_t)b * P.n;
-        const double *wdx = P.wake + nbn + (int64_t)b * P.n, *wdy = P.wake + 2 * nbn + (int64_t)b * P.n;
-        const double *wqx = P.wake + 3 * nbn + (int64_t)b * P.n, *wqy = P.wake + 4 * nbn + (int64_t)b * P.n;
-        const int64_t e = P.seg_end[s], step = P.seg_step[s];
-        for (int64_t i0 = P.seg_begin[s] + tid; i0 < e; i0 += kUnroll * step) {
-            double zz[kUnroll], d[kUnroll];
-            uint8_t ff[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + u * step;
-                ff[u] = i < e ? P.flag[i] : (uint8_t)3u;
-                zz[u] = i < e ? P.z[i] : 0.0;
-                d[u] = (i < e && P.planes[0]) ? P.dp[i] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                const int64_t i = i0 + u * step;
-                if (!bbi_alive(ff[u])) continue;
-                const int k = bbi_bin(zz[u], P);
-                if (k < 0) continue;
-                if (P.planes[0]) P.dp[i] = d[u] + wz[k] / P.energy / P.beta2;
-                if (P.td) {
-                    // the time domain's order: Z, Dx, Dy, Qx, Qy
-                    // (src/MPBunch.cpp:2113-2121)
-                    if (tx) {
-                        double v = P.px[i];
-                        if (P.planes[1]) v += wdx[k] / P.energy / P.beta2 / P.bx;
-                        if (P.planes[3]) v += wqx[k] / P.energy / P.beta2 / P.bx * P.x[i];
-                        P.px[i] = v;
-                    }
-                    if (ty) {
-                        double v = P.py[i];
-                        if (P.planes[2]) v += wdy[k] / P.energy / P.beta2 / P.by;
-                        if (P.planes[4]) v += wqy[k] / P.energy / P.beta2 / P.by * P.y[i];
-                        P.py[i] = v;
-                    }
-                    continue;
-                }
-                // the frequency domain's order: Z, Qx, Qy, then Dx, Dy
-                if (tx) {
-                    double v = P.px[i];
-                    if (P.planes[3]) v += wqx[k] / P.energy / P.beta2 * P.x[i] / P.bx;
-                    if (P.planes[1]) v += wdx[k] / P.energy / P.beta2 / P.bx;
-                    P.px[i] = v;
-                }
-                if (ty) {
-                    double v = P.py[i];
-                    if (P.planes[4]) v += wqy[k] / P.energy / P.beta2 * P.y[i] / P.by;
-                    if (P.planes[2]) v += wdy[k] / P.energy / P.beta2 / P.by;
-                    P.py[i] = v;
-                }
-            }
-        }
+    const double *w = P.kick + (int64_t)b * P.n + k;
+    if (P.planes[0]) P.dp[i] = d + w[0];
+    if (P.td) {
+        // the time domain's order: Z, Dx, Dy, Qx, Qy (src/MPBunch.cpp:2113-2121)
+        if (dx) px += w[nbn];
+        if (qx) px += w[3 * nbn] * x;
+        if (dy) py += w[2 * nbn];
+        if (qy) py += w[4 * nbn] * y;
+    } else {
+        // the frequency domain's: Z, Qx, Qy, then Dx, Dy
+        if (qx) px += w[3 * nbn] * x / P.bx;
+        if (dx) px += w[nbn];
+        if (qy) py += w[4 * nbn] * y / P.by;
+        if (dy) py += w[2 * nbn];
     }
+    if (dx || qx) P.px[i] = px;
+    if (dy || qy) P.py[i] = py;
 }
 
 size_t bbi_bin_lds(bool dip)
@@ -500,20 +468,24 @@ size_t bbi_bin_lds(bool dip)
            (dip ? (size_t)4 * kBbiDipWin * sizeof(unsigned long long) : 0);
 }
 
-hipError_t launch_bbi_bin(const BbiParams &p, int nwg, hipStream_t st)
+hipError_t launch_bbi_bin(const BbiParams &p, int nitem, hipStream_t st)
 {
+    if (nitem == 0) return hipSuccess;
     const bool dip = p.planes[1] || p.planes[2];
-    hipLaunchKernelGGL(k_bbi_bin, dim3(nwg), dim3(kBlock), bbi_bin_lds(dip), st, p);
+    hipLaunchKernelGGL(k_bbi_bin, dim3(nitem), dim3(kBbiBinBlock), bbi_bin_lds(dip), st, p);
     return hipGetLastError();
 }
 hipError_t launch_bbi_wake(const BbiParams &p, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_bbi_wake, dim3(p.nb), dim3(kBlock), 0, st, p);
+    const bool dip = p.planes[1] || p.planes[2];
+    hipLaunchKernelGGL(k_bbi_prof, dim3(p.nb, dip ? 3 : 1), dim3(kBlock), 0, st, p);
+    hipLaunchKernelGGL(k_bbi_wake, dim3(p.nb, (p.n + kBlock - 1) / kBlock, 5), dim3(kBlock), 0, st, p);
     return hipGetLastError();
 }
-hipError_t launch_bbi_kick(const BbiParams &p, int nwg, hipStream_t st)
+hipError_t launch_bbi_kick(const BbiParams &p, int nitem, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_bbi_kick, dim3(nwg), dim3(kBlock), 0, st, p);
+    if (nitem == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_bbi_kick, dim3(nitem), dim3(kBlock), 0, st, p);
     return hipGetLastError();
 }
 

@@ -290,7 +290,7 @@ int lrwake_table(const cts_lrwake_config &c, double t0, int harmonic, LrwTable &
 // filter, set up on the host.
 constexpr int kBbiTaps = 51;          // the Gaussian filter's window
 constexpr int kBbiWin = 8192;         // bins of one LDS histogram window (32 KB of counts)
-constexpr int kBbiWinCopies = 2048;   // narrower ranges: one copy per wave in the same 32 KB
+constexpr int kBbiBinBlock = 256;     // threads of a binning block
 constexpr int kBbiDipWin = 1535;      // with the dipolar planes: counts and x, y limb sums (55 KB)
 constexpr int kBbiMaxGridFD = 16383;  // 2 nimp - 1 (the host forms the kernel in O(n^2))
 constexpr int kBbiMaxGridTD = 65535;  // (int)(bucket / dz)
@@ -307,23 +307,27 @@ int bbimp_table(const cts_bbimp_config &c, const cts_ring &ring, BbiTable &t, st
 struct BbiParams {
     int n, is, ie, nb, td, nw;
     int planes[5];
-    double zmin, dz, half, energy, beta2, bx, by;
-    const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg, *seg_step;
+    double zmin, dz, inv_dz, half, energy, beta2, bx, by;
+    const int64_t *bunch_off;
+    // blocks that share a bunch's particles, of the binning and of the kick
+    // (256 each): the bunch of every one, and every bunch's first
+    const int32_t *item_bunch, *item_first, *kick_bunch, *kick_first;
+    const cts_moments *cur;  // survivors' z range
     const double *x, *y, *z;
     double *px, *py, *dp;
     const uint8_t *flag;
     uint32_t *hist;        // [nb][n], zero between turns
     unsigned long long *dsum;  // [nb][n][4] x, y limb sums (dipolar planes; else null), zero between turns
     double *prof;          // [3][nb][n]: charge, x-weighted, y-weighted (time domain: charge, mean x, mean y)
-    double *wake;          // [5][nb][n], flag order
+    double *wake, *kick;   // [5][nb][n], flag order: the voltage; over energy, beta^2 (and beta function)
+    int *range;            // [nb][2] first and last bin with particles
     const double *g;       // [5][n] kernels, or [5][nw] wake table
     const double *scale;   // [nb] charge per macroparticle (frequency domain: times c / dz; 0: skipped)
     double taps[kBbiTaps];
 };
-hipError_t launch_bbi_bin(const BbiParams &p, int nwg, hipStream_t st);
+hipError_t launch_bbi_bin(const BbiParams &p, int nitem, hipStream_t st);
 hipError_t launch_bbi_wake(const BbiParams &p, hipStream_t st);
-hipError_t launch_bbi_kick(const BbiParams &p, int nwg, hipStream_t st);
+hipError_t launch_bbi_kick(const BbiParams &p, int nitem, hipStream_t st);
 
 // Host: beam-loaded cavities, tabulated per turn (cts_bl.cpp).
 // the state of a walked cavity (kBlS doubles): bin-by-bin and feedback
