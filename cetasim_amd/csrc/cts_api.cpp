@@ -159,6 +159,7 @@ struct cts_handle {
     // items of the electron-side kick (kBlock particles of one bunch each)
     int32_t *d_item_bunch = nullptr, *d_item_first = nullptr;
     int nitem = 0;
+    Stage stage;  // pinned ring of cts_download
     // blocks of the binning over the reference's edges
     int32_t *d_bin_bunch = nullptr, *d_bin_first = nullptr;
     int nbin_item = 0;
@@ -1193,6 +1194,7 @@ int cts_destroy(cts_handle *h)
     resolve_timers(h);
     graph_reset(h);
     for (hipEvent_t e : h->event_pool) (void)hipEventDestroy(e);
+    stage_free(h->stage);
     if (h->d_turn) (void)hipFree(h->d_turn);
     if (h->d_ntab) (void)hipFree(h->d_ntab);
     free_bunch_state(h);
@@ -1362,6 +1364,16 @@ int cts_download(cts_handle *h, double *x, double *px, double *y, double *py, do
     int rc = check_ready(h);
     if (rc) return rc;
     if ((rc = flush_kick(h))) return rc;
+    {
+        StageParams p{};
+        const double *src[6] = {h->d_x, h->d_px, h->d_y, h->d_py, h->d_z, h->d_dp};
+        double *const dst[6] = {x, px, y, py, z, dp};
+        std::copy(src, src + 6, p.src);
+        p.flag = h->d_flag;
+        bool done = false;
+        HIPCHK(stage_download(h->stage, p, h->ntot, dst, lost, h->stream, done));
+        if (done) return CTS_OK;
+    }
     const size_t bytes = (size_t)h->ntot * sizeof(double);
     HIPCHK(hipStreamSynchronize(h->stream));
     if (x) HIPCHK(hipMemcpy(x, h->d_x, bytes, hipMemcpyDeviceToHost));

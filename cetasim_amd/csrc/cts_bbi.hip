@@ -201,8 +201,8 @@ __host__ __device__ constexpr int bbi_count_words(bool dip) { return dip ? ((kBb
 // bunch's sums directly.  A bunch fills few bins, so the window is kept in as
 // many copies as fit, up to one per wave: the atomics of different waves do
 // not meet.  With one window of the whole grid per workgroup of the pass 37 us
-// on 60 bunches of 6e4 with both dipolar planes, 27 now (blocks of 512
-// threads 29, of 1024 40); without the planes 15 (512: 16, 1024: 22).
+// on 60 bunches of 6e4 with both dipolar planes, 31 now (blocks of 512
+// threads 30, of 1024 40); without the planes 15 (512: 16, 1024: 22).
 __global__ void __launch_bounds__(kBbiBinBlock) k_bbi_bin(BbiParams P)
 {
     extern __shared__ __attribute__((aligned(16))) uint32_t hl[];

@@ -405,6 +405,27 @@ hipError_t launch_pass(const PassParams &p, int nwg, hipStream_t st);
 // Host: the NormalTab contents (2 * kNormTab float2, sc then lg).
 void build_normal_tables(float2 *out);
 // device turn counter of graph replays: *t = v
+// The particle state on its way to the host (cts_stage.hip): a ring of
+// pinned stretches, kept by the handle.
+constexpr int64_t kStageRows = 65536;  // macroparticles of a stretch (3.4 MB)
+constexpr int kStageSlots = 2, kStageThreads = 8;
+struct Stage {
+    void *host = nullptr, *dev = nullptr;
+    int64_t rows = 0;
+    int slots = 0;
+    hipEvent_t ev[kStageSlots] = {};
+};
+struct StageParams {
+    const double *src[6];
+    const uint8_t *flag;
+    double *out;
+    int64_t i0, n, rows;
+    uint32_t want;  // bit q: coordinate q; bit 6: loss codes
+};
+void stage_free(Stage &S);
+// done: false where no pinned memory could be had and nothing was copied
+hipError_t stage_download(Stage &S, StageParams P, int64_t n, double *const coord[6], int32_t *lost, hipStream_t st,
+                          bool &done);
 hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st);
 hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_t st);
 // nitem: binning blocks (0: none)
