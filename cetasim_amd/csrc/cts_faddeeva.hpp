@@ -404,7 +404,9 @@ __device__ __forceinline__ void be_plan_store(const BeField &F, double *g)
     g[0] = (double)F.mode; g[1] = F.isx; g[2] = F.isy; g[3] = F.isig; g[4] = F.r;
     g[5] = F.ir; g[6] = F.coeff; g[7] = F.hx; g[8] = F.hy; g[9] = F.sx;
 }
-__device__ __forceinline__ BeField be_plan_load(cdptr g)
+// (g: wave-uniform, a cdptr, or per lane)
+template <typename Ptr>
+__device__ __forceinline__ BeField be_plan_load(Ptr g)
 {
     BeField F;
     F.mode = (int32_t)g[0]; F.isx = g[1]; F.isy = g[2]; F.isig = g[3]; F.r = g[4];

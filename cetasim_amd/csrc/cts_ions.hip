@@ -119,8 +119,16 @@ __device__ __forceinline__ bool ion_wave_slot(int w, int w_old, int64_t len, int
 // 1.97 ms per turn there, and 1.49, 1.40, 1.38, 1.41 on a train whose ions live
 // 12 passages; cohorts of 2 and 8 waves 2.14 and 2.31, five or six waves per
 // SIMD alike.
-template <bool SUR>
-__global__ void __launch_bounds__(kIonBlock, SUR ? 3 : kIonWavesPerEU)
+//
+// With the surrogate, FEW is for clouds of up to nine waves per SIMD by the
+// host's bound (the capacity after some turns): four blocks of the network's
+// points in flight in 143 registers.  A turn of 24 passages with 2.4e4 new
+// ions takes 205 us instead of 258, with 1.9e5 241 instead of 282, with 4.8e5
+// 448 instead of 474 and with 5.8e5 514 and 510; beyond that the waves overlap
+// each other and the smaller variant holds one more per SIMD: 807 against 844
+// us with 9.6e5.
+template <bool SUR, bool FEW>
+__global__ void __launch_bounds__(kIonBlock, SUR ? (FEW ? 2 : 3) : kIonWavesPerEU)
 k_ion_turn(IonTurnParams P)
 {
     struct NoNet {};
@@ -201,7 +209,7 @@ k_ion_turn(IonTurnParams P)
                 double fx = 0.0, fy = 0.0;
                 const BeField F = be_plan_load(bplan + q * kBePlan);
                 if constexpr (SUR) {
-                    const bool ok = sur_field(L, P.sur_norm, alive, dx, dy, bview[4 * q + 2], bview[4 * q + 3], fx, fy);
+                    const bool ok = sur_field<FEW ? 4 : 1>(L, P.sur_norm, alive, dx, dy, bview[4 * q + 2], bview[4 * q + 3], fx, fy);
                     if (alive && !ok) be_field(dx, dy, F, fx, fy);
                 } else if (alive) {
                     be_field(dx, dy, F, fx, fy);
@@ -487,10 +495,12 @@ hipError_t launch_ion_turn(const IonTurnParams &p, int nspec, int64_t wave_bound
     if (blocks > kIonTurnMaxBlocks) blocks = kIonTurnMaxBlocks;
     if (blocks < 1) blocks = 1;
     const dim3 grid((unsigned)blocks, (unsigned)nspec);
-    if (p.sur_params)
-        hipLaunchKernelGGL(k_ion_turn<true>, grid, dim3(kIonBlock), 0, st, p);
+    if (p.sur_params && wave_bound * nspec <= 9 * kSimds)
+        hipLaunchKernelGGL((k_ion_turn<true, true>), grid, dim3(kIonBlock), 0, st, p);
+    else if (p.sur_params)
+        hipLaunchKernelGGL((k_ion_turn<true, false>), grid, dim3(kIonBlock), 0, st, p);
     else
-        hipLaunchKernelGGL(k_ion_turn<false>, grid, dim3(kIonBlock), 0, st, p);
+        hipLaunchKernelGGL((k_ion_turn<false, false>), grid, dim3(kIonBlock), 0, st, p);
     return hipGetLastError();
 }
 

@@ -1033,7 +1033,7 @@ k_ion_kick_sur(IonKickParams P)
             for (int p = 0; p < P.nspec; p++) {
                 double fx = 0.0, fy = 0.0;
                 const double dx = x - c[5 * p + 1], dy = y - c[5 * p + 2];
-                const bool ok = sur_field(L, P.sur_norm, active, dx, dy, c[5 * p + 3], c[5 * p + 4], fx, fy);
+                const bool ok = sur_field<4>(L, P.sur_norm, active, dx, dy, c[5 * p + 3], c[5 * p + 4], fx, fy);
                 if (ok) {
                     fxs = fxs + c[5 * p] * fx;
                     fys = fys + c[5 * p] * fy;
@@ -1065,7 +1065,9 @@ k_ion_kick_sur(IonKickParams P)
     }
 }
 
-// Exact kicks of the queued points (the species in each entry's mask).
+// Exact kicks of the queued points (the species in each entry's mask), with
+// the cloud's field constants as the exact kick has them (the general field
+// forms its own per point: 32 us on 4.8e5 macroparticles, now 5.3).
 __global__ void __launch_bounds__(kBlock)
 k_ion_kick_fb(IonKickParams P)
 {
@@ -1081,12 +1083,13 @@ k_ion_kick_fb(IonKickParams P)
             else hi = mid;
         }
         const double *c = P.ion_e + (int64_t)lo * CTS_MAX_SPECIES * 5;
+        const double *g = P.ion_f + (int64_t)lo * CTS_MAX_SPECIES * kBePlan;
         const double x = P.x[i], y = P.y[i];
         double fxs = 0.0, fys = 0.0;
         for (int p = 0; p < P.nspec; p++) {
             if (!(mask & (1u << p))) continue;
             double fx, fy;
-            ion_field(x - c[5 * p + 1], y - c[5 * p + 2], c[5 * p + 3], c[5 * p + 4], fx, fy);
+            be_field(x - c[5 * p + 1], y - c[5 * p + 2], be_plan_load(g + p * kBePlan), fx, fy);
             fxs = fxs + c[5 * p] * fx;
             fys = fys + c[5 * p] * fy;
         }

@@ -144,6 +144,10 @@ __device__ __forceinline__ void load_mlp_lds(MlpLds &L, const float *W, int tid,
     if (tid == 0) { L.b3[0] = W[MP_B3]; L.b3[1] = W[MP_B3 + 1]; }
 }
 
+// UNROLL blocks of 16 points are in flight at a time: four let a wave that has
+// its SIMD to itself overlap the chains of one with those of the next, for 15
+// more registers.
+template <int UNROLL = 1>
 __device__ __forceinline__ void mlp_forward_wave(const MlpLds &L, float a0, float a1, float a2, float &out0,
                                                  float &out1)
 {
@@ -151,7 +155,7 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpLds &L, float a0, floa
     const int l = threadIdx.x & 63;
     const int lr = l & 15, lg = (l >> 4) & 3;
     float q0 = 0.0f, q1 = 0.0f;
-#pragma unroll 1
+#pragma unroll UNROLL
     for (int nb = 0; nb < 4; nb++) {
         // first layer for samples s = 16 nb + lr in the B layout: features
         // k = 32 kb + 8 lg + i
@@ -218,6 +222,7 @@ struct SurNorm { float mx, sx, my, sy; };
 // its domain; returns false for the other lanes (and for inactive lanes),
 // which take the exact path.  Every lane of the wave must call it: the
 // network runs on the whole wave's points at once.
+template <int UNROLL>
 __device__ __forceinline__ bool sur_field(const MlpLds &L, const SurNorm &nm, bool active, double x, double y,
                                           double sx, double sy, double &fx, double &fy)
 {
@@ -233,7 +238,7 @@ __device__ __forceinline__ bool sur_field(const MlpLds &L, const SurNorm &nm, bo
     float a[3];
     sur_features(dom ? au : 1.0, dom ? av : 1.0, dom ? r : 0.5, a);
     float o0, o1;
-    mlp_forward_wave(L, a[0], a[1], a[2], o0, o1);
+    mlp_forward_wave<UNROLL>(L, a[0], a[1], a[2], o0, o1);
     if (!dom) return false;
     float bx, by;
     sur_envelope((float)au, (float)av, (float)r, bx, by);
