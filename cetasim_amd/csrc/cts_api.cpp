@@ -311,14 +311,12 @@ void free_bunch_state(cts_handle *h)
     free_bl_state(h);
     free_bbi_state(h);
     void *ptrs[] = {h->d_x, h->d_px, h->d_y, h->d_py, h->d_z, h->d_dp, h->d_flag,
-                    h->d_seg_begin, h->d_seg_end, h->d_bunch_off, h->d_bunch_count,
-                    h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part, h->d_shift,
+                    h->d_seg_begin, h->d_bunch_off, h->d_bunch_count, h->d_seg_part, h->d_shift,
                     h->d_cur, h->d_hist, h->d_sigz, h->d_zrange, h->d_noise, h->d_ion_e, h->d_ion_bview,
-                    h->d_ion_f, h->d_ion_bplan, h->d_item_bunch, h->d_item_first,
-                    h->d_bin_bunch, h->d_bin_first,
+                    h->d_ion_f, h->d_item_bunch,
                     h->d_bhist, h->d_counts, h->d_kick, h->d_poten, h->d_edges_prev,
                     h->d_edges_now, h->d_table, h->d_scale, h->d_terms,
-                    h->d_fb_count, h->d_fb_list, h->d_eig, h->d_seg_rank, h->d_seg_order, h->d_seg_step};
+                    h->d_fb_count, h->d_fb_list, h->d_eig};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     h->d_eig = nullptr;
@@ -854,42 +852,45 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
         std::vector<int32_t> next(wgseg.begin(), wgseg.end() - 1);
         for (int s = 0; s < nseg; s++) rank[next[segs[s].wg]++] = s;
     }
-    std::vector<int64_t> sb(nseg), se(nseg);
-    std::vector<int32_t> sbunch(nseg), sstep(nseg);
-    for (int s = 0; s < nseg; s++) {
-        const Seg &g = segs[rank[s]];
-        sb[s] = g.begin;
-        se[s] = g.end;
-        sbunch[s] = g.bunch;
-        sstep[s] = g.step;
-    }
+    // the tables in one block: begin and end (64 bits), then step, bunch, the
+    // workgroups' and the bunches' first segments, and (unless the order of
+    // the segments is the particles') rank and order
     bool identity = true;
     for (int s = 0; s < nseg && identity; s++) identity = rank[s] == s;
-    void *old[] = {h->d_seg_begin, h->d_seg_end, h->d_seg_bunch, h->d_wg_seg, h->d_bunch_seg, h->d_seg_part,
-                   h->d_seg_rank, h->d_seg_order, h->d_seg_step};
-    for (void *p : old)
-        if (p) (void)hipFree(p);
+    const size_t words = 2 * (size_t)nseg + nwg + 1 + nb + 1 + (identity ? 0 : 2 * (size_t)nseg);
+    std::vector<int64_t> block(2 * (size_t)nseg + (words + 1) / 2);
+    int32_t *w32 = reinterpret_cast<int32_t *>(block.data() + 2 * (size_t)nseg);
+    for (int s = 0; s < nseg; s++) {
+        const Seg &g = segs[rank[s]];
+        block[s] = g.begin;
+        block[nseg + s] = g.end;
+        w32[s] = g.step;
+        w32[nseg + s] = g.bunch;
+    }
+    std::copy(wgseg.begin(), wgseg.end(), w32 + 2 * (size_t)nseg);
+    std::copy(bseg.begin(), bseg.end(), w32 + 2 * (size_t)nseg + nwg + 1);
+    int32_t *r32 = w32 + 2 * (size_t)nseg + nwg + 1 + nb + 1;
+    for (int s = 0; s < nseg && !identity; s++) {
+        r32[s] = rank[s];
+        r32[nseg + rank[s]] = s;
+    }
+    if (h->d_seg_begin) (void)hipFree(h->d_seg_begin);
+    if (h->d_seg_part) (void)hipFree(h->d_seg_part);
     h->d_seg_begin = h->d_seg_end = nullptr;
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = h->d_seg_rank = h->d_seg_order = h->d_seg_step = nullptr;
     h->d_seg_part = nullptr;
     int rc;
-    if ((rc = dalloc(&h->d_seg_begin, nseg)) || (rc = dalloc(&h->d_seg_end, nseg)) ||
-        (rc = dalloc(&h->d_seg_bunch, nseg)) || (rc = dalloc(&h->d_seg_step, nseg)) || (rc = dalloc(&h->d_wg_seg, nwg + 1)) ||
-        (rc = dalloc(&h->d_bunch_seg, nb + 1)) || (rc = dalloc(&h->d_seg_part, (size_t)nseg * kNPart)) ||
-        (!identity && ((rc = dalloc(&h->d_seg_rank, nseg)) || (rc = dalloc(&h->d_seg_order, nseg)))))
-        return rc;
+    if ((rc = dalloc(&h->d_seg_begin, block.size())) || (rc = dalloc(&h->d_seg_part, (size_t)nseg * kNPart))) return rc;
+    HIPCHK(hipMemcpy(h->d_seg_begin, block.data(), block.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    h->d_seg_end = h->d_seg_begin + nseg;
+    h->d_seg_step = reinterpret_cast<int32_t *>(h->d_seg_end + nseg);
+    h->d_seg_bunch = h->d_seg_step + nseg;
+    h->d_wg_seg = h->d_seg_bunch + nseg;
+    h->d_bunch_seg = h->d_wg_seg + nwg + 1;
     if (!identity) {
-        std::vector<int32_t> order(nseg);
-        for (int sg = 0; sg < nseg; sg++) order[rank[sg]] = sg;
-        HIPCHK(hipMemcpy(h->d_seg_rank, rank.data(), rank.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(h->d_seg_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        h->d_seg_rank = h->d_bunch_seg + nb + 1;
+        h->d_seg_order = h->d_seg_rank + nseg;
     }
-    HIPCHK(hipMemcpy(h->d_seg_begin, sb.data(), sb.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->d_seg_end, se.data(), se.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->d_seg_step, sstep.data(), sstep.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->d_seg_bunch, sbunch.data(), sbunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->d_wg_seg, wgseg.data(), wgseg.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(h->d_bunch_seg, bseg.data(), bseg.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     h->nwg = nwg;
     h->nseg = nseg;
     h->tile = tile;
@@ -1247,30 +1248,33 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
     if ((rc = layout_segments(h, h->wg_target, h->tile))) return rc;
     // items of kernels that split the bunches themselves: the electron-side
     // ion kick (a block of particles each) and the binning
-    const auto cut_items = [&](auto items_of, int32_t **d_bunch, int32_t **d_first, int *count) -> int {
-        std::vector<int32_t> first(nb + 1, 0), bunch;
+    std::vector<int32_t> items;  // bunch of every item, every bunch's first, for both
+    const auto cut_items = [&](auto items_of, int *count) -> bool {
+        std::vector<int32_t> first(nb + 1, 0);
         for (int b = 0; b < nb; b++) {
-            const int64_t items = items_of(counts[b]);
-            if (first[b] + items > INT32_MAX / 2) return fail(CTS_ERR_ARG, "cts_set_bunches: too many particles");
-            first[b + 1] = first[b] + (int32_t)items;
-            bunch.insert(bunch.end(), (size_t)items, b);
+            const int64_t m = items_of(counts[b]);
+            if (first[b] + m > INT32_MAX / 2) return false;
+            first[b + 1] = first[b] + (int32_t)m;
+            items.insert(items.end(), (size_t)m, b);
         }
         *count = first[nb];
-        int r;
-        if ((r = dalloc(d_bunch, bunch.size())) || (r = dalloc(d_first, first.size()))) return r;
-        HIPCHK(hipMemcpy(*d_bunch, bunch.data(), bunch.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(*d_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-        return CTS_OK;
+        items.insert(items.end(), first.begin(), first.end());
+        return true;
     };
     const auto kick_items = [](int64_t n) { return (n + kBlock - 1) / kBlock; };
     const auto bin_items = [](int64_t n) {
         return std::min(std::max(kBinBlocks, n / kBinMax), (n + kBinMin - 1) / kBinMin);
     };
-    if ((rc = cut_items(kick_items, &h->d_item_bunch, &h->d_item_first, &h->nitem)) ||
-        (rc = cut_items(bin_items, &h->d_bin_bunch, &h->d_bin_first, &h->nbin_item)) ||
-        (rc = dalloc(&h->d_ion_f, (size_t)nb * CTS_MAX_SPECIES * kBePlan)) ||
-        (rc = dalloc(&h->d_ion_bplan, (size_t)nb * kBePlan)))
+    if (!cut_items(kick_items, &h->nitem) || !cut_items(bin_items, &h->nbin_item))
+        return fail(CTS_ERR_ARG, "cts_set_bunches: too many particles");
+    if ((rc = dalloc(&h->d_item_bunch, items.size())) ||
+        (rc = dalloc(&h->d_ion_f, (size_t)nb * (CTS_MAX_SPECIES + 1) * kBePlan)))
         return rc;
+    h->d_item_first = h->d_item_bunch + h->nitem;
+    h->d_bin_bunch = h->d_item_first + nb + 1;
+    h->d_bin_first = h->d_bin_bunch + h->nbin_item;
+    h->d_ion_bplan = h->d_ion_f + (size_t)nb * CTS_MAX_SPECIES * kBePlan;
+    HIPCHK(hipMemcpy(h->d_item_bunch, items.data(), items.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_off, h->offsets.data(), (nb + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_count, h->counts.data(), nb * sizeof(int64_t), hipMemcpyHostToDevice));
     h->kick_pending = false;
