@@ -797,7 +797,8 @@ void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int reside
     if (strided) {
         int64_t blocks = 0;
         for (int b = 0; b < nb; b++) blocks += (off[b + 1] - off[b] + kBlock - 1) / kBlock;
-        nwg = (int)std::max<int64_t>(1, std::min<int64_t>(wg, blocks));
+        // a stride below 2^31 (then a workgroup has a block of a bunch at most)
+        nwg = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(wg, INT32_MAX / kBlock), blocks));
         int64_t first = 0;  // the next bunch starts at the workgroup the last one stopped at
         for (int b = 0; b < nb; b++) {
             const int64_t nblk = (off[b + 1] - off[b] + kBlock - 1) / kBlock;
@@ -2660,6 +2661,29 @@ int cts_kernel_time(cts_handle *h, const char *name, double *avg_ms, int64_t *la
     }
     if (avg_ms) *avg_ms = it->second.total_ms / (double)it->second.n;
     if (launches) *launches = it->second.n;
+    return CTS_OK;
+}
+
+int cts_debug_layout(int32_t nb, const int64_t *counts, int32_t nwg, int32_t tile, int32_t ncu, int64_t *nseg,
+                     int64_t *begin, int64_t *end, int32_t *step, int32_t *bunch, int32_t *wg)
+{
+    if (nb < 1 || !counts || nwg < 0 || tile < 0 || ncu < 1 || !nseg || !begin || !end || !step || !bunch || !wg)
+        return fail(CTS_ERR_ARG, "cts_debug_layout");
+    std::vector<int64_t> off(nb + 1, 0);
+    for (int b = 0; b < nb; b++) off[b + 1] = off[b] + counts[b];
+    std::vector<Seg> segs;
+    int n = 1;
+    cut_segments(off, nwg, tile, kPassPerCu * ncu, segs, n);
+    const int64_t room = *nseg;
+    *nseg = (int64_t)segs.size();
+    if (*nseg > room) return fail(CTS_ERR_ARG, "cts_debug_layout: more segments than room (count returned)");
+    for (int64_t s = 0; s < *nseg; s++) {
+        begin[s] = segs[s].begin;
+        end[s] = segs[s].end;
+        step[s] = segs[s].step;
+        bunch[s] = segs[s].bunch;
+        wg[s] = segs[s].wg;
+    }
     return CTS_OK;
 }
 

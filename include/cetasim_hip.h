@@ -446,6 +446,13 @@ int cts_debug_faddeeva(cts_handle *h, int64_t n, const double *re, const double 
  * branches, src/MPBunch.cpp:1128-1147, per unit line charge) at n points:
  * in = {x[n], y[n], sx[n], sy[n]}, out = {fx[n], fy[n]}. */
 int cts_debug_kick_field(cts_handle *h, int64_t n, const double *in, double *out);
+/* Test hook: the segment table that a layout (cts_set_layout; nwg 0: the
+ * default one) of bunches of counts[b] macroparticles gets on a device of ncu
+ * compute units, no device needed.  *nseg in: room in the arrays, out: segments;
+ * segment s is the blocks of 256 macroparticles that start at begin, begin +
+ * step, ... below end, all of one bunch, walked by workgroup wg. */
+int cts_debug_layout(int32_t nb, const int64_t *counts, int32_t nwg, int32_t tile, int32_t ncu, int64_t *nseg,
+                     int64_t *begin, int64_t *end, int32_t *step, int32_t *bunch, int32_t *wg);
 /* Test hook: the device quantum-excitation stream for particles
  * [base, base+n) at `turn` (noise_out[5][n]). */
 int cts_debug_qe_normals(cts_handle *h, uint64_t seed, int32_t turn, uint64_t base,
