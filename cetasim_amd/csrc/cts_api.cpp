@@ -750,7 +750,7 @@ struct Seg {
 //  wg == 0 (the default), by what the 256-CU device measured (us per pass):
 //    one bunch: blocks of 256 round-robin over the resident workgroups, which
 //    streams in grid-stride order (1e7 macroparticles: 246 as 1024 chunks,
-//    235); few particles: equal pieces of whole blocks that never cross a
+//    235), chunks where the stride's 32-bit offsets end; few particles: equal pieces of whole blocks that never cross a
 //    bunch (a workgroup with two segments takes twice the latency where a
 //    segment is one block); up to 6144 per resident workgroup, one chunk each
 //    (3.5e6 in 60 bunches: 112 over 1024 workgroups, 97); above, a workgroup
@@ -770,7 +770,7 @@ void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int reside
         wg = resident;
         tile = 0;
         least = kBlock;
-        if (nb == 1) tile = kBlock;
+        if (nb == 1) tile = n < (int64_t)1 << 31 ? kBlock : 0;
         else if (nb <= resident / 8 && n <= (int64_t)resident * 1024) {
             int64_t piece = std::max<int64_t>(1, (n + wg - 1) / wg);
             int64_t total;

@@ -48,3 +48,12 @@ def check_walk(counts, begin, end, step, bunch, wg):
     ([1_200_000_000] * 2, 2**31 - 1, 256), ([1_200_000_000, 2_100_000_000, 1000], 1 << 24, 256)])
 def test_every_macroparticle_once(counts, nwg, tile):
     check_walk(counts, *segments(counts, nwg, tile))
+
+
+@pytest.mark.parametrize("n", [2**31 - 1, 2**31, 4_500_000_000])
+def test_one_bunch_in_few_segments(n):
+    """The default layout of one bunch: a segment per resident workgroup (a
+    prologue and a reduction each), also beyond the strided layout's reach."""
+    t = segments([n])
+    check_walk([n], *t)
+    assert len(t[0]) <= 1024
