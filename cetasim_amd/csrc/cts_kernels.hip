@@ -1214,8 +1214,11 @@ hipError_t launch_eigen_sums(const double *x, const double *px, const double *y,
 // the next pass.  Each source is a chain of a few loads and a division, so
 // the turns go to the block's 16 waves and the bunches of a turn to the lanes
 // (with the turns one after another on 256 threads 22.9 us for 80 bunches and
-// 21 turns, now 6.3); the partial sums are folded in a fixed order.
-constexpr int kLrWaves = 16;
+// 21 turns, now 6.3), those of fewer turns than half the waves to the lanes of
+// several waves (480 bunches and 1, 3, 5 turns: 11.4, 14.5, 15.2 us with a wave
+// each, 6.6, 9.6, 12.0; 700 and 3: 23.4, 11.1); the partial sums are folded in
+// a fixed order.
+constexpr int kLrWaves = 16, kLrWholeBlocks = 2 * 256;
 __global__ void __launch_bounds__(64 * kLrWaves)
 k_lrwake(LrwParams P)
 {
@@ -1228,13 +1231,14 @@ k_lrwake(LrwParams P)
     const int hj = P.harm[j];
     double f0 = 0.0, f1 = 0.0, f2 = 0.0;
     bool ahead = false;
-    for (int n = wave; n < T; n += kLrWaves) {
+    const int waves = blockDim.x / 64, per_turn = T < waves ? waves / T : 1, sub = wave % per_turn;
+    for (int n = wave / per_turn; n < T; n += waves / per_turn) {
         int i0 = 0, i1 = nb - 1;
         if (n == 0) i1 = j - 1;
         else if (n == T - 1) i0 = j;
         const int slot = now >= n ? now - n : now - n + T;
         const double *pn = n == 0 ? P.cen : P.ring + (int64_t)slot * nb * 3;
-        for (int i = i0 + lane; i <= i1; i += 64) {
+        for (int i = i0 + sub * 64 + lane; i <= i1; i += per_turn * 64) {
             const int ntau = P.harm[i] - hj - n * P.harmonic;
             const double tau = ntau * P.trf + (zj - pn[3 * i + 2]) / kClight / P.rbeta;
             if (tau > 0) {
@@ -1266,7 +1270,7 @@ k_lrwake(LrwParams P)
     if (tid < 3) {
         P.ring[(int64_t)now * nb * 3 + 3 * j + tid] = P.cen[3 * j + tid];
         double f = 0;
-        for (int w = 0; w < kLrWaves; w++) f += red[tid][w];
+        for (int w = 0; w < waves; w++) f += red[tid][w];
         f *= P.scale;
         P.kick[3 * j + tid] = f;
         // px, py and (fix_dp) dp means
@@ -1279,7 +1283,14 @@ k_lrwake(LrwParams P)
 }
 hipError_t launch_lrwake(const LrwParams &p, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_lrwake, dim3(p.nb), dim3(64 * kLrWaves), 0, st, p);
+    // few turns: no more waves than shares of 64 bunches, and half a block where
+    // the device would hold two whole ones per compute unit and need more
+    int waves = kLrWaves;
+    if (p.nturns < kLrWaves / 2) {
+        const int share = (p.nb + 63) / 64;
+        waves = std::min(p.nb > kLrWholeBlocks ? kLrWaves / 2 : kLrWaves, std::max(4, p.nturns * share));
+    }
+    hipLaunchKernelGGL(k_lrwake, dim3(p.nb), dim3(64 * waves), 0, st, p);
     return hipGetLastError();
 }
 

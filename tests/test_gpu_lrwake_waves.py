@@ -35,3 +35,10 @@ def test_split_of_the_long_range_sum(nb, nturns):
     for b in range(nb):
         assert np.array_equal(h[b]["mean"][[1, 3]], m[b]["mean"][[1, 3]])
     tr.close()
+
+
+@pytest.mark.parametrize("nb,nturns", [(150, 1), (150, 3), (90, 5), (70, 7), (64, 9)])
+def test_several_waves_for_a_turn(nb, nturns):
+    """Fewer turns than half the waves: the bunches of a turn over the lanes
+    of several waves, with waves left over, in blocks of 4 to 16 waves."""
+    test_split_of_the_long_range_sum(nb, nturns)
