@@ -423,7 +423,8 @@ struct StageParams {
     uint32_t want;  // bit q: coordinate q; bit 6: loss codes
 };
 void stage_free(Stage &S);
-// done: false where no pinned memory could be had and nothing was copied
+// done: false where nothing was copied (no pinned memory to be had, no arrays, or
+// so few that direct copies are faster)
 hipError_t stage_download(Stage &S, StageParams P, int64_t n, double *const coord[6], int32_t *lost, hipStream_t st,
                           bool &done);
 hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st);

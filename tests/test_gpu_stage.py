@@ -35,3 +35,25 @@ def test_download_at_the_edges_of_a_stretch():
         assert np.array_equal(only, lost)
         capi.check(tr.lib.cts_download(tr.h, *[None] * 7))
     tr.close()
+
+
+def test_download_of_few_arrays():
+    """One and two arrays on both sides of the sizes from which they are copied
+    directly (131 072 and 262 144 macroparticles), with and without loss codes."""
+    ring, secs, _ = configs.lattice()
+    tr = Tracker(ring, secs)
+    rng = np.random.default_rng(6)
+    for n in (131_072, 131_073, 262_144, 262_145):
+        print(f"few arrays of {n}", flush=True)
+        q, ne = configs.bunch_scalars([n], ring)
+        tr.set_bunches([n], q, ne)
+        parts = {c: rng.standard_normal(n) for c in COORDS}
+        lost = rng.integers(0, 3, n).astype(np.int32)
+        tr.upload(parts, lost)
+        for names in (("z",), ("x", "dp"), ("px", "lost"), ("y", "py", "lost")):
+            out = {c: np.full(n, -7, np.int32 if c == "lost" else np.float64) for c in names}
+            args = [capi.dptr(out[c]) if c in out else None for c in COORDS]
+            capi.check(tr.lib.cts_download(tr.h, *args, capi.i32ptr(out["lost"]) if "lost" in out else None))
+            for c in names:
+                assert np.array_equal(out[c], lost if c == "lost" else parts[c]), c
+    tr.close()
