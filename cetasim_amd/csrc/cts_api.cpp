@@ -114,6 +114,9 @@ struct cts_handle {
     int32_t *d_seg_step = nullptr;
     int32_t *d_seg_order = nullptr;  // inverse of d_seg_rank: the segment at each place in particle order
     double *d_seg_part = nullptr;
+    int nfold = 0;                 // groups of segments (0: no bunch has many)
+    int32_t *d_fold_seg = nullptr, *d_fold_first = nullptr;  // a group's, a bunch's first
+    double *d_fold_part = nullptr;
 
     // moments
     double *d_shift = nullptr;
@@ -320,7 +323,9 @@ void free_bunch_state(cts_handle *h)
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     h->d_eig = nullptr;
-    h->d_seg_rank = h->d_seg_order = h->d_seg_step = nullptr;
+    h->d_seg_rank = h->d_seg_order = h->d_seg_step = h->d_fold_seg = h->d_fold_first = nullptr;
+    h->d_fold_part = nullptr;
+    h->nfold = 0;
     h->eig_cap = 0;
     h->d_x = h->d_px = h->d_y = h->d_py = h->d_z = h->d_dp = nullptr;
     h->d_flag = nullptr;
@@ -580,8 +585,30 @@ int run_pass(cts_handle *h, const PassParams &p, const char *name = "pass")
     return CTS_OK;
 }
 
-int run_finalize(cts_handle *h, const FinParams &f)
+// What closes the turn reads the partial sums of all of a bunch's segments (the
+// blocks of k_close each for themselves): many are first folded in groups.
+int run_fold(cts_handle *h, FinParams &f)
 {
+    if (h->nfold == 0) return CTS_OK;
+    FoldParams p;
+    p.seg_part = f.seg_part;
+    p.fold_seg = h->d_fold_seg;
+    p.out = h->d_fold_part;
+    p.nseg = h->nseg;
+    p.ngroup = h->nfold;
+    p.ops = f.ops;
+    f.seg_part = h->d_fold_part;
+    f.bunch_seg = h->d_fold_first;
+    f.nseg = h->nfold;
+    TimedScope ts(h, "fold");
+    HIPCHK(launch_fold(p, h->stream));
+    return CTS_OK;
+}
+
+int run_finalize(cts_handle *h, FinParams f)
+{
+    int rc = run_fold(h, f);
+    if (rc) return rc;
     TimedScope ts(h, "finalize");
     HIPCHK(launch_finalize(f, h->stream));
     return CTS_OK;
@@ -635,7 +662,11 @@ int run_close(cts_handle *h, const FinParams *f)
 {
     CloseParams c;
     std::memset(&c, 0, sizeof c);
-    if (f) c.f = *f;
+    if (f) {
+        c.f = *f;
+        const int rc = run_fold(h, c.f);
+        if (rc) return rc;
+    }
     c.fin = f != nullptr;
     c.edges_given = f == nullptr;
     c.edges_now = h->d_edges_now;
@@ -853,12 +884,26 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
         std::vector<int32_t> next(wgseg.begin(), wgseg.end() - 1);
         for (int s = 0; s < nseg; s++) rank[next[segs[s].wg]++] = s;
     }
+    // groups of segments, where a bunch has many
+    std::vector<int32_t> fold;
+    int nfold = 0, most = 0;
+    for (int b = 0; b < nb; b++) most = std::max(most, bseg[b + 1] - bseg[b]);
+    if (most > kFoldFrom) {
+        std::vector<int32_t> first(nb + 1);
+        for (int b = 0; b < nb; b++) {
+            first[b] = (int32_t)fold.size();
+            for (int s = bseg[b]; s < bseg[b + 1]; s += kFoldGroup) fold.push_back(s);
+        }
+        first[nb] = nfold = (int)fold.size();
+        fold.push_back(nseg);
+        fold.insert(fold.end(), first.begin(), first.end());
+    }
     // the tables in one block: begin and end (64 bits), then step, bunch, the
-    // workgroups' and the bunches' first segments, and (unless the order of
-    // the segments is the particles') rank and order
+    // workgroups' and the bunches' first segments, the groups, and (unless the
+    // order of the segments is the particles') rank and order
     bool identity = true;
     for (int s = 0; s < nseg && identity; s++) identity = rank[s] == s;
-    const size_t words = 2 * (size_t)nseg + nwg + 1 + nb + 1 + (identity ? 0 : 2 * (size_t)nseg);
+    const size_t words = 2 * (size_t)nseg + nwg + 1 + nb + 1 + fold.size() + (identity ? 0 : 2 * (size_t)nseg);
     std::vector<int64_t> block(2 * (size_t)nseg + (words + 1) / 2);
     int32_t *w32 = reinterpret_cast<int32_t *>(block.data() + 2 * (size_t)nseg);
     for (int s = 0; s < nseg; s++) {
@@ -871,6 +916,7 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
     std::copy(wgseg.begin(), wgseg.end(), w32 + 2 * (size_t)nseg);
     std::copy(bseg.begin(), bseg.end(), w32 + 2 * (size_t)nseg + nwg + 1);
     int32_t *r32 = w32 + 2 * (size_t)nseg + nwg + 1 + nb + 1;
+    r32 = std::copy(fold.begin(), fold.end(), r32);
     for (int s = 0; s < nseg && !identity; s++) {
         r32[s] = rank[s];
         r32[nseg + rank[s]] = s;
@@ -879,17 +925,26 @@ int layout_segments(cts_handle *h, int wg_target, int tile)
     if (h->d_seg_part) (void)hipFree(h->d_seg_part);
     h->d_seg_begin = h->d_seg_end = nullptr;
     h->d_seg_bunch = h->d_wg_seg = h->d_bunch_seg = h->d_seg_rank = h->d_seg_order = h->d_seg_step = nullptr;
-    h->d_seg_part = nullptr;
+    h->d_seg_part = h->d_fold_part = nullptr;
+    h->d_fold_seg = h->d_fold_first = nullptr;
     int rc;
-    if ((rc = dalloc(&h->d_seg_begin, block.size())) || (rc = dalloc(&h->d_seg_part, (size_t)nseg * kNPart))) return rc;
+    if ((rc = dalloc(&h->d_seg_begin, block.size())) ||
+        (rc = dalloc(&h->d_seg_part, (size_t)(nseg + nfold) * kNPart)))
+        return rc;
     HIPCHK(hipMemcpy(h->d_seg_begin, block.data(), block.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     h->d_seg_end = h->d_seg_begin + nseg;
     h->d_seg_step = reinterpret_cast<int32_t *>(h->d_seg_end + nseg);
     h->d_seg_bunch = h->d_seg_step + nseg;
     h->d_wg_seg = h->d_seg_bunch + nseg;
     h->d_bunch_seg = h->d_wg_seg + nwg + 1;
+    h->nfold = nfold;
+    if (nfold > 0) {
+        h->d_fold_seg = h->d_bunch_seg + nb + 1;
+        h->d_fold_first = h->d_fold_seg + nfold + 1;
+        h->d_fold_part = h->d_seg_part + (size_t)nseg * kNPart;
+    }
     if (!identity) {
-        h->d_seg_rank = h->d_bunch_seg + nb + 1;
+        h->d_seg_rank = h->d_bunch_seg + nb + 1 + fold.size();
         h->d_seg_order = h->d_seg_rank + nseg;
     }
     h->nwg = nwg;
@@ -1614,6 +1669,7 @@ static int turn_body(cts_handle *h, int32_t turn)
     if (h->capturing && h->cap_off == 1) f.advance = h->d_turn;
     if (wake && h->wake_mode == 1) {
         // fixed grid: moments and wake in one launch
+        if ((rc = run_fold(h, f))) return rc;
         TimedScope ts(h, "post");
         HIPCHK(launch_post(f, wake_params(h), h->stream));
         h->hist_parity = 1 - h->hist_parity;

@@ -259,6 +259,22 @@ struct FinParams {
     double *lr_cen;       // [nb][3] post-map centroids (OP_LRC)
 };
 
+// Partial sums of kFoldGroup segments at a time, between the pass and the
+// kernels that close the turn, where a bunch has more than kFoldFrom segments.
+// Those kernels read all of a bunch's sums in one block, k_close in each of its
+// blocks, whose number grows with the bunch too.  Without / with the fold (6 to
+// 7 us of it) in us, k_post and k_close: 1220 segments 10.5 and 32; 2441 of 1e7
+// macroparticles 14.6 / 13, 37 / 36; 4883 22.6 / 13.5, 48 / 37; 12 207 of 1e8
+// 49 / 13, 858 / 375; 48 829 of 4e8 172 / 14, 4912 / 654.
+constexpr int kFoldGroup = 256, kFoldFrom = 2048;
+struct FoldParams {
+    const double *seg_part;   // [kNPart][nseg]
+    const int32_t *fold_seg;  // [ngroup + 1] the groups' first segments, in particle order
+    double *out;              // [kNPart][ngroup]
+    int32_t nseg, ngroup;
+    uint32_t ops;
+};
+
 // MPBeam::LRWakeBeamIntaction for one turn: one block per receiving bunch.
 struct LrwParams {
     const double *table;   // [3][np] W_x, W_y, W_z at tau = -i dt
@@ -432,6 +448,7 @@ hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_
 // nitem: binning blocks (0: none)
 hipError_t launch_close(CloseParams c, int nitem, hipStream_t st);
 hipError_t launch_ion_kick(const IonKickParams &p, int nwg, hipStream_t st);
+hipError_t launch_fold(const FoldParams &p, hipStream_t st);
 hipError_t launch_finalize(const FinParams &p, hipStream_t st);
 hipError_t launch_post(const FinParams &f, const WakeParams &w, hipStream_t st);
 hipError_t launch_wake(const WakeParams &p, int nb, hipStream_t st);

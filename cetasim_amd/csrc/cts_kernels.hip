@@ -668,6 +668,20 @@ __device__ __forceinline__ void fold_parts(const FinParams &P, int s0, int s1, i
     }
 }
 
+// A group of segments to one partial sum each (kFoldGroup: one round of the
+// loads of fold_parts).
+__global__ void __launch_bounds__(kPostBlock) k_fold(FoldParams P)
+{
+    __shared__ double tot[kNPart + 2];
+    FinParams F;
+    F.seg_part = P.seg_part;
+    F.nseg = P.nseg;
+    const int g = blockIdx.x, tid = threadIdx.x;
+    fold_parts(F, P.fold_seg[g], P.fold_seg[g + 1], 4 * (tid >> 6), P.ops, tot);
+    __syncthreads();
+    if (tid < kNPart && part_needed(P.ops, tid)) P.out[(int64_t)tid * P.ngroup + g] = tot[tid];
+}
+
 // The reference's bin edges from the survivors' z range and rms after the
 // pass (src/MPBunch.cpp:1900-1908): {lo, width}.
 __device__ __forceinline__ void ref_edges(const double *tot, int nbins, double &sig, double &lo, double &dz)
@@ -1563,6 +1577,11 @@ hipError_t launch_close(CloseParams c, int nitem, hipStream_t st)
     c.tab_blocks = (2 * c.t.nbins - 1 + kPostWaves - 1) / kPostWaves;
     const int64_t grid = (int64_t)(c.fin ? c.nb : 0) + (int64_t)c.tables * c.tab_blocks + nitem;
     hipLaunchKernelGGL(k_close, dim3((unsigned)grid), dim3(kPostBlock), (size_t)c.t.nbins * sizeof(uint32_t), st, c);
+    return hipGetLastError();
+}
+hipError_t launch_fold(const FoldParams &p, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_fold, dim3(p.ngroup), dim3(kPostBlock), 0, st, p);
     return hipGetLastError();
 }
 hipError_t launch_finalize(const FinParams &p, hipStream_t st)
