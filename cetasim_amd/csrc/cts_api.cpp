@@ -1304,33 +1304,35 @@ int cts_set_bunches(cts_handle *h, int32_t nb, const int64_t *counts, const doub
     if ((rc = layout_segments(h, h->wg_target, h->tile))) return rc;
     // items of kernels that split the bunches themselves: the electron-side
     // ion kick (a block of particles each) and the binning
-    std::vector<int32_t> items;  // bunch of every item, every bunch's first, for both
-    const auto cut_items = [&](auto items_of, int *count) -> bool {
-        std::vector<int32_t> first(nb + 1, 0);
+    const auto cut_items = [&](auto items_of, std::vector<int32_t> &first) -> bool {
+        first.assign(nb + 1, 0);
         for (int b = 0; b < nb; b++) {
             const int64_t m = items_of(counts[b]);
             if (first[b] + m > INT32_MAX / 2) return false;
             first[b + 1] = first[b] + (int32_t)m;
-            items.insert(items.end(), (size_t)m, b);
         }
-        *count = first[nb];
-        items.insert(items.end(), first.begin(), first.end());
         return true;
     };
     const auto kick_items = [](int64_t n) { return (n + kBlock - 1) / kBlock; };
     const auto bin_items = [](int64_t n) {
         return std::min(std::max(kBinBlocks, n / kBinMax), (n + kBinMin - 1) / kBinMin);
     };
-    if (!cut_items(kick_items, &h->nitem) || !cut_items(bin_items, &h->nbin_item))
+    std::vector<int32_t> first, bin_first;  // every bunch's first item
+    if (!cut_items(kick_items, first) || !cut_items(bin_items, bin_first))
         return fail(CTS_ERR_ARG, "cts_set_bunches: too many particles");
-    if ((rc = dalloc(&h->d_item_bunch, items.size())) ||
+    h->nitem = first[nb];
+    h->nbin_item = bin_first[nb];
+    first.insert(first.end(), bin_first.begin(), bin_first.end());
+    if ((rc = dalloc(&h->d_item_bunch, (size_t)h->nitem + h->nbin_item + first.size())) ||
         (rc = dalloc(&h->d_ion_f, (size_t)nb * (CTS_MAX_SPECIES + 1) * kBePlan)))
         return rc;
-    h->d_item_first = h->d_item_bunch + h->nitem;
-    h->d_bin_bunch = h->d_item_first + nb + 1;
-    h->d_bin_first = h->d_bin_bunch + h->nbin_item;
+    h->d_bin_bunch = h->d_item_bunch + h->nitem;
+    h->d_item_first = h->d_bin_bunch + h->nbin_item;
+    h->d_bin_first = h->d_item_first + nb + 1;
     h->d_ion_bplan = h->d_ion_f + (size_t)nb * CTS_MAX_SPECIES * kBePlan;
-    HIPCHK(hipMemcpy(h->d_item_bunch, items.data(), items.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(h->d_item_first, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIPCHK(launch_item_bunch(h->d_item_first, nb, h->d_item_bunch, h->stream));
+    HIPCHK(launch_item_bunch(h->d_bin_first, nb, h->d_bin_bunch, h->stream));
     HIPCHK(hipMemcpy(h->d_bunch_off, h->offsets.data(), (nb + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(h->d_bunch_count, h->counts.data(), nb * sizeof(int64_t), hipMemcpyHostToDevice));
     h->kick_pending = false;

@@ -443,6 +443,8 @@ void stage_free(Stage &S);
 // so few that direct copies are faster)
 hipError_t stage_download(Stage &S, StageParams P, int64_t n, double *const coord[6], int32_t *lost, hipStream_t st,
                           bool &done);
+// the bunch of every item, from every bunch's first
+hipError_t launch_item_bunch(const int32_t *first, int nb, int32_t *bunch, hipStream_t st);
 hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st);
 hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_t st);
 // nitem: binning blocks (0: none)

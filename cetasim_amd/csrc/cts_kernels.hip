@@ -1567,6 +1567,18 @@ hipError_t launch_set_turn(uint32_t *t, uint32_t v, hipStream_t st)
     hipLaunchKernelGGL(k_set_turn, dim3(1), dim3(64), 0, st, t, v);
     return hipGetLastError();
 }
+// (made here: the list is one item for every 256 macroparticles, and host pages
+// and a copy for it took a quarter of cts_set_bunches on 6e7 of them)
+__global__ void __launch_bounds__(kBlock) k_item_bunch(const int32_t *first, int32_t *bunch)
+{
+    const int b = blockIdx.x, i1 = first[b + 1];
+    for (int i = first[b] + (int)(blockIdx.y * kBlock + threadIdx.x); i < i1; i += (int)gridDim.y * kBlock) bunch[i] = b;
+}
+hipError_t launch_item_bunch(const int32_t *first, int nb, int32_t *bunch, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_item_bunch, dim3(nb, 16), dim3(kBlock), 0, st, first, bunch);
+    return hipGetLastError();
+}
 hipError_t launch_wake_terms(const WakeTableParams &p, double *terms, hipStream_t st)
 {
     hipLaunchKernelGGL(k_wake_terms, dim3((kWakeSteps + kBlock - 1) / kBlock, p.nres), dim3(kBlock), 0, st, p, terms);
