@@ -791,7 +791,7 @@ struct Seg {
 //    1205 in tiles of 8192).  Chunks of whole blocks, or of a power of two,
 //    put the workgroups on the same memory channels (8.4e6: 229).
 //    `tile` returns the layout that this chose.
-void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
+void cut_layout(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
 {
     const int nb = (int)off.size() - 1;
     const int64_t n = off[nb];
@@ -859,6 +859,18 @@ void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int reside
             p = e;
         }
     }
+}
+
+// The layout asked for; the workgroups and tile that the default layout of these
+// bunches reports (cts_get_layout) stand for it, so that a program can go back.
+void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
+{
+    if (wg > 0) {
+        int t = 0;
+        cut_layout(off, 0, t, resident, out, nwg);
+        if (nwg == wg && t == tile) return;
+    }
+    cut_layout(off, wg, tile, resident, out, nwg);
 }
 
 // Segment table on the device (cut_segments): the segments in workgroup

@@ -352,7 +352,8 @@ int cts_autotune(cts_handle *h, int32_t *nwg_out);
 /* Sets the layout the autotuner chooses between (no counterpart in the
  * reference): tile = 0 cuts the particles into nwg contiguous chunks,
  * tile > 0 into tiles of that many particles (rounded up to 256) dealt
- * round-robin to min(nwg, tiles) workgroups. */
+ * round-robin to min(nwg, tiles) workgroups; the values that cts_get_layout
+ * reports for the default layout of the bunches restore it. */
 int cts_set_layout(cts_handle *h, int32_t nwg, int32_t tile);
 /* The layout in use: workgroups of the streaming pass and tile (0: chunks). */
 int cts_get_layout(cts_handle *h, int32_t *nwg, int32_t *tile);

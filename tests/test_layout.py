@@ -57,3 +57,16 @@ def test_one_bunch_in_few_segments(n):
     t = segments([n])
     check_walk([n], *t)
     assert len(t[0]) <= 1024
+
+
+@pytest.mark.parametrize("counts", [[3000] * 8, [100, 70_000, 9], [9_001] * 90, [700, 3] * 60, [40_000] * 100,
+                                    [80_000] * 60])
+def test_reported_default_restores_it(counts):
+    """The workgroups and tile that the default layout reports stand for it
+    (here pieces and chunks: tile 0), and other counts of workgroups do not."""
+    default = segments(counts)
+    nwg = int(default[4].max()) + 1
+    again, fewer = segments(counts, nwg, 0), segments(counts, nwg - 1, 0)
+    assert all(np.array_equal(a, b) for a, b in zip(default, again))
+    assert fewer[4].max() < nwg - 1
+    check_walk(counts, *fewer)
