@@ -1166,7 +1166,7 @@ int ion_phase(cts_handle *h, int32_t turn, int k)
     IonKickParams ik;
     ik.x = h->d_x; ik.y = h->d_y; ik.px = h->d_px; ik.py = h->d_py; ik.flag = h->d_flag;
     ik.seg_begin = h->d_seg_begin; ik.seg_end = h->d_seg_end;
-    ik.seg_bunch = h->d_seg_bunch; ik.wg_seg = h->d_wg_seg; ik.seg_step = h->d_seg_step;
+    ik.seg_bunch = h->d_seg_bunch; ik.seg_step = h->d_seg_step;
     ik.ion_e = h->d_ion_e;
     ik.ion_f = h->d_ion_f;
     ik.item_bunch = h->d_item_bunch; ik.item_first = h->d_item_first; ik.nitem = h->nitem;

@@ -419,12 +419,12 @@ __device__ __forceinline__ bool w_kick_region(double x, double y)
     return x < 100.0 && y < 1000.0;
 }
 
-// Weideman's approximation at NP points, their Horner recurrences
+// Weideman's approximation at the formula's two points, their recurrences
 // interleaved.
-template <int NP>
 __device__ __forceinline__ void w_weideman(const double *zr, const double *zi, double *wr, double *wi)
 {
 #pragma clang fp contract(fast)
+    constexpr int NP = 2;
     // the coefficients through an opaque pointer: their scalar loads stay in
     // the step loop instead of being hoisted out of the caller's loops and
     // kept (and spilled) in scalar registers
@@ -539,7 +539,7 @@ __device__ __forceinline__ void be_field(double x, double y, const BeField &F, d
         zi[1] = zi[0] * F.ir;
         // Weideman's approximation for both points; a point outside the kick
         // region (rare: far from the beam) takes the far-field form instead
-        w_weideman<2>(zr, zi, wr, wi);
+        w_weideman(zr, zi, wr, wi);
         if (!w_kick_region(zr[0], zi[1])) {  // the larger of each
 #pragma nounroll
             for (int q = 0; q < 2; q++) {

@@ -123,7 +123,7 @@ struct IonKickParams {
     double *px, *py;
     const uint8_t *flag;
     const int64_t *seg_begin, *seg_end;
-    const int32_t *seg_bunch, *wg_seg, *seg_step;
+    const int32_t *seg_bunch, *seg_step;
     const double *ion_e;  // per bunch CTS_MAX_SPECIES x {coeffE, xbar, ybar, sx, sy}
     const double *ion_f;  // per bunch CTS_MAX_SPECIES x the cloud's field constants (kBePlan)
     // the exact kick's items, up to kBlock particles of one bunch each: the
