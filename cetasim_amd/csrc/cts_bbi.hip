@@ -201,8 +201,9 @@ __host__ __device__ constexpr int bbi_count_words(bool dip) { return dip ? ((kBb
 // bunch's sums directly.  A bunch fills few bins, so the window is kept in as
 // many copies as fit, up to one per wave: the atomics of different waves do
 // not meet.  With one window of the whole grid per workgroup of the pass 37 us
-// on 60 bunches of 6e4 with both dipolar planes, 31 now (blocks of 512
-// threads 30, of 1024 40); without the planes 15 (512: 16, 1024: 22).
+// on 60 bunches of 6e4 with both dipolar planes, 31 now by events around the
+// launch, 28 in a kernel trace (by events, blocks of 512 threads 30, of 1024
+// 40); without the planes 15 (512: 16, 1024: 22).
 __global__ void __launch_bounds__(kBbiBinBlock) k_bbi_bin(BbiParams P)
 {
     extern __shared__ __attribute__((aligned(16))) uint32_t hl[];
@@ -422,8 +423,8 @@ __global__ void __launch_bounds__(kBlock) k_bbi_wake(BbiParams P)
 }
 
 // A block of up to 256 macroparticles of one bunch, one per thread with all
-// its loads issued at once (the kick moves 42 to 74 bytes of each and little
-// else; with four per thread in a loop and the divisions by energy, beta^2
+// its loads issued at once (the kick moves 25 bytes of each, 73 with all planes,
+// and little else; with four per thread in a loop and the divisions by energy, beta^2
 // and the beta functions 59.4 us on 60 bunches of 6e4, now 42).
 __global__ void __launch_bounds__(kBlock) k_bbi_kick(BbiParams P)
 {

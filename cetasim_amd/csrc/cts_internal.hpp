@@ -19,9 +19,11 @@ constexpr int kPostWaves = 8;  // waves of a block that closes a turn (moments o
 constexpr int kPostBlock = 64 * kPostWaves;
 // Workgroups of the streaming pass that the device holds at one time: three
 // of 256 threads per compute unit (the turn's variants use 130 to 152
-// registers).  The default layouts cut the particles for exactly that many,
-// so that no workgroup waits for a second round: with 1024 on 256 compute
-// units the 480-bunch train's pass took 1.50 ms, with 768 1.33 ms.
+// registers).  The default layouts in blocks, pieces and chunks cut the
+// particles for exactly that many, so that no workgroup waits for a second
+// round: with 1024 chunks on 256 compute units the 480-bunch train's pass took
+// 1.50 ms, with 768 1.33 ms (tiles with a workgroup each, which large trains
+// take, 1.21).
 constexpr int kPassPerCu = 3;
 constexpr uint32_t kNewLost = 0x80u;
 

@@ -71,10 +71,11 @@ k_mlp_samples(int64_t n, uint64_t seed, uint32_t tag, float *out, double *exact)
 // What it is bound by: the chain of a batch (record gather, two layers, the
 // sums in order) on one or two waves per SIMD.  One wave per 64-sample batch
 // with every operand staged in 145 KB of LDS, one wave on a compute unit, took
-// 126 us for 512 blocks of two batches; this takes 32 us (about 8 us a batch
-// with two blocks on a compute unit) and gives the same gradients, since every
-// sum keeps its order.  With the waves' sums joined only once, over 32 samples
-// each, 24 us, but the weights of a long training run drift from the others'.
+// 126 us for 512 blocks of two batches; this takes 33 us (two blocks on a
+// compute unit, each with its two batches one after the other; 256 blocks of
+// one batch 18) and gives the same gradients, since every sum keeps its order.
+// With the waves' sums joined only once, over 32 samples each, 24 us, but the
+// weights of a long training run drift from the others'.
 struct MlpTrainParams {
     const float *params;    // kMlpParams
     const float *samples;   // [n][5]

@@ -341,18 +341,22 @@ int cts_flush(cts_handle *h);
  * transmission/ion status is polled after every replay. */
 int cts_run_turns(cts_handle *h, int32_t first, int32_t nturns, int32_t use_graph);
 /* Autotuner (no counterpart in the reference): times the turn's streaming
- * pass on a copy of the particles for two layouts of the particle range
- * (one contiguous chunk per workgroup, for workgroup counts that are
- * multiples of the device's compute units; tiles of 2048-16384 particles
- * dealt round-robin to 2-4 workgroups per compute unit) and keeps the
- * fastest; *nwg_out gets the chosen workgroup count.  Moments and bin
+ * pass on a copy of the particles for layouts of the particle range (one
+ * contiguous chunk per workgroup, for workgroup counts that are multiples of
+ * the device's compute units; tiles of 2048-16384 particles dealt round-robin
+ * to 2-4 workgroups per compute unit, or with a workgroup each; the layout in
+ * use) and keeps the fastest; *nwg_out gets the chosen workgroup count.  Moments and bin
  * counts do not depend on the layout beyond the order of floating-point
  * partial sums. */
 int cts_autotune(cts_handle *h, int32_t *nwg_out);
-/* Sets the layout the autotuner chooses between (no counterpart in the
- * reference): tile = 0 cuts the particles into nwg contiguous chunks,
- * tile > 0 into tiles of that many particles (rounded up to 256) dealt
- * round-robin to min(nwg, tiles) workgroups; the values that cts_get_layout
+/* Sets a layout as the autotuner chooses between (no counterpart in the
+ * reference): tile = 0 cuts the particles into up to nwg contiguous chunks of
+ * 2048 at least, tile > 0 into tiles of that many particles (rounded up to 256)
+ * dealt round-robin to min(nwg, tiles) workgroups; with tile = 256 the blocks of
+ * every bunch are dealt by themselves, a workgroup's blocks of a bunch together.
+ * Until then the layout is chosen by size: one bunch in blocks of 256, few
+ * particles in equal pieces within the bunches, more in a chunk per workgroup
+ * that the device holds, large trains in tiles with a workgroup each.  The values that cts_get_layout
  * reports for the default layout of the bunches restore it. */
 int cts_set_layout(cts_handle *h, int32_t nwg, int32_t tile);
 /* The layout in use: workgroups of the streaming pass and tile (0: chunks). */
