@@ -791,7 +791,7 @@ struct Seg {
 //    1205 in tiles of 8192).  Chunks of whole blocks, or of a power of two,
 //    put the workgroups on the same memory channels (8.4e6: 229).
 //    `tile` returns the layout that this chose.
-void cut_layout(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
+void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
 {
     const int nb = (int)off.size() - 1;
     const int64_t n = off[nb];
@@ -861,16 +861,14 @@ void cut_layout(const std::vector<int64_t> &off, int wg, int &tile, int resident
     }
 }
 
-// The layout asked for; the workgroups and tile that the default layout of these
-// bunches reports (cts_get_layout) stand for it, so that a program can go back.
-void cut_segments(const std::vector<int64_t> &off, int wg, int &tile, int resident, std::vector<Seg> &out, int &nwg)
+// Whether a layout asked for is what the default layout of these bunches reports
+// (cts_get_layout): it then stands for the default, so that a program can go back.
+bool is_default_layout(const std::vector<int64_t> &off, int wg, int tile, int resident)
 {
-    if (wg > 0) {
-        int t = 0;
-        cut_layout(off, 0, t, resident, out, nwg);
-        if (nwg == wg && t == tile) return;
-    }
-    cut_layout(off, wg, tile, resident, out, nwg);
+    std::vector<Seg> segs;
+    int t = 0, n = 1;
+    cut_segments(off, 0, t, resident, segs, n);
+    return n == wg && t == tile;
 }
 
 // Segment table on the device (cut_segments): the segments in workgroup
@@ -1864,6 +1862,7 @@ int cts_set_layout(cts_handle *h, int32_t nwg, int32_t tile)
     if ((rc = flush_kick(h))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     graph_reset(h);
+    if (is_default_layout(h->offsets, nwg, tile, kPassPerCu * h->ncu)) nwg = 0;
     h->wg_target = nwg;
     return layout_segments(h, nwg, tile);
 }
@@ -2743,6 +2742,7 @@ int cts_debug_layout(int32_t nb, const int64_t *counts, int32_t nwg, int32_t til
     for (int b = 0; b < nb; b++) off[b + 1] = off[b] + counts[b];
     std::vector<Seg> segs;
     int n = 1;
+    if (is_default_layout(off, nwg, tile, kPassPerCu * ncu)) nwg = 0;
     cut_segments(off, nwg, tile, kPassPerCu * ncu, segs, n);
     const int64_t room = *nseg;
     *nseg = (int64_t)segs.size();

@@ -99,3 +99,24 @@ def test_cloud_of_many_waves(nspec, n_new, nb):
         for c in ("x", "y", "vx", "vy"):
             np.testing.assert_allclose(cloud[c], ec[c], rtol=1e-9, atol=1e-9 * np.max(np.abs(ec[c])))
     tr.close()
+
+
+def test_default_layout_comes_back():
+    """What the default layout reports restores it, for later bunches too."""
+    ring, secs, _ = configs.lattice()
+    tr = Tracker(ring, secs)
+
+    def bunches(counts):
+        q, ne = configs.bunch_scalars(counts, ring)
+        tr.set_bunches(counts, q, ne, configs.train_gaps(len(counts), 2, ring.harmonic))
+        return tr.layout()
+
+    small, large = [3000] * 8, [300_000] * 20
+    first, other = bunches(small), bunches(large)
+    assert first != other
+    bunches(small)
+    tr.set_layout(7, 512)
+    assert tr.layout() == (7, 512)
+    tr.set_layout(*first)
+    assert tr.layout() == first and bunches(large) == other
+    tr.close()
